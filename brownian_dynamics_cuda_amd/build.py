@@ -17,8 +17,12 @@ SOURCES = ["bd_forces.hip", "bd_integrate.hip", "bd_chol.hip", "bd_engine.hip", 
            "bd_rng.hip", "bd_potrf.hip", "bd_adjoint.hip"]
 
 # -packed-fp32-ops: no v_pk_*_f32 (packed FP32) instructions in any kernel.
+# -amdgpu-mfma-vgpr-form: matrix-core accumulators in ordinary vector
+# registers; the diagonal tile's factor reads each product's result at once,
+# and copies out of the accumulation registers would be on its chain.
 HIPFLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC", "-shared",
             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+            "-mllvm", "-amdgpu-mfma-vgpr-form=1",
             "-Wno-unused-result", "-I" + os.path.join(ROOT, "include")]
 
 

@@ -92,8 +92,8 @@ __device__ __forceinline__ void tri_index(int idx, int &i, int &j) {
     j = idx - r * (r + 1) / 2;
 }
 
-__device__ __forceinline__ void diag_factor_inv(double *T, double *LP, double *X, double *A, int ld, int d0,
-                                                double *Linv, int *neg);
+__device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, double *A, int ld, int d0, double *Linv,
+                                                int *neg);
 
 // FACTOR: workgroup 0 (tile (0,0)) then factors and inverts its tile in
 // place of a separate first-tile launch, beside the other tiles' assembly
@@ -102,8 +102,7 @@ template <bool FACTOR>
 __global__ void __launch_bounds__(256) k_rpy(Stat s, Geo g, const double *rad_all, double *A, int m, int ld,
                                              double a1, double a2, int *neg, double *Linv) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *neg = 0;  // negative-pivot count of the factor that follows
-    __shared__ double T[TB * LDP];
-    __shared__ double LP[FACTOR ? TB * TB : 1], X[FACTOR ? TB * LDP : 1];
+    __shared__ double T[(FACTOR ? 2 : 1) * TB * LDP];
     int ti, tj;
     tri_index(blockIdx.x, ti, tj);
     const int r0 = ti * TB, c0 = tj * TB, nhi = m / 3;
@@ -148,7 +147,7 @@ __global__ void __launch_bounds__(256) k_rpy(Stat s, Geo g, const double *rad_al
     if constexpr (FACTOR) {
         if (fac) {
             __syncthreads();
-            diag_factor_inv(T, LP, X, A, ld, 0, Linv, neg);
+            diag_factor_inv(T, T, A, ld, 0, Linv, neg);
         }
     }
 }
@@ -312,31 +311,6 @@ __device__ __forceinline__ void acc_to_lds(double *C, V acc[2][2], double sign, 
             }
 }
 
-// Copies up to four tiles from global memory into LDS with every global
-// load of the thread in flight before the first LDS store (n: tiles used).
-__device__ __forceinline__ void load_tiles(int n, const double *const (&src)[4], const int (&ld)[4],
-                                           double *const (&dst)[4]) {
-    constexpr int PER = TB * TB / 2 / NTHR;
-    dbl2 v[4][PER];
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-        if (t < n)
-#pragma unroll
-            for (int i = 0; i < PER; i++) {
-                const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
-                v[t][i] = *reinterpret_cast<const dbl2 *>(src[t] + (size_t)r * ld[t] + c);
-            }
-#pragma unroll
-    for (int t = 0; t < 4; t++)
-        if (t < n)
-#pragma unroll
-            for (int i = 0; i < PER; i++) {
-                const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
-                dst[t][r * LDP + c] = v[t][i].x;
-                dst[t][r * LDP + c + 1] = v[t][i].y;
-            }
-}
-
 // A 16x16 output block of the FP64 matrix cores (mapping of mma_f64:
 // register v of lane l is element (l/16 + 4v, l%16) of the block) into C.
 __device__ __forceinline__ void blk_to_lds(double *C, int I, int J, dbl4 acc, double sign, bool overwrite) {
@@ -430,398 +404,507 @@ __device__ __forceinline__ void syrk_lower(const double *P, double *C) {
     else syrk_blocks<2, 3, 2, 3, 3, 0, 0>(P, C);
 }
 
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-    int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
-    int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
-    return __hiloint2double(hi, lo);
-}
-
 // ---------------------------------------------------------------------------
-// Diagonal tile: factor and inverse by the four wavefronts of a workgroup.
+// Diagonal tile: factor L and inverse inv(L) by the four wavefronts of a
+// workgroup, as one forward elimination of [C | I].
 //
-// Wavefront w holds 16 columns of every row (lane = row) in g[]: panels w
-// and w + 4 of the 8 panels of 8 columns, which it factors in turn: the CPU
-// algorithm of func.cpp:806-836 in right-looking order -- pivot f (|f| and
-// a count if f < 0), column scaled by 1/sqrt(f) -- with the updates inside
-// a panel taken from the owning lanes by readlane.  A finished panel goes
-// to LP in panel order, LP[p][row][q] = L[row][8p + q], and the other
-// wavefronts apply it to their columns (rank-8 updates that read the 8
-// entries of a column as broadcast 16-byte LDS loads).  With the panels
-// dealt round-robin, the owner of the next panel has only that panel's 8
-// columns to bring up to date before it pivots: that catch-up and the
-// pivots are the critical path.  The wavefronts with time left build
-// X = inv(L) from 16x16 blocks: the diagonal blocks from 8x8 substitutions,
-// the off-diagonal blocks on the matrix cores,
-//   X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj.
+// What bounds it is the chain of 64 pivots, so the tile is cut into 16x16
+// blocks, a block row's pivots stay in the registers of one wavefront, and
+// everything off the chain goes to the other three.  Roles are fixed:
+//
+//   wavefront 0 holds the diagonal block of block row b, one column per lane
+//     (the four groups of 16 lanes alike), its 16 rows in registers.  A
+//     pivot's row times -1/|f| is added to the rows below with the factor of
+//     row k taken from the lane of column k inside the FMA (DPP row
+//     broadcast).  1/|f| is v_rcp_f64 with one third-order step; no square
+//     root is on the chain: L and inv(L) are scaled by 1/sqrt(|f|) when they
+//     are stored.  |f| where f < 0 (func.cpp:825-835), counted.
+//   wavefront 1 eliminates the four other blocks of the block row side by
+//     side, one per lane group: C_bj for j > b and the blocks of I for
+//     j <= b; it follows wavefront 0 by a panel of four rows.
+//   wavefronts 2 and 3 hold the blocks below (matrix-core result registers)
+//     and subtract the panels' rank-4 products as they come; after the last
+//     panel the blocks of row b + 1 go to wavefronts 0 and 1 through LDS.
+//     In the last block row, where nothing is below, they store the rows
+//     before it.
+//
+// Rows and columns of a 16x16 block are permuted alike, index i at position
+// pos(i) = i/4 + 4 (i%4): register v of lane (g, c) of a matrix-core result
+// is then row 4g + v, and a panel's rows serve as either operand.
+// Panel buffers: W(b, j) and E(b, j), 16x16 each, element [64 p + 4 c + k] =
+// row 4p + k, column position c.
+//
+// Measured alone, warm: 15.0k cycles (6.2 us) against 25.1k for one wavefront
+// owning panels of 8 columns with rank-8 updates through LDS; of a block
+// column's launch 16.0 -> 13.4 us.  What was in the way on gfx950: an FP64 FMA
+// issues every 5 cycles from one wavefront, dependent or not, v_rcp_f64 and
+// v_rsq_f64 take 16, a dependent 16x16x4 FP64 product 69 (and no FP64 FMA
+// beside it), a store to LDS and the read back 135-165, so the pivots' updates
+// stay in registers and the matrix cores do what is off the chain.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ constexpr int pos16(int i) { return i / 4 + 4 * (i % 4); }
 
-// g[C0 .. C0+NC) -= sum_q x[q] * lp[col*8 + q] for the columns col =
-// colbase + C0 + c, each column's sum in increasing q.  Four columns at a
-// time, their FMA chains interleaved (with two chains the dependent FP64
-// FMA latency, not the issue rate, set the pace); the entries of the next
-// four columns (broadcast 16-byte LDS loads) are loaded one group ahead (a
-// scheduling barrier per group keeps that distance).
-template <int C0, int NC>
-__device__ __forceinline__ void panel_update16(double (&g)[16], const double (&x)[8], const double *lp,
-                                               int colbase) {
-    constexpr int NG = NC / 4;
-    const double2 *l2 = reinterpret_cast<const double2 *>(lp) + (colbase + C0) * 4;
-    double2 e[NG][16];
-#pragma unroll
-    for (int k = 0; k < 16; k++) e[0][k] = l2[k];
-#pragma unroll
-    for (int i = 0; i < NG; i++) {
-        if (i + 1 < NG)
-#pragma unroll
-            for (int k = 0; k < 16; k++) e[i + 1][k] = l2[(i + 1) * 16 + k];
-        const int c = C0 + 4 * i;
-        double s[4] = {g[c], g[c + 1], g[c + 2], g[c + 3]};
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-#pragma unroll
-            for (int m = 0; m < 4; m++) s[m] -= x[2 * k] * e[i][4 * m + k].x;
-#pragma unroll
-            for (int m = 0; m < 4; m++) s[m] -= x[2 * k + 1] * e[i][4 * m + k].y;
-        }
-#pragma unroll
-        for (int m = 0; m < 4; m++) g[c + m] = s[m];
-        __builtin_amdgcn_sched_barrier(0);
+// Rows in registers: the factor of row k times a scaled pivot row is one FMA
+// whose first operand comes from the lane of column k of the same 16 lanes
+// (v_fmac_f64_dpp row_newbcast).  The compiler does not form it, so these
+// steps are inline code, in an order that keeps two instructions between a
+// VALU write and the DPP read of the register (what the hardware needs, and
+// the compiler does not add around inline code) with as few s_nop as possible:
+// an s_nop 1 costs 8 cycles of the chain, an FMA 5, v_rcp_f64 16.
+#define BD_POS_0 "0"
+#define BD_POS_1 "4"
+#define BD_POS_2 "8"
+#define BD_POS_3 "12"
+#define BD_POS_4 "1"
+#define BD_POS_5 "5"
+#define BD_POS_6 "9"
+#define BD_POS_7 "13"
+#define BD_POS_8 "2"
+#define BD_POS_9 "6"
+#define BD_POS_10 "10"
+#define BD_POS_11 "14"
+#define BD_POS_12 "3"
+#define BD_POS_13 "7"
+#define BD_POS_14 "11"
+#define BD_POS_15 "15"
+#define BD_DPP " row_mask:0xf bank_mask:0xf\n\t"
+// row k += (column k of row j) m
+#define BD_FM(k, j, m) "v_fmac_f64_dpp %[w" #k "], %[w" #j "], %[" #m "] row_newbcast:" BD_POS_##k BD_DPP
+// 1/|f_j| (third-order step from its seed y = v_rcp_f64(|f|): y (1 + e + e^2),
+// e = 1 - |f| y) and m = -w_j / |f_j|
+#define BD_RM(j)                                                                          \
+    "v_fma_f64 %[e], -|%[f]|, %[y], 1.0\n\tv_fma_f64 %[e], %[e], %[e], %[e]\n\t"          \
+    "v_fma_f64 %[r], %[y], %[e], %[y]\n\tv_mul_f64 %[m], %[w" #j "], -%[r]\n\t"
+// the next pivot (column j of row j) and its seed
+#define BD_NEXT(j) "v_mov_b64_dpp %[f], %[w" #j "] row_newbcast:" BD_POS_##j BD_DPP
+#define BD_SEED "v_rcp_f64 %[y], |%[f]|\n\t"
+#define BD_PIVOT(J, TEXT)                                                                                           \
+    {                                                                                                               \
+    asm volatile(TEXT                                                                                               \
+                 : [w0] "+v"(w[0]), [w1] "+v"(w[1]), [w2] "+v"(w[2]), [w3] "+v"(w[3]), [w4] "+v"(w[4]),             \
+                   [w5] "+v"(w[5]), [w6] "+v"(w[6]), [w7] "+v"(w[7]), [w8] "+v"(w[8]), [w9] "+v"(w[9]),             \
+                   [w10] "+v"(w[10]), [w11] "+v"(w[11]), [w12] "+v"(w[12]), [w13] "+v"(w[13]), [w14] "+v"(w[14]),   \
+                   [w15] "+v"(w[15]), [r] "=&v"(r[J]), [m] "=&v"(m), [e] "=&v"(e), [y] "+v"(y), [f] "+v"(f)         \
+                 : [n] "v"(n));                                                                                     \
+    n = m;                                                                                                          \
     }
+// Pivots J of wavefront 0: y, f the seed and the pivot; the products of the
+// two last rows are left to the next pivot (n: its m) while there are enough.
+template <int J>
+__device__ __forceinline__ void pivot(double (&w)[16], double (&r)[16], double &y, double &f, double &n) {
+    double m, e;
+    if constexpr (J == 0)
+        BD_PIVOT(0, "s_nop 1\n\t" BD_NEXT(0) BD_SEED "s_nop 0\n\t" BD_RM(0) "s_nop 1\n\t" BD_FM(1, 0, m) BD_FM(2, 0, m) BD_FM(3, 0, m)
+                 BD_NEXT(1) BD_FM(4, 0, m) BD_SEED BD_FM(5, 0, m) BD_FM(6, 0, m) BD_FM(7, 0, m) BD_FM(8, 0, m)
+                 BD_FM(9, 0, m) BD_FM(10, 0, m) BD_FM(11, 0, m) BD_FM(12, 0, m) BD_FM(13, 0, m));
+    if constexpr (J == 1)
+        BD_PIVOT(1, BD_RM(1) BD_FM(14, 0, n) BD_FM(15, 0, n) BD_FM(2, 1, m) BD_FM(3, 1, m) BD_FM(4, 1, m)
+                 BD_NEXT(2) BD_FM(5, 1, m) BD_SEED BD_FM(6, 1, m) BD_FM(7, 1, m) BD_FM(8, 1, m) BD_FM(9, 1, m)
+                 BD_FM(10, 1, m) BD_FM(11, 1, m) BD_FM(12, 1, m) BD_FM(13, 1, m));
+    if constexpr (J == 2)
+        BD_PIVOT(2, BD_RM(2) BD_FM(14, 1, n) BD_FM(15, 1, n) BD_FM(3, 2, m) BD_FM(4, 2, m) BD_FM(5, 2, m)
+                 BD_NEXT(3) BD_FM(6, 2, m) BD_SEED BD_FM(7, 2, m) BD_FM(8, 2, m) BD_FM(9, 2, m) BD_FM(10, 2, m)
+                 BD_FM(11, 2, m) BD_FM(12, 2, m) BD_FM(13, 2, m));
+    if constexpr (J == 3)
+        BD_PIVOT(3, BD_RM(3) BD_FM(14, 2, n) BD_FM(15, 2, n) BD_FM(4, 3, m) BD_FM(5, 3, m) BD_FM(6, 3, m)
+                 BD_NEXT(4) BD_FM(7, 3, m) BD_SEED BD_FM(8, 3, m) BD_FM(9, 3, m) BD_FM(10, 3, m) BD_FM(11, 3, m)
+                 BD_FM(12, 3, m) BD_FM(13, 3, m));
+    if constexpr (J == 4)
+        BD_PIVOT(4, BD_RM(4) BD_FM(14, 3, n) BD_FM(15, 3, n) BD_FM(5, 4, m) BD_FM(6, 4, m) BD_FM(7, 4, m)
+                 BD_NEXT(5) BD_FM(8, 4, m) BD_SEED BD_FM(9, 4, m) BD_FM(10, 4, m) BD_FM(11, 4, m) BD_FM(12, 4, m)
+                 BD_FM(13, 4, m));
+    if constexpr (J == 5)
+        BD_PIVOT(5, BD_RM(5) BD_FM(14, 4, n) BD_FM(15, 4, n) BD_FM(6, 5, m) BD_FM(7, 5, m) BD_FM(8, 5, m)
+                 BD_NEXT(6) BD_FM(9, 5, m) BD_SEED BD_FM(10, 5, m) BD_FM(11, 5, m) BD_FM(12, 5, m) BD_FM(13, 5, m));
+    if constexpr (J == 6)
+        BD_PIVOT(6, BD_RM(6) BD_FM(14, 5, n) BD_FM(15, 5, n) BD_FM(7, 6, m) BD_FM(8, 6, m) BD_FM(9, 6, m)
+                 BD_NEXT(7) BD_FM(10, 6, m) BD_SEED BD_FM(11, 6, m) BD_FM(12, 6, m) BD_FM(13, 6, m));
+    if constexpr (J == 7)
+        BD_PIVOT(7, BD_RM(7) BD_FM(14, 6, n) BD_FM(15, 6, n) BD_FM(8, 7, m) BD_FM(9, 7, m) BD_FM(10, 7, m)
+                 BD_NEXT(8) BD_FM(11, 7, m) BD_SEED BD_FM(12, 7, m) BD_FM(13, 7, m));
+    if constexpr (J == 8)
+        BD_PIVOT(8, BD_RM(8) BD_FM(14, 7, n) BD_FM(15, 7, n) BD_FM(9, 8, m) BD_FM(10, 8, m) BD_FM(11, 8, m)
+                 BD_NEXT(9) BD_FM(12, 8, m) BD_SEED BD_FM(13, 8, m));
+    if constexpr (J == 9)
+        BD_PIVOT(9, BD_RM(9) BD_FM(14, 8, n) BD_FM(15, 8, n) BD_FM(10, 9, m) BD_FM(11, 9, m) BD_FM(12, 9, m)
+                 BD_NEXT(10) BD_FM(13, 9, m) BD_SEED BD_FM(14, 9, m) BD_FM(15, 9, m));
+    if constexpr (J == 10)
+        BD_PIVOT(10, BD_RM(10) "s_nop 1\n\t" BD_FM(11, 10, m) BD_FM(12, 10, m) BD_FM(13, 10, m) BD_NEXT(11)
+                 BD_FM(14, 10, m) BD_SEED BD_FM(15, 10, m));
+    if constexpr (J == 11)
+        BD_PIVOT(11, BD_RM(11) "s_nop 1\n\t" BD_FM(12, 11, m) BD_FM(13, 11, m) BD_FM(14, 11, m) BD_NEXT(12)
+                 BD_SEED BD_FM(15, 11, m));
+    if constexpr (J == 12)
+        BD_PIVOT(12, BD_RM(12) "s_nop 1\n\t" BD_FM(13, 12, m) BD_FM(14, 12, m) BD_FM(15, 12, m) BD_NEXT(13)
+                 BD_SEED "s_nop 0\n\t");
+    if constexpr (J == 13)
+        BD_PIVOT(13, BD_RM(13) "s_nop 1\n\t" BD_FM(14, 13, m) BD_FM(15, 13, m) "s_nop 0\n\t" BD_NEXT(14)
+                 BD_SEED "s_nop 0\n\t");
+    if constexpr (J == 14)
+        BD_PIVOT(14, BD_RM(14) "s_nop 1\n\t" BD_FM(15, 14, m) "s_nop 1\n\t" BD_NEXT(15) BD_SEED "s_nop 0\n\t");
+    if constexpr (J == 15) BD_PIVOT(15, BD_RM(15));
 }
 
-// Pivots of panel P (columns 8P..8P+7) held in g[L0 .. L0+7]; publishes the
-// panel to LP and the pivot inverses 1/L_jj of its lanes to ivs.
-// Branch-free, so the row stays in registers.
-template <int P, int L0>
-__device__ __forceinline__ void pivot_panel(double (&g)[16], double *LP, double *ivs, double &myinv, int &nneg) {
+// Rows of another block column: the panel's own rows x[K..K+3] by the pivot
+// rows u before them, m_j = -x_j / |f_j| ...
+template <int K>
+__device__ __forceinline__ void follow_rows(double (&x)[16], const double (&u)[4], const double (&r)[4],
+                                            double (&m)[4]) {
+#define BD_FX(d, s, q, c) "v_fmac_f64_dpp %[" d "], %[" s "], %[" q "] row_newbcast:%[" c "]" BD_DPP
+#define BD_MX(q, d, s) "v_mul_f64 %[" q "], %[" d "], -%[" s "]\n\ts_nop 1\n\t"
+    asm volatile(BD_MX("m0", "x0", "r0") BD_FX("x1", "u0", "m0", "c1") BD_FX("x2", "u0", "m0", "c2")
+                     BD_FX("x3", "u0", "m0", "c3") BD_MX("m1", "x1", "r1") BD_FX("x2", "u1", "m1", "c2")
+                         BD_FX("x3", "u1", "m1", "c3") BD_MX("m2", "x2", "r2") BD_FX("x3", "u2", "m2", "c3")
+                 : [x1] "+v"(x[K + 1]), [x2] "+v"(x[K + 2]), [x3] "+v"(x[K + 3]), [m0] "=&v"(m[0]), [m1] "=&v"(m[1]),
+                   [m2] "=&v"(m[2])
+                 : [x0] "v"(x[K]), [u0] "v"(u[0]), [u1] "v"(u[1]), [u2] "v"(u[2]), [r0] "v"(r[0]), [r1] "v"(r[1]),
+                   [r2] "v"(r[2]), [c1] "n"(pos16(K + 1)), [c2] "n"(pos16(K + 2)), [c3] "n"(pos16(K + 3)));
+    m[3] = x[K + 3] * -r[3];
+}
+// ... and four rows x[K..K+3] below by all four
+template <int K>
+__device__ __forceinline__ void below_rows(double (&x)[16], const double (&u)[4], const double (&m)[4]) {
+    asm volatile("s_nop 1\n\t" BD_FX("x0", "u0", "m0", "c0") BD_FX("x1", "u0", "m0", "c1") BD_FX("x2", "u0", "m0", "c2")
+                     BD_FX("x3", "u0", "m0", "c3") BD_FX("x0", "u1", "m1", "c0") BD_FX("x1", "u1", "m1", "c1")
+                         BD_FX("x2", "u1", "m1", "c2") BD_FX("x3", "u1", "m1", "c3") BD_FX("x0", "u2", "m2", "c0")
+                             BD_FX("x1", "u2", "m2", "c1") BD_FX("x2", "u2", "m2", "c2") BD_FX("x3", "u2", "m2", "c3")
+                                 BD_FX("x0", "u3", "m3", "c0") BD_FX("x1", "u3", "m3", "c1")
+                                     BD_FX("x2", "u3", "m3", "c2") BD_FX("x3", "u3", "m3", "c3")
+                 : [x0] "+v"(x[K]), [x1] "+v"(x[K + 1]), [x2] "+v"(x[K + 2]), [x3] "+v"(x[K + 3])
+                 : [u0] "v"(u[0]), [u1] "v"(u[1]), [u2] "v"(u[2]), [u3] "v"(u[3]), [m0] "v"(m[0]), [m1] "v"(m[1]),
+                   [m2] "v"(m[2]), [m3] "v"(m[3]), [c0] "n"(pos16(K)), [c1] "n"(pos16(K + 1)), [c2] "n"(pos16(K + 2)),
+                   [c3] "n"(pos16(K + 3)));
+}
+
+// LDS of the elimination: two tiles of pitch LDP, the second of which may
+// hold the tile itself until it is in registers
+struct DiagLds {
+    double *base;
+    // panel buffers W(b, j), j >= b, and E(b, j), j <= b, 256 each
+    __device__ __forceinline__ double *W(int b, int j) const { return base + (b * (9 - b) / 2 + j - b) * 256; }
+    __device__ __forceinline__ double *E(int b, int j) const { return base + (10 + b * (b + 1) / 2 + j) * 256; }
+    // blocks of the next block row, element [18 c + row]: lane group q of
+    // wavefront 1, q = 4 wavefront 0
+    __device__ __forceinline__ double *next(int q) const { return base + 5120 + 288 * q; }
+    __device__ __forceinline__ double *R() const { return base + 6560; }  // 1/|f|, 64
+    __device__ __forceinline__ double *S() const { return base + 6624; }  // 1/sqrt(|f|), 64
+};
+constexpr int kNextPitch = 18;
+static_assert(6688 <= 2 * TB * LDP, "the elimination fits two tiles");
+
+// the operand register of a panel: lane (k, c) holds row k, column c
+__device__ __forceinline__ double panel_op(const double *S, int p) {
     const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int jc = 8 * P + j;
-        const double f0 = readlane_f64(g[L0 + j], jc);
-        nneg += f0 < 0 ? 1 : 0;
-        const double f = fabs(f0);
-        const double inv = rsqrt_f64(f);
-        const double lj = lane > jc ? g[L0 + j] * inv : (lane == jc ? f * inv : 0.0);
-        myinv = lane == jc ? inv : myinv;
-        g[L0 + j] = lj;
-#pragma unroll
-        for (int c = j + 1; c < 8; c++) g[L0 + c] -= lj * readlane_f64(lj, 8 * P + c);
-    }
-    double *lp = LP + P * (TB * 8);
-#pragma unroll
-    for (int q = 0; q < 8; q += 2) {
-        double2 v;
-        v.x = g[L0 + q];
-        v.y = g[L0 + q + 1];
-        *reinterpret_cast<double2 *>(lp + lane * 8 + q) = v;
-    }
-    if (lane >= 8 * P && lane < 8 * P + 8) ivs[lane] = myinv;
+    return S[64 * p + 4 * (lane & 15) + (lane >> 4)];
 }
-
-// this lane's row of panel P, from LP
+__device__ __forceinline__ dbl4 rank4(double a, double b, dbl4 acc) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+}
+// rows 4P..4P+3 of w to a panel buffer (this lane's column)
 template <int P>
-__device__ __forceinline__ void panel_row(const double *LP, double (&x)[8]) {
-    const double2 *r = reinterpret_cast<const double2 *>(LP + P * (TB * 8) + (threadIdx.x & 63) * 8);
+__device__ __forceinline__ void put_rows(double *S, const double (&w)[16]) {
+    double2 *d = reinterpret_cast<double2 *>(S + 64 * P + 4 * (threadIdx.x & 15));
+    d[0] = make_double2(w[4 * P], w[4 * P + 1]);
+    d[1] = make_double2(w[4 * P + 2], w[4 * P + 3]);
+}
+__device__ __forceinline__ void load_rows(double (&w)[16], const double *src) {
+    const double2 *s = reinterpret_cast<const double2 *>(src);
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const double2 d = r[k];
-        x[2 * k] = d.x;
-        x[2 * k + 1] = d.y;
+    for (int i = 0; i < 8; i++) {
+        const double2 v = s[i];
+        w[2 * i] = v.x;
+        w[2 * i + 1] = v.y;
     }
 }
 
-// X_ww = inv(L_ww) for the 16x16 diagonal block w, by wavefront w, in 8x8
-// blocks: L_ww = [[A, 0], [B, C]] gives X_ww = [[A^-1, 0], [-C^-1 B A^-1, C^-1]].
-// Lanes 0-7 solve A y = e_r and lanes 8-15 C y = e_r by substitution, side
-// by side (y_c = (e_r[c] - sum_{j<c} L_cj y_j) / L_cc, eight steps); then
-// every lane forms one entry of Y = B A^-1 and one of -C^-1 Y.  The upper
-// triangle and the upper right block are written as zeros (the products
-// that read X_ww take whole 16x16 blocks).  S: the wavefront's LDS scratch
-// (8 rows of pitch 17).
-__device__ __forceinline__ void diag_block_inverse(const double *LP, const double *ivs, double *X, double *S, int w) {
-    const int lane = threadIdx.x & 63;
-    {
-        const int h = (lane >> 3) & 1, r = lane & 7;
-        const int b0 = 16 * w + 8 * h;  // first row and column of block A (h = 0) or C (h = 1)
-        // L[b0 + c][b0 + j] = lh[c*8 + j]: panel 2w + h, rows b0..b0+7
-        const double *lh = LP + (2 * w + h) * (TB * 8) + b0 * 8;
-        const double2 *i2 = reinterpret_cast<const double2 *>(ivs + b0);
-        double iw[8];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const double2 v = i2[k];
-            iw[2 * k] = v.x;
-            iw[2 * k + 1] = v.y;
-        }
-        double y[8];
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-            double l[8];
-#pragma unroll
-            for (int j = 0; j < c; j += 2) {
-                const double2 v = *reinterpret_cast<const double2 *>(lh + c * 8 + j);
-                l[j] = v.x;
-                l[j + 1] = v.y;
-            }
-            double sum = (c == r) ? 1.0 : 0.0;
-#pragma unroll
-            for (int j = 0; j < c; j++) sum -= y[j] * l[j];
-            y[c] = sum * iw[c];
-        }
-        if (lane < 16) {
-#pragma unroll
-            for (int c = 0; c < 8; c++) X[(b0 + c) * LDP + b0 + r] = y[c];
-            if (h)
-#pragma unroll
-                for (int c = 0; c < 8; c++) X[(16 * w + c) * LDP + b0 + r] = 0.0;
-        }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const int a = lane >> 3, b = lane & 7, d0 = 16 * w;
-    // Y[a][b] = sum_k B[a][k] A^-1[k][b], B[a][k] = L[d0 + 8 + a][d0 + k] (panel 2w)
-    const double *lb = LP + 2 * w * (TB * 8) + (d0 + 8 + a) * 8;
-    double yv = 0.0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) yv += lb[k] * X[(d0 + k) * LDP + d0 + b];
-    S[a * 17 + b] = yv;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    double z = 0.0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) z += X[(d0 + 8 + a) * LDP + d0 + 8 + k] * S[k * 17 + b];
-    X[(d0 + 8 + a) * LDP + d0 + b] = -z;
-}
-
-// 16x16 block products on the matrix cores (v_mfma_f64_16x16x4f64; result
-// register v of lane l is element (l/16 + 4v, l%16)), one wavefront each.
-// acc += L_ik X_kj, with L in panel order (LP) and X of pitch LDP.
-__device__ __forceinline__ dbl4 mm_lx(dbl4 acc, const double *LP, const double *X, int i, int k, int j) {
-    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
-#pragma unroll
-    for (int kk = 0; kk < 16; kk += 4) {
-        const int col = 16 * k + kk + k4;
-        const double a = LP[(col >> 3) * (TB * 8) + (16 * i + i16) * 8 + (col & 7)];
-        const double b = X[(16 * k + kk + k4) * LDP + 16 * j + i16];
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    }
-    return acc;
-}
-// acc += X_ii S, S a 16x16 block of pitch 17
-__device__ __forceinline__ dbl4 mm_xs(dbl4 acc, const double *X, const double *S, int i) {
-    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
-#pragma unroll
-    for (int kk = 0; kk < 16; kk += 4) {
-        const double a = X[(16 * i + i16) * LDP + 16 * i + kk + k4];
-        const double b = S[(kk + k4) * 17 + i16];
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    }
-    return acc;
-}
-// D (a 16x16 block of the given pitch) = sign * acc; the wavefront's later
-// LDS reads of D are ordered after these stores
-__device__ __forceinline__ void put_block(double *D, int pitch, dbl4 acc, double sign) {
-    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
-#pragma unroll
-    for (int v = 0; v < 4; v++) D[(k4 + 4 * v) * pitch + i16] = sign * acc[v];
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-// S = sum_{k=j}^{i-1} L_ik X_kj (the sum of X_ij = -X_ii S without X_ii)
-__device__ __forceinline__ void x_sum(const double *LP, const double *X, double *S, int i, int j) {
-    dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-    for (int k = j; k < i; k++) acc = mm_lx(acc, LP, X, i, k, j);
-    put_block(S, 17, acc, 1.0);
-}
-// X_ij = -X_ii S from a sum S formed by x_sum (possibly by another wavefront)
-__device__ __forceinline__ void x_final(double *X, const double *S, int i, int j) {
-    const dbl4 z = {0.0, 0.0, 0.0, 0.0};
-    put_block(X + 16 * i * LDP + 16 * j, LDP, mm_xs(z, X, S, i), -1.0);
-}
-// S (+)= sum_{k=k0}^{k1-1} L_3k X_kj: terms of the part of X_3j that does
-// not need X_33, S_3j = sum_{k=j}^{2} L_3k X_kj; with ADD the sum continues
-// from the partial sum already in S (the same order as in one pass).
-__device__ __forceinline__ void s3_part(const double *LP, const double *X, double *S, int j, int k0, int k1,
-                                        bool add) {
-    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
-    dbl4 acc = {0.0, 0.0, 0.0, 0.0};
-    if (add)
-#pragma unroll
-        for (int v = 0; v < 4; v++) acc[v] = S[(k4 + 4 * v) * 17 + i16];
-    for (int k = k0; k < k1; k++) acc = mm_lx(acc, LP, X, 3, k, j);
-    put_block(S, 17, acc, 1.0);
-}
-// Rows r0 .. r0+15 of inv(L) from X to global memory (row-major 64x64), with
-// zeros in the 16x16 blocks above the diagonal; one wavefront.
-__device__ __forceinline__ void store_xrows(const double *X, double *Linv, int r0) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int e = lane; e < 16 * (TB / 2); e += 64) {
-        const int r = r0 + e / (TB / 2), c = 2 * (e % (TB / 2));
-        dbl2 v;
-        const bool keep = (r >> 4) >= (c >> 4);
-        v.x = keep ? X[r * LDP + c] : 0.0;
-        v.y = keep ? X[r * LDP + c + 1] : 0.0;
-        *reinterpret_cast<dbl2 *>(Linv + r * TB + c) = v;
-    }
-}
-
-// Columns 8G..8G+7 of this lane's g (group G = 0 or 1) to row[0..7]: 8
-// columns of row d0 + lane of L (zeros above the diagonal: a lane above a
-// pivot column takes 0 at that pivot)
-__device__ __forceinline__ void store_lrow8(const double (&g)[16], int G, double *row) {
-#pragma unroll
-    for (int c = 0; c < 8; c += 2) {
-        dbl2 v;
-        v.x = g[8 * G + c];
-        v.y = g[8 * G + c + 1];
-        *reinterpret_cast<dbl2 *>(row + c) = v;
-    }
-}
-
-// One panel step of the factor (all four wavefronts; ends with a barrier).
-// Wavefront w owns panels w and w + 4 (columns 8w.. in g[0..7], 32 + 8w..
-// in g[8..15]).  The owner of panel P applies panel P-1 to the panel's 8
-// columns (the earlier panels are already in them), pivots it and stores
-// its 8 columns of L.  The other wavefronts apply panel P-1 to their columns
-// not yet pivoted; the owner of the previous step, which skipped its other
-// group while pivoting, applies panel P-2 to that group first, so every
-// column receives the panels in increasing order.  Beside this, the
-// wavefronts with time left build inv(L), each piece as soon as its inputs
-// are final: X_00 (step 2), S_10 = L_10 X_00 (3), X_11 (4), X_10 = -X_11
-// S_10, S_21 = L_21 X_11 and the k = 1 term of S_31 (5), X_22, S_20 and the
-// k < 2 terms of S_30 (6), X_20, X_21 and S_32 = L_32 X_22 (7); rows 0-15
-// (5) and 16-31 (7) of inv(L) go to global memory.  S: the wavefront's
-// 16x17 scratch (the four lie SW apart, and a sum left in one wavefront's
-// scratch is read by another in a later step), S3: the partial sums S_3j.
+// Panel P of wavefront 0.  Its rows and 1/|f| are published with the next
+// panel's first pivot between their LDS stores and the barrier.
 template <int P>
-__device__ __forceinline__ void factor_step(double (&g)[16], double *LP, double *ivs, double *X, double *S,
-                                            double *S3, double &myinv, int &nneg, int w, double *lrow,
-                                            double *Linv) {
-    constexpr int O = P & 3, LOC = P >> 2, SW = 16 * 17;
-    if (w == O) {
-        if constexpr (P > 0) {
-            double x[8];
-            panel_row<P - 1>(LP, x);
-            __builtin_amdgcn_sched_barrier(0);
-            panel_update16<8 * LOC, 8>(g, x, LP + (P - 1) * (TB * 8), 8 * P - 8 * LOC);
-        }
-        pivot_panel<P, 8 * LOC>(g, LP, ivs, myinv, nneg);
-        store_lrow8(g, LOC, lrow + 8 * P);
-    } else {
-        if constexpr (P > 0) {
-            double x[8];
-            panel_row<P - 1>(LP, x);
-            __builtin_amdgcn_sched_barrier(0);
-            if (w > P) panel_update16<0, 8>(g, x, LP + (P - 1) * (TB * 8), 8 * w);
-            if (w + 4 > P) {
-                if constexpr (P >= 2) {
-                    if (w == P - 1) {
-                        double x2[8];
-                        panel_row<P - 2>(LP, x2);
-                        __builtin_amdgcn_sched_barrier(0);
-                        panel_update16<8, 8>(g, x2, LP + (P - 2) * (TB * 8), 8 * w + 24);
-                    }
-                }
-                panel_update16<8, 8>(g, x, LP + (P - 1) * (TB * 8), 8 * w + 24);
-            }
-        }
-        if constexpr (P == 2) {
-            if (w == 0) diag_block_inverse(LP, ivs, X, S, 0);
-        } else if constexpr (P == 3) {
-            if (w == 1) x_sum(LP, X, S, 1, 0);
-        } else if constexpr (P == 4) {
-            if (w == 2) diag_block_inverse(LP, ivs, X, S, 1);
-        } else if constexpr (P == 5) {
-            if (w == 0) {
-                x_final(X, S + SW, 1, 0);
-                store_xrows(X, Linv, 0);
-            } else if (w == 2) {
-                x_sum(LP, X, S, 2, 1);
-                s3_part(LP, X, S3 + SW, 1, 1, 2, false);
-            }
-        } else if constexpr (P == 6) {
-            if (w == 0) {
-                diag_block_inverse(LP, ivs, X, S, 2);
-            } else if (w == 1) {
-                x_sum(LP, X, S, 2, 0);
-                s3_part(LP, X, S3, 0, 0, 2, false);
-            }
-        } else if constexpr (P == 7) {
-            if (w == 0) {
-                x_final(X, S + SW, 2, 0);
-                store_xrows(X, Linv, 16);
-            } else if (w == 1) {
-                x_final(X, S + SW, 2, 1);
-            } else {
-                s3_part(LP, X, S3 + 2 * SW, 2, 2, 3, false);
-            }
-        }
+__device__ __forceinline__ void pivot_panel(double (&w)[16], double (&r)[16], double &y, double &f, double &n,
+                                            const DiagLds &l, int b) {
+    if constexpr (P == 0) pivot<0>(w, r, y, f, n);
+    pivot<4 * P + 1>(w, r, y, f, n);
+    pivot<4 * P + 2>(w, r, y, f, n);
+    pivot<4 * P + 3>(w, r, y, f, n);
+    const int lane = threadIdx.x & 63;
+    if (lane < 16) put_rows<P>(l.W(b, b), w);
+    if (lane == 16) {
+        double2 *d = reinterpret_cast<double2 *>(l.R() + 16 * b + 4 * P);
+        d[0] = make_double2(r[4 * P], r[4 * P + 1]);
+        d[1] = make_double2(r[4 * P + 2], r[4 * P + 3]);
     }
+    if constexpr (P < 3) pivot<4 * P + 4>(w, r, y, f, n);
     __syncthreads();
 }
 
-// Called by all four wavefronts.  T: the tile (LDS, pitch LDP) at (d0, d0),
-// free for scratch once the rows are in registers (ivs and the per-wavefront
-// scratch of the inverse); LP: LDS, 64*64; X: LDS, 64*LDP.  L goes to A
-// (lower, zeros above) and inv(L), row-major 64x64, to Linv.
-__device__ __forceinline__ void diag_factor_inv(double *T, double *LP, double *X, double *A, int ld, int d0,
-                                                double *Linv, int *neg) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    double g[16];
+// Panel P of wavefront 1: rows 4P..4P+3 of its four blocks by the pivot rows
+// of wavefront 0, published, and the rows below them.
+template <int P>
+__device__ __forceinline__ void follow_panel(double (&x)[16], const DiagLds &l, double *Y, int b) {
+    __syncthreads();
+    const double2 *u2 = reinterpret_cast<const double2 *>(l.W(b, b) + 64 * P + 4 * (threadIdx.x & 15));
+    const double2 *r2 = reinterpret_cast<const double2 *>(l.R() + 16 * b + 4 * P);
+    const double2 ua = u2[0], ub = u2[1], ra = r2[0], rb = r2[1];
+    const double u[4] = {ua.x, ua.y, ub.x, ub.y}, r[4] = {ra.x, ra.y, rb.x, rb.y};
+    double m[4];
+    follow_rows<4 * P>(x, u, r, m);
+    put_rows<P>(Y, x);
+    if constexpr (P < 3) below_rows<4 * P + 4>(x, u, m);
+    if constexpr (P < 2) below_rows<4 * P + 8>(x, u, m);
+    if constexpr (P < 1) below_rows<4 * P + 12>(x, u, m);
+}
+
+// L(b + q, b) for q < 4 - b, inv(L)(b, q - (4 - b)) after them: block q of
+// the five that block row b leaves, scaled by 1/sqrt(|f|) and stored.
+__device__ __forceinline__ void store_block(const DiagLds &l, int b, int q, double *A, int ld, int d0, double *Linv) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
+    const bool isl = q < 4 - b;
+    const int j = isl ? b + q : q - (4 - b);
+    const double2 *s = reinterpret_cast<const double2 *>((isl ? l.W(b, j) : l.E(b, j)) + 64 * g + 4 * c);
+    const double2 *i2 = reinterpret_cast<const double2 *>(l.S() + 16 * b + 4 * g);
+    const double2 x0 = s[0], x1 = s[1], i0 = i2[0], i1 = i2[1];
+    double x[4] = {x0.x * i0.x, x0.y * i0.y, x1.x * i1.x, x1.y * i1.y};
+    if (isl) {
+        if (j == b) {  // lower triangle of the diagonal block, L_jj = |f| / sqrt(|f|)
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-        g[c] = T[lane * LDP + 8 * w + c];
-        g[8 + c] = T[lane * LDP + 32 + 8 * w + c];
-    }
-    __syncthreads();
-    double *ivs = T, *S = T + TB + w * (16 * 17), *S3 = T + TB + 4 * (16 * 17);
-    double *lrow = A + (size_t)(d0 + lane) * ld + d0;
-    int nneg = 0;
-    double myinv = 0.0;
-    factor_step<0>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    factor_step<1>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    factor_step<2>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    factor_step<3>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    factor_step<4>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    factor_step<5>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    factor_step<6>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    factor_step<7>(g, LP, ivs, X, S, S3, myinv, nneg, w, lrow, Linv);
-    if (nneg && lane == 0) atomicAdd(neg, nneg);
-    // X_33, the k = 2 terms of S_30 and S_31, and rows 32-47 of inv(L)
-    if (w == 3) {
-        diag_block_inverse(LP, ivs, X, S, 3);
-    } else if (w == 0) {
-        s3_part(LP, X, S3, 0, 2, 3, true);
-    } else if (w == 1) {
-        s3_part(LP, X, S3 + 16 * 17, 1, 2, 3, true);
+            for (int v = 0; v < 4; v++) x[v] = 4 * g + v > ci ? 0.0 : 4 * g + v == ci ? fabs(x[v]) : x[v];
+        }
+        double *row = A + (size_t)(d0 + 16 * j + ci) * ld + d0 + 16 * b + 4 * g;
+        *reinterpret_cast<dbl2 *>(row) = dbl2{x[0], x[1]};
+        *reinterpret_cast<dbl2 *>(row + 2) = dbl2{x[2], x[3]};
     } else {
-        store_xrows(X, Linv, 32);
+#pragma unroll
+        for (int v = 0; v < 4; v++) Linv[(16 * b + 4 * g + v) * TB + 16 * j + ci] = x[v];
+    }
+}
+
+// Block (i, j) of the tile, i <= j, in matrix-core result registers
+__device__ __forceinline__ dbl4 tile_block(const double *T, int i, int j) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
+    dbl4 x;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int r = 16 * i + 4 * g + v, k = 16 * j + ci;
+        x[v] = T[max(r, k) * LDP + min(r, k)];
+    }
+    return x;
+}
+// a finished block of block row b + 1 to its reader
+__device__ __forceinline__ void put_next(const DiagLds &l, int q, dbl4 x) {
+    const int lane = threadIdx.x & 63;
+    double2 *d = reinterpret_cast<double2 *>(l.next(q) + kNextPitch * (lane & 15) + 4 * (lane >> 4));
+    d[0] = make_double2(x[0], x[1]);
+    d[1] = make_double2(x[2], x[3]);
+}
+
+// Panel p of block row B on the blocks that wavefront 2 + U holds, rows from
+// I0 to I1: U = 0 has C11 C12 C22 C23 C33 E31, U = 1 has C13 E10 E20 E21 E30 E32.
+template <int B, int U, int I0, int I1>
+__device__ __forceinline__ void below_panel(dbl4 (&Z)[6], const DiagLds &l, int p) {
+    const int g = (threadIdx.x & 63) >> 4;
+    const double rn = -l.R()[16 * B + 4 * p + g];
+    double a[4], e[3];
+#pragma unroll
+    for (int i = B + 1; i < 4; i++) a[i] = panel_op(l.W(B, i), p);
+#pragma unroll
+    for (int j = 0; j <= B; j++)
+        if (U == 0 ? j == 1 : j != 1 || B == 1) e[j] = panel_op(l.E(B, j), p) * rn;
+    auto in = [](int i) { return i > B && i >= I0 && i <= I1; };
+    if constexpr (U == 0) {
+        if (in(1)) Z[0] = rank4(a[1], a[1] * rn, Z[0]);
+        if (in(1)) Z[1] = rank4(a[1], a[2] * rn, Z[1]);
+        if (in(2)) Z[2] = rank4(a[2], a[2] * rn, Z[2]);
+        if (in(2)) Z[3] = rank4(a[2], a[3] * rn, Z[3]);
+        if (in(3)) Z[4] = rank4(a[3], a[3] * rn, Z[4]);
+        if constexpr (B >= 1)
+            if (in(3)) Z[5] = rank4(a[3], e[1], Z[5]);
+    } else {
+        if (in(1)) Z[0] = rank4(a[1], a[3] * rn, Z[0]);
+        if (in(1)) Z[1] = rank4(a[1], e[0], Z[1]);
+        if (in(2)) Z[2] = rank4(a[2], e[0], Z[2]);
+        if constexpr (B >= 1)
+            if (in(2)) Z[3] = rank4(a[2], e[1], Z[3]);
+        if (in(3)) Z[4] = rank4(a[3], e[0], Z[4]);
+        if constexpr (B >= 2)
+            if (in(3)) Z[5] = rank4(a[3], e[2], Z[5]);
+    }
+}
+template <int B, int U>
+__device__ __forceinline__ void below_row(dbl4 (&Z)[6], const DiagLds &l) {
+    __syncthreads();
+#pragma unroll 1
+    for (int p = 0; p < 3; p++) {
+        __syncthreads();
+        below_panel<B, U, B + 1, 3>(Z, l, p);
     }
     __syncthreads();
-    // X_3j = -X_33 S_3j straight from the matrix-core registers to rows
-    // 48-63, columns 16j..16j+15 of inv(L) (register v of lane l: element
-    // (l/16 + 4v, l%16))
-    if (w < 3) {
+    below_panel<B, U, B + 1, B + 1>(Z, l, 3);
+    if constexpr (U == 0) {
+        put_next(l, 4, Z[B == 0 ? 0 : B == 1 ? 2 : 4]);
+        put_next(l, B == 2 ? 1 : 0, Z[B == 0 ? 1 : B == 1 ? 3 : 5]);
+    } else {
+        put_next(l, B == 2 ? 0 : 1, Z[B == 0 ? 0 : B == 1 ? 2 : 4]);
+        put_next(l, 2, Z[B == 0 ? 1 : B == 1 ? 3 : 5]);
+    }
+    __syncthreads();
+    if constexpr (B < 2) below_panel<B, U, B + 2, 3>(Z, l, 3);
+}
+
+// Called by all four wavefronts.  lds: two tiles; T, one of them, holds the
+// tile (pitch LDP) at (d0, d0), of which the lower triangle is read.  L goes
+// to A (lower triangle), inv(L), row-major 64x64 with zeros above its
+// diagonal, to Linv.
+__device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, double *A, int ld, int d0, double *Linv,
+                                                int *neg) {
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
+    const DiagLds l = {lds};
+    if (wv == 0) {
+        double w[16], r[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) w[k] = T[max(k, ci) * LDP + min(k, ci)];
+        __syncthreads();
+#pragma unroll 1
+        for (int b = 0; b < 4; b++) {
+            if (b) load_rows(w, l.next(4) + kNextPitch * c);
+            double y = 0.0, f = 0.0, n = 0.0;
+            pivot_panel<0>(w, r, y, f, n, l, b);
+            pivot_panel<1>(w, r, y, f, n, l, b);
+            pivot_panel<2>(w, r, y, f, n, l, b);
+            pivot_panel<3>(w, r, y, f, n, l, b);
+            // the scale factors of the block row and its negative pivots
+            const double fd = l.W(b, b)[64 * (c >> 2) + 4 * pos16(c) + (c & 3)];
+            if (lane < 16) l.S()[16 * b + c] = rsqrt_f64(fabs(fd));
+            const unsigned long long nm = __ballot(lane < 16 && fd < 0);
+            if (nm && lane == 0) atomicAdd(neg, __popcll(nm));
+            __syncthreads();
+            if (b < 3) __syncthreads();
+        }
+    } else if (wv == 1) {
+        double x[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = g < 3 ? T[(16 * (g + 1) + ci) * LDP + k] : k == ci ? 1.0 : 0.0;
+        __syncthreads();
+#pragma unroll 1
+        for (int b = 0; b < 4; b++) {
+            if (b) {
+                load_rows(x, l.next(min(g, 2)) + kNextPitch * c);
+#pragma unroll
+                for (int k = 0; k < 16; k++) x[k] = g < 3 ? x[k] : k == ci ? 1.0 : 0.0;
+            }
+            double *Y = g < 3 - b ? l.W(b, b + 1 + g) : l.E(b, b + g - 3);
+            follow_panel<0>(x, l, Y, b);
+            follow_panel<1>(x, l, Y, b);
+            follow_panel<2>(x, l, Y, b);
+            follow_panel<3>(x, l, Y, b);
+            __syncthreads();
+            if (b < 3) __syncthreads();
+        }
+    } else {
         const dbl4 z = {0.0, 0.0, 0.0, 0.0};
-        const dbl4 x3 = mm_xs(z, X, S3 + w * (16 * 17), 3);
-        const int i16 = lane & 15, k4 = lane >> 4;
+        // the blocks of inv(L) above its diagonal
 #pragma unroll
-        for (int v = 0; v < 4; v++) Linv[(48 + k4 + 4 * v) * TB + 16 * w + i16] = -x3[v];
-    } else {
-        // X_33 to rows 48-63, columns 48-63 of inv(L)
-#pragma unroll
-        for (int e = lane; e < 16 * 8; e += 64) {
-            const int r = 48 + e / 8, c = 48 + 2 * (e % 8);
-            dbl2 v;
-            v.x = X[r * LDP + c];
-            v.y = X[r * LDP + c + 1];
-            *reinterpret_cast<dbl2 *>(Linv + r * TB + c) = v;
+        for (int t = 0; t < 3; t++) {
+            const int k = 3 * (wv - 2) + t, bi = k < 3 ? 0 : k < 5 ? 1 : 2, bj = k < 3 ? k + 1 : k < 5 ? k - 1 : 3;
+            dbl2 *o = reinterpret_cast<dbl2 *>(Linv + (16 * bi + (lane >> 2)) * TB + 16 * bj + 4 * (lane & 3));
+            o[0] = o[1] = dbl2{0.0, 0.0};
+        }
+        if (wv == 2) {
+            dbl4 Z[6] = {tile_block(T, 1, 1), tile_block(T, 1, 2), tile_block(T, 2, 2), tile_block(T, 2, 3),
+                         tile_block(T, 3, 3), z};
+            __syncthreads();
+            below_row<0, 0>(Z, l);
+            below_row<1, 0>(Z, l);
+            below_row<2, 0>(Z, l);
+        } else {
+            dbl4 Z[6] = {tile_block(T, 1, 3), z, z, z, z, z};
+            __syncthreads();
+            below_row<0, 1>(Z, l);
+            below_row<1, 1>(Z, l);
+            below_row<2, 1>(Z, l);
+        }
+        // block rows 0 to 2 are complete: 15 blocks, beside the last pivots
+#pragma unroll 1
+        for (int p = 0; p < 5; p++) {
+            __syncthreads();
+            if (p < 4)
+                for (int t = 4 * p + wv - 2; t < min(4 * p + 4, 15); t += 2) store_block(l, t / 5, t % 5, A, ld, d0, Linv);
         }
     }
+    store_block(l, 3, wv, A, ld, d0, Linv);
+    if (wv == 0) store_block(l, 3, 4, A, ld, d0, Linv);
 }
 
+// a tile between global memory, registers and LDS (pitch LDP), 16-byte
+// accesses, every load of a thread in flight at once
+constexpr int PERT = TB * TB / 2 / NTHR;
+__device__ __forceinline__ void tile_to_regs(const double *src, int ld, dbl2 (&v)[PERT]) {
+#pragma unroll
+    for (int i = 0; i < PERT; i++) {
+        const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        v[i] = *reinterpret_cast<const dbl2 *>(src + (size_t)r * ld + c);
+    }
+}
+__device__ __forceinline__ void regs_to_lds(const dbl2 (&v)[PERT], double *S) {
+#pragma unroll
+    for (int i = 0; i < PERT; i++) {
+        const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        S[r * LDP + c] = v[i].x;
+        S[r * LDP + c + 1] = v[i].y;
+    }
+}
+// C -= Pi Pj^T for an off-diagonal tile C in global memory, from registers
+// (element mapping of mma_*)
+template <int MODE>
+__device__ __forceinline__ void tile_update(const double *Pi, const double *Pj, double *C, int ld) {
+    typename AccOf<MODE>::T acc[2][2];
+    for (int a = 0; a < 2; a++)
+        for (int b = 0; b < 2; b++) acc[a][b] = {};
+    tile_mma<MODE>(Pi, Pj, acc);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int wr = (w >> 1) * 32, wc = (w & 1) * 32, i16 = lane & 15, k4 = lane >> 4;
+    constexpr bool f64 = MODE == 0;
+    double cv[2][2][4];
+#pragma unroll
+    for (int mi = 0; mi < 2; mi++)
+#pragma unroll
+        for (int ni = 0; ni < 2; ni++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = wr + 16 * mi + (f64 ? k4 + 4 * v : 4 * k4 + v), c = wc + 16 * ni + i16;
+                cv[mi][ni][v] = C[(size_t)r * ld + c];
+            }
+#pragma unroll
+    for (int mi = 0; mi < 2; mi++)
+#pragma unroll
+        for (int ni = 0; ni < 2; ni++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = wr + 16 * mi + (f64 ? k4 + 4 * v : 4 * k4 + v), c = wc + 16 * ni + i16;
+                C[(size_t)r * ld + c] = cv[mi][ni][v] + -1.0 * (double)acc[mi][ni][v];
+            }
+}
+// C -= P P^T for a diagonal tile: read into T (LDS) first, left there for the
+// factor (keep) or stored, its lower triangle
+template <int MODE>
+__device__ __forceinline__ void diag_tile_update(const double *P, double *T, double *C, int ld, bool keep) {
+    dbl2 v[PERT];
+    tile_to_regs(C, ld, v);
+    regs_to_lds(v, T);
+    __syncthreads();
+    if (MODE == 0) {
+        syrk_lower(P, T);
+    } else {
+        typename AccOf<MODE>::T acc[2][2];
+        for (int a = 0; a < 2; a++)
+            for (int b = 0; b < 2; b++) acc[a][b] = {};
+        tile_mma<MODE>(P, P, acc);
+        acc_to_lds(T, acc, -1.0, false);
+    }
+    if (keep) return;
+    __syncthreads();
+    store_tile(C, ld, 0, 0, T, true);
+}
 
 // Trailing tiles of block column kb restricted to the first jcols trailing
 // block columns, row-major: rows ii = 0..M-1, columns jj <= min(ii, jcols-1)
@@ -854,12 +937,12 @@ __device__ __forceinline__ void trap_index(int idx, int jcols, int &i, int &j) {
 // exchange for one launch (and one kernel boundary) per block column.
 // jcols < M restricts the update to the columns of a super-panel.
 template <int MODE>
-__global__ void __launch_bounds__(256) k_step(double *A, int ld, int kb, int jcols, double *Linv, int *neg) {
-    // three tiles of LDS: inv(L_kb,kb), the row's panel block, and a third
-    // holding the target tile in the diagonal tiles' workgroups (the factor's
-    // T) and the column's panel block in the others, whose target tile is
-    // updated in registers
-    __shared__ double W[TB * LDP], As[TB * LDP], BC[TB * LDP];
+__global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int jcols, double *Linv, int *neg) {
+    // two tiles of LDS (two workgroups per CU): first inv(L_kb,kb) and the
+    // row's panel block, then the column's panel block in place of the row's,
+    // then the two panel tiles; the target tile stays in registers
+    __shared__ double S[2 * TB * LDP];
+    double *S0 = S, *S1 = S + TB * LDP;
     // workgroups go round-robin over the eight XCDs (b % 8); XCD x takes a
     // contiguous run of tiles, so the tiles of a block row, which read the
     // same panel tile, share an L2 (workgroup 0, the diagonal tile, stays 0)
@@ -870,72 +953,45 @@ __global__ void __launch_bounds__(256) k_step(double *A, int ld, int kb, int jco
     trap_index(lb, jcols, ii, jj);
     const int ib = kb + 1 + ii, jb = kb + 1 + jj;
     const bool diag = ib == jb;
+    if (lb == 0) __builtin_amdgcn_s_setprio(3);
+    dbl2 vi[PERT], vj[PERT];
     {
-        // inv(L_kb,kb), the panel blocks (or the diagonal target tile), all in flight
-        const double *const src[4] = {Linv + (size_t)kb * TB * TB, A + (size_t)ib * TB * ld + kb * TB,
-                                      diag ? A + (size_t)ib * TB * ld + jb * TB : A + (size_t)jb * TB * ld + kb * TB,
-                                      nullptr};
-        const int lds[4] = {TB, ld, ld, 0};
-        double *const dst[4] = {W, As, BC, nullptr};
-        load_tiles(3, src, lds, dst);
+        dbl2 vw[PERT];
+        tile_to_regs(Linv + (size_t)kb * TB * TB, TB, vw);
+        tile_to_regs(A + (size_t)ib * TB * ld + kb * TB, ld, vi);
+        if (!diag) tile_to_regs(A + (size_t)jb * TB * ld + kb * TB, ld, vj);
+        regs_to_lds(vw, S0);
+        regs_to_lds(vi, S1);
     }
     __syncthreads();
-    {
-        dbl4 pi[4], pj[4];
-        for (int J = 0; J < 4; J++) pi[J] = pj[J] = dbl4{0.0, 0.0, 0.0, 0.0};
-        mma_panel(As, W, pi);
-        if (!diag) mma_panel(BC, W, pj);
-        __syncthreads();
-        panel_to_lds(As, pi);
-        if (!diag) panel_to_lds(BC, pj);
-    }
+    dbl4 pi[4];
+    for (int J = 0; J < 4; J++) pi[J] = dbl4{0.0, 0.0, 0.0, 0.0};
+    mma_panel(S1, S0, pi);
     __syncthreads();
-    if (jj == 0) store_tile(A, ld, kb * TB, ib * TB, As, false);
     if (diag) {
-        if (MODE == 0) {
-            syrk_lower(As, BC);
-        } else {
-            typename AccOf<MODE>::T acc[2][2];
-            for (int a = 0; a < 2; a++)
-                for (int b = 0; b < 2; b++) acc[a][b] = {};
-            tile_mma<MODE>(As, As, acc);
-            acc_to_lds(BC, acc, -1.0, false);
-        }
+        panel_to_lds(S1, pi);
         __syncthreads();
-        if (ii == 0)
-            diag_factor_inv(BC, W, As, A, ld, ib * TB, Linv + (size_t)ib * TB * TB, neg);
-        else
-            store_tile(A, ld, ib * TB, jb * TB, BC, true);
+        if (jj == 0) store_tile(A, ld, kb * TB, ib * TB, S1, false);
+        diag_tile_update<MODE>(S1, S0, A + (size_t)ib * TB * ld + jb * TB, ld, ii == 0);
+        if (ii == 0) {
+            __syncthreads();
+            diag_factor_inv(S, S0, A, ld, ib * TB, Linv + (size_t)ib * TB * TB, neg);
+        }
         return;
     }
-    typename AccOf<MODE>::T acc[2][2];
-    for (int a = 0; a < 2; a++)
-        for (int b = 0; b < 2; b++) acc[a][b] = {};
-    tile_mma<MODE>(As, BC, acc);
-    // C -= acc in place from registers (the element mapping of acc_to_lds)
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wr = (w >> 1) * 32, wc = (w & 1) * 32, i16 = lane & 15, k4 = lane >> 4;
-    constexpr bool f64 = MODE == 0;
-    double *C = A + (size_t)ib * TB * ld + jb * TB;
-    double cv[2][2][4];
-#pragma unroll
-    for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-        for (int ni = 0; ni < 2; ni++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = wr + 16 * mi + (f64 ? k4 + 4 * v : 4 * k4 + v), c = wc + 16 * ni + i16;
-                cv[mi][ni][v] = C[(size_t)r * ld + c];
-            }
-#pragma unroll
-    for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-        for (int ni = 0; ni < 2; ni++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = wr + 16 * mi + (f64 ? k4 + 4 * v : 4 * k4 + v), c = wc + 16 * ni + i16;
-                C[(size_t)r * ld + c] = cv[mi][ni][v] + -1.0 * (double)acc[mi][ni][v];
-            }
+    regs_to_lds(vj, S1);
+    __syncthreads();
+    {
+        dbl4 pj[4];
+        for (int J = 0; J < 4; J++) pj[J] = dbl4{0.0, 0.0, 0.0, 0.0};
+        mma_panel(S1, S0, pj);
+        __syncthreads();
+        panel_to_lds(S0, pi);
+        panel_to_lds(S1, pj);
+    }
+    __syncthreads();
+    if (jj == 0) store_tile(A, ld, kb * TB, ib * TB, S0, false);
+    tile_update<MODE>(S0, S1, A + (size_t)ib * TB * ld + jb * TB, ld);
 }
 
 // The same block column in two launches, for wide trailing matrices (many
@@ -949,11 +1005,11 @@ __global__ void __launch_bounds__(256) k_panel(double *A, int ld, int kb, const 
     __shared__ double W[TB * LDP], As[TB * LDP];
     const int ib = kb + 1 + blockIdx.x;
     {
-        const double *const src[4] = {Linv + (size_t)kb * TB * TB, A + (size_t)ib * TB * ld + kb * TB, nullptr,
-                                      nullptr};
-        const int lds[4] = {TB, ld, 0, 0};
-        double *const dst[4] = {W, As, nullptr, nullptr};
-        load_tiles(2, src, lds, dst);
+        dbl2 vw[PERT], va[PERT];
+        tile_to_regs(Linv + (size_t)kb * TB * TB, TB, vw);
+        tile_to_regs(A + (size_t)ib * TB * ld + kb * TB, ld, va);
+        regs_to_lds(vw, W);
+        regs_to_lds(va, As);
     }
     __syncthreads();
     dbl4 pi[4];
@@ -966,8 +1022,9 @@ __global__ void __launch_bounds__(256) k_panel(double *A, int ld, int kb, const 
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(256) k_update(double *A, int ld, int kb, int jcols, double *Linv, int *neg) {
-    __shared__ double As[TB * LDP], Bs[TB * LDP], Cs[TB * LDP];
+__global__ void __launch_bounds__(256, 2) k_update(double *A, int ld, int kb, int jcols, double *Linv, int *neg) {
+    __shared__ double S[2 * TB * LDP];
+    double *S0 = S, *S1 = S + TB * LDP;
     int lb = blockIdx.x;  // XCD-contiguous runs of tiles, as in k_step
     const int G8 = gridDim.x / 8;
     if (lb < 8 * G8) lb = (lb % 8) * G8 + lb / 8;
@@ -975,29 +1032,25 @@ __global__ void __launch_bounds__(256) k_update(double *A, int ld, int kb, int j
     trap_index(lb, jcols, ii, jj);
     const int ib = kb + 1 + ii, jb = kb + 1 + jj;
     const bool diag = ib == jb;
+    if (lb == 0) __builtin_amdgcn_s_setprio(3);
     {
-        // the parked panel tiles L_ib,kb and L_jb,kb and the target tile
-        const double *const src[4] = {A + (size_t)kb * TB * ld + ib * TB, A + (size_t)ib * TB * ld + jb * TB,
-                                      A + (size_t)kb * TB * ld + jb * TB, nullptr};
-        const int lds[4] = {ld, ld, ld, 0};
-        double *const dst[4] = {As, Cs, Bs, nullptr};
-        load_tiles(diag ? 2 : 3, src, lds, dst);
+        // the parked panel tiles L_ib,kb and L_jb,kb
+        dbl2 vi[PERT], vj[PERT];
+        tile_to_regs(A + (size_t)kb * TB * ld + ib * TB, ld, vi);
+        if (!diag) tile_to_regs(A + (size_t)kb * TB * ld + jb * TB, ld, vj);
+        regs_to_lds(vi, S1);
+        if (!diag) regs_to_lds(vj, S0);
     }
     __syncthreads();
-    if (MODE == 0 && diag) {
-        syrk_lower(As, Cs);
-    } else {
-        typename AccOf<MODE>::T acc[2][2];
-        for (int a = 0; a < 2; a++)
-            for (int b = 0; b < 2; b++) acc[a][b] = {};
-        tile_mma<MODE>(As, diag ? As : Bs, acc);
-        acc_to_lds(Cs, acc, -1.0, false);
+    if (!diag) {
+        tile_update<MODE>(S1, S0, A + (size_t)ib * TB * ld + jb * TB, ld);
+        return;
     }
-    __syncthreads();
-    if (ii == 0 && jj == 0)
-        diag_factor_inv(Cs, As, Bs, A, ld, ib * TB, Linv + (size_t)ib * TB * TB, neg);
-    else
-        store_tile(A, ld, ib * TB, jb * TB, Cs, diag);
+    diag_tile_update<MODE>(S1, S0, A + (size_t)ib * TB * ld + jb * TB, ld, ii == 0);
+    if (ii == 0) {
+        __syncthreads();
+        diag_factor_inv(S, S0, A, ld, ib * TB, Linv + (size_t)ib * TB * TB, neg);
+    }
 }
 
 // Trailing update of a super-panel: block columns k0 .. k0+nb-1 are
@@ -1010,22 +1063,6 @@ __global__ void __launch_bounds__(256) k_update(double *A, int ld, int kb, int j
 // Workgroups are grouped in 8x8 blocks of tiles, 64 consecutive workgroups
 // per block, so the panel tiles of a block's 8 rows and 8 columns are
 // shared through the L2; workgroups past the triangle or the edge exit.
-constexpr int NTHR_T = 256;
-__device__ __forceinline__ void tile_to_regs(const double *src, int ld, dbl2 (&v)[TB * TB / 2 / NTHR_T]) {
-#pragma unroll
-    for (int i = 0; i < TB * TB / 2 / NTHR_T; i++) {
-        const int e = threadIdx.x + i * NTHR_T, r = e / (TB / 2), c = 2 * (e % (TB / 2));
-        v[i] = *reinterpret_cast<const dbl2 *>(src + (size_t)r * ld + c);
-    }
-}
-__device__ __forceinline__ void regs_to_lds(const dbl2 (&v)[TB * TB / 2 / NTHR_T], double *S) {
-#pragma unroll
-    for (int i = 0; i < TB * TB / 2 / NTHR_T; i++) {
-        const int e = threadIdx.x + i * NTHR_T, r = e / (TB / 2), c = 2 * (e % (TB / 2));
-        S[r * LDP + c] = v[i].x;
-        S[r * LDP + c + 1] = v[i].y;
-    }
-}
 template <int MODE>
 __global__ void __launch_bounds__(256, 2) k_trail(double *A, int ld, int k0, int nb, int j0, int nt) {
     __shared__ double As[TB * LDP], Bs[TB * LDP];
@@ -1034,8 +1071,7 @@ __global__ void __launch_bounds__(256, 2) k_trail(double *A, int ld, int k0, int
     const int ib = j0 + 8 * SI + ((blockIdx.x >> 3) & 7), jb = j0 + 8 * SJ + (blockIdx.x & 7);
     if (ib >= nt || jb > ib) return;
     const bool diag = ib == jb;
-    constexpr int PER = TB * TB / 2 / NTHR_T;
-    dbl2 va[PER], vb[PER];
+    dbl2 va[PERT], vb[PERT];
     typename AccOf<MODE>::T acc[2][2];
     for (int a = 0; a < 2; a++)
         for (int b = 0; b < 2; b++) acc[a][b] = {};
@@ -1413,11 +1449,11 @@ __global__ void __launch_bounds__(256, 2) k_trail_pk(double *A, int ld, const do
 // tile after a super-panel's trailing update, or the first tile of a
 // caller's matrix); clear != 0 also restarts the negative-pivot count.
 __global__ void __launch_bounds__(256) k_diag(double *A, int ld, int d, double *Linv, int *neg, int clear) {
-    __shared__ double T[TB * LDP], LP[TB * TB], X[TB * LDP];
+    __shared__ double T[2 * TB * LDP];
     if (clear && threadIdx.x == 0) *neg = 0;
     load_tile(A, ld, d * TB, d * TB, T);
     __syncthreads();
-    diag_factor_inv(T, LP, X, A, ld, d * TB, Linv + (size_t)d * TB * TB, neg);
+    diag_factor_inv(T, T, A, ld, d * TB, Linv + (size_t)d * TB * TB, neg);
 }
 
 // rd = s2dt * L * p (rd_cal, func_cuda.cu:634-647): one wavefront per row,

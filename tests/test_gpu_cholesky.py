@@ -39,6 +39,36 @@ def test_sizes_against_lapack(m):
     assert np.all(np.triu(L, 1) == 0)
 
 
+@pytest.mark.parametrize("m", [2, 15, 16, 17, 33, 47, 63, 80, 127, 129])
+def test_blocks_of_the_diagonal_tile(m):
+    """Sizes around the 16x16 blocks of the diagonal tile's elimination, with
+    the |f| rule in every block: D = U diag(s) U^T with U unit lower
+    triangular and signs s, so pivot i is s_i and the factor the algorithm of
+    func.cpp:806-836 gives, here in extended precision."""
+    g = np.random.default_rng(m)
+    U = np.tril(g.uniform(-0.5, 0.5, (m, m)) / np.sqrt(m), -1) + np.eye(m)
+    s = np.where(g.random(m) < 0.3, -1.0, 1.0) * g.uniform(0.5, 2.0, m)
+    s[0] = abs(s[0])
+    D = (U * s) @ U.T
+    D = np.tril(D) + np.tril(D, -1).T
+    C = D.astype(np.longdouble)
+    L = np.zeros_like(C)
+    neg = 0
+    for j in range(m):
+        f = C[j, j]
+        neg += int(f < 0)
+        L[j:, j] = C[j:, j] / np.sqrt(abs(f))
+        L[j, j] = np.sqrt(abs(f))
+        C[j + 1:, j + 1:] -= np.outer(L[j + 1:, j], L[j + 1:, j])
+    Lg, ng = E.cholesky_device(D)
+    assert ng == neg
+    assert rel_err(Lg, L.astype(np.float64)) <= 1e-12
+    # a power of four in D is its root in L, exactly
+    for k in (-600, 600):
+        Ls, _ = E.cholesky_device(np.ldexp(D, k))
+        assert np.array_equal(Ls, np.ldexp(Lg, k // 2))
+
+
 def test_super_panel_size_and_mixed_modes():
     """4500 rows: 71 block columns, factored in super-panels of 8."""
     D = spd(4500, 7)
