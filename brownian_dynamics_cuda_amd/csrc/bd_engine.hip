@@ -73,8 +73,9 @@ struct bd_context {
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_gate = nullptr;
     // force pass 1 waits for the factor to pass this block column (-1: the
-    // default fraction of the block columns; BD_GATE_KB overrides it)
+    // default of enqueue_step; BD_GATE_KB overrides it)
     int gate_kb = -1;
+    int ncu = 256;  // compute units of the device
     // branches of the two force passes of a step (streams shared, events per pass)
     ForceStreams fstr[2]{};
     std::vector<void *> allocs;
@@ -178,15 +179,23 @@ struct Marker {
     }
 };
 
-// The force pass at configuration g into f (energy only when Epart given).
-// Pass 2 (pass == 1) runs its branches on their own streams unless the
-// timing markers are on; pass 1 stays on one stream, because it already
-// shares the GPU with the factorisation on the side stream.
-void enqueue_forces(bd_context *c, const Geo &g, const Frc &f, double *Epart, int terms, int pass,
+// The force pass at configuration g into f (energy only when Epart given);
+// with branch its branches run on their own streams, unless the timing
+// markers are on.
+void enqueue_forces(bd_context *c, const Geo &g, const Frc &f, double *Epart, int terms, int pass, bool branch,
                     bool sites_done = false) {
     launch_forces(c->st, g, c->sites, f, c->fw, Epart, terms, c->stream, c->timing ? mark_cb : nullptr, c,
-                  (c->timing || pass == 0) ? nullptr : &c->fstr[pass], sites_done);
+                  (c->timing || !branch) ? nullptr : &c->fstr[pass], sites_done);
 }
+
+// Force pass 1 shares the GPU with the factorisation on the side stream,
+// which any second branch of it slows (100 nucleosomes: 970 us a step with
+// branches, 906 on one stream).  Up to this many block columns the factor is
+// shorter than the pass's chain of kernels, and the branches are the shorter
+// way (us a step on one stream / branched: 12 nucleosomes, 4 block columns,
+// 295 / 249; 25 with linker histones, 8 block columns, 389 / 330; 32, 11 block
+// columns, 356 / 368; 16 block columns, all beads, 380 / 411).
+constexpr int kBranchTiles = 9;
 
 void enqueue_factor(bd_context *c, const Geo &g, hipStream_t q, hipEvent_t gate = nullptr, int gate_kb = -1) {
     Marker M{c};
@@ -220,11 +229,18 @@ void enqueue_step(bd_context *c, bool refactor) {
         (void)hipStreamWaitEvent(c->side, c->ev_fork, 0);
         qf = c->side;
     }
-    // force pass 1 starts once the factor is past block column gate_kb:
-    // the early block columns fill the GPU, and force kernels beside them
-    // hold the CUs that the diagonal-tile workgroups wait for
+    // force pass 1 starts once the factor is past block column gate_kb: the
+    // early block columns fill the GPU, and force kernels beside them hold
+    // the CUs that the diagonal-tile workgroups wait for.  By default the
+    // first column whose trailing tiles fit the CUs one by one, 23 before the
+    // last on 256 CUs: 50 nucleosomes (17 block columns) 465 us a step at
+    // columns 0-2, 495 at 6, 534 at 9; 100 (33) flat from 6 to 13, +1% at 17
+    // and 4; 157 in FP32 (52) 1776 at 29, 1838 at 15; 500 (164) -0.6% from 90
+    // to 120-141, 1000 in BF16 (328) -1.3% from 180 to 305.
     const int nt = c->chol.mpad / 64;
-    const int gate_kb = c->gate_kb >= 0 ? c->gate_kb : (nt - 1) * 55 / 100;
+    int fit = 0;
+    while ((fit + 1) * (fit + 2) / 2 <= c->ncu) fit++;
+    const int gate_kb = c->gate_kb >= 0 ? c->gate_kb : std::max(0, nt - 1 - fit);
     const bool gated = refactor && qf != q;
     if (refactor) enqueue_factor(c, c->cur, qf, gated ? c->ev_gate : nullptr, gate_kb);
     const double *du = nullptr;
@@ -237,7 +253,7 @@ void enqueue_step(bd_context *c, bool refactor) {
     // LH bending angles at the current state (3497)
     M(K_BETAS, 0); launch_betas(s, c->cur, 0, 1, q); M(K_BETAS, 1);
     // force pass 1 at x0 and its energy (3556-3615)
-    enqueue_forces(c, c->cur, c->f0, c->Epart, BD_TERM_ALL, 0);
+    enqueue_forces(c, c->cur, c->f0, c->Epart, BD_TERM_ALL, 0, !refactor || nt <= kBranchTiles);
     M(K_EREDUCE, 0); launch_energy_reduce(c->Epart, c->ne, c->energy, q); M(K_EREDUCE, 1);
     if (qf != q) {
         (void)hipEventRecord(c->ev_join, qf);
@@ -257,7 +273,7 @@ void enqueue_step(bd_context *c, bool refactor) {
     }
     M(K_FRAMES, 1);
     // force pass 2 (3628-3646)
-    enqueue_forces(c, c->pred, c->f1, nullptr, BD_TERM_ALL, 1, sites_done);
+    enqueue_forces(c, c->pred, c->f1, nullptr, BD_TERM_ALL, 1, true, sites_done);
     // corrector from x0 with the averaged forces, same rd and rr (3648-3652)
     // (the Heun means of forces and torques formed where they are read)
     M(K_TRANSLATE, 0);
@@ -572,6 +588,7 @@ int bd_create(const bd_system *sys, const bd_options *opt, bd_context **out) {
         hipDeviceProp_t prop;
         if (hipGetDeviceProperties(&prop, o.device) == hipSuccess && prop.multiProcessorCount > 0)
             ncu = prop.multiProcessorCount;
+        c->ncu = ncu;
         c->chol.split_tiles = ncu * 19 / 10;
     }
     r |= c->alloc(&c->chol.A, (size_t)c->chol.ld * c->chol.ld);
@@ -867,7 +884,7 @@ int bd_forces(bd_context *c, int terms, double *F, double *T, double *tF, double
     if (check(c)) return BD_E_ARG;
     if (!c->state_set) return fail(BD_E_STATE, "bd_set_state must be called first");
     HIPCHK(hipSetDevice(c->device));
-    enqueue_forces(c, c->cur, c->f0, c->Epart, terms, 0);
+    enqueue_forces(c, c->cur, c->f0, c->Epart, terms, 0, true);
     launch_energy_reduce(c->Epart, c->ne, c->energy, c->stream);
     HIPCHK(hipGetLastError());
     if (c->timing) collect_timing(c);

@@ -1438,9 +1438,8 @@ void launch_forces(const Stat &s, const Geo &g, const Sites &st, const Frc &f, c
                                                                           E(off_core), terms, cs[0], cs[1]);
         M(K_CORE, 1);
     };
-    // with branches (force pass 2, after the factor has joined) the chunk
-    // spheres take the sites launch; in pass 1 beside the factor the extra
-    // launch measured faster
+    // with branches the chunk spheres take the sites launch; on one stream
+    // beside the factor the extra launch measured faster
     if (!sites_done) { M(K_SITES, 0); launch_sites(s, g, st, w.cc_count, q, fs != nullptr); M(K_SITES, 1); }
     // The enqueue orders were measured (cfg2): on one stream, beside the
     // factorisation, tail and LH first and core-core last; with branches,
