@@ -22,10 +22,23 @@
 // and dphi/dq_k = q_l (uz gh + eps eh) with gh = g_DH / (q_k q_l),
 // eh = E_DH / (q_k q_l) (the excluded volume does not depend on charge).
 //
-// Layout: one workgroup per core i, its charge sites dealt over the
-// threads; the partner cores of i (CSR list, both directions) staged one
-// at a time in LDS.  Every pair is evaluated from both sides, so each
-// output has one owner and no atomics: the results are deterministic.
+// Layout: a workgroup owns a block of KB charges of a core i (blockIdx.y),
+// one per lane; the partner charges of the core (CSR list, both directions)
+// pass through LDS as one stream of records, dealt over the workgroup's
+// wavefronts (and, for KB < 64, over the lanes' groups of KB), and their
+// partial sums are added in a fixed order at the end.  Every pair is
+// evaluated from both sides, so each site's output has one owner and there
+// are no atomics: the results are deterministic.  A core's energy needs its
+// blocks' parts: with a work buffer each block leaves its part there and
+// k_cc_esum adds them, without one a single workgroup takes all the core's
+// blocks in turn (bd_cc_forward).
+//
+// What bounds it: FP32 (FP64) VALU issue, ~40 instructions a pair forward and
+// ~55 backward.  With one 256-thread workgroup per core (300 charges: three
+// rounds, the last with 44 lanes) 50 cores kept 50 of 256 CUs at 4 wavefronts
+// each, and the IEEE root, quotient and expf of a pair were most of its
+// instructions.  50 cores of 300 charges, forward and backward: 3689 -> 152 us
+// in FP32, 4734 -> 334 us in FP64; 300 cores 3982 -> 741 and 6277 -> 1629 us.
 // Templated on the arithmetic (float for the FP32 force passes of the
 // differentiable trajectory, double for its FP64 checks).
 #include <hip/hip_runtime.h>
@@ -39,164 +52,222 @@
 namespace bd {
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kMaxSites = 640;  // charges per core held in LDS
+constexpr int kThreads = 1024;
+constexpr int kMaxSites = 640;  // charges per core
+constexpr int kTile = 1024;     // partner records in LDS at a time
 
 struct CCParams {
-    double ke, kappa, kex, sigma, cut_ev;
+    double ke, kappa, kex, sigma;
+};
+
+// The distance terms of a pair in the two arithmetics: 1/d and d from d2,
+// exp(-kappa d), and the reference's d <= 8 as a test of d2 (the largest
+// number whose correctly rounded root is 8).
+template <typename T> struct Arith;
+template <> struct Arith<float> {
+    static constexpr float kD8 = 0x1.000002p+6f;
+    static __device__ __forceinline__ float rsqrt(float f) {  // v_rsq_f32 and one Newton step
+        const float y = __builtin_amdgcn_rsqf(f);
+        return __builtin_fmaf(0.5f * y, __builtin_fmaf(-f * y, y, 1.0f), y);
+    }
+    // e^x = 2^(x log2 e), the product's rounding error carried into a factor
+    static __device__ __forceinline__ float exp(float x) {
+        const float p = x * 0x1.715476p+0f;
+        const float e = __builtin_fmaf(x, 0x1.4ae0cp-26f, __builtin_fmaf(x, 0x1.715476p+0f, -p));
+        const float y = __builtin_amdgcn_exp2f(p);
+        return __builtin_fmaf(y, e * 0x1.62e43p-1f, y);
+    }
+};
+template <> struct Arith<double> {
+    static constexpr double kD8 = 0x1.0000000000001p+6;
+    static __device__ __forceinline__ double rsqrt(double f) { return rsqrt_f64(f); }
+    // below -745 the result is 0; exp_neg takes arguments above -800
+    static __device__ __forceinline__ double exp(double x) { return exp_neg(fmax(x, -800.0)); }
 };
 
 template <typename T>
 struct PairTerms {
-    T g, gp, e, gh, eh;  // g, g', energy, g_DH/(q_k q_l), E_DH/(q_k q_l)
+    T id, g, gp, e, gh, eh;  // 1/d, g, g', energy, g_DH/(q_k q_l), E_DH/(q_k q_l)
 };
 
-template <typename T>
-__device__ __forceinline__ PairTerms<T> pair_terms(T d, T qkql, const CCParams &p) {
-    const T id = T(1) / d;
+template <typename T, bool GP>
+__device__ __forceinline__ PairTerms<T> pair_terms(T d2, T qkql, const CCParams &p) {
     const T kap = (T)p.kappa, ke = (T)p.ke;
-    const T ex = exp(-kap * d);
+    const T id = Arith<T>::rsqrt(d2), kd = kap * (d2 * id);
     PairTerms<T> r;
-    r.eh = ke * ex * id;
-    r.gh = r.eh * (kap * d + T(1)) * id;
+    r.id = id;
+    r.eh = ke * Arith<T>::exp(-kd) * id;
+    r.gh = r.eh * (kd + T(1)) * id;
     r.e = qkql * r.eh;
     r.g = qkql * r.gh;
-    r.gp = -qkql * ke * ex * (kap * kap * d * d + T(2) * kap * d + T(2)) * id * id * id;
-    if (d <= (T)p.cut_ev) {
+    if (GP) r.gp = -qkql * r.eh * (kd * (kd + T(2)) + T(2)) * (id * id);
+    if (d2 <= Arith<T>::kD8) {
         const T sd = (T)p.sigma * id, s2 = sd * sd, s6 = s2 * s2 * s2, s12 = s6 * s6, kex = (T)p.kex;
         r.e += kex * (s12 - s6);
         r.g += kex * (T(12) * s12 - T(6) * s6) * id;
-        r.gp += kex * (T(-156) * s12 + T(42) * s6) * id * id;
+        if (GP) r.gp += kex * (T(-156) * s12 + T(42) * s6) * (id * id);
     }
     return r;
 }
 
-template <typename T>
-__device__ __forceinline__ T block_sum(T v, T *buf) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+template <typename T> struct alignas(4 * sizeof(T)) Rec4 {
+    T x, y, z, w;
+};
+
+// The sums v of the workgroup's slots (SL slots of KB lanes), added in slot
+// order by the first KB NV threads: result of value u of lane k on thread
+// u KB + k.
+template <typename T, int KB, int NV>
+__device__ __forceinline__ T slot_sum(const T (&v)[NV], T *buf) {
+    constexpr int SL = kThreads / KB;
+    const int k = threadIdx.x % KB, s = threadIdx.x / KB;
     __syncthreads();
-    if (lane == 0) buf[w] = v;
+#pragma unroll
+    for (int u = 0; u < NV; u++) buf[(s * NV + u) * KB + k] = v[u];
     __syncthreads();
-    T s = T(0);
-    if (threadIdx.x == 0)
-        for (int k = 0; k < kThreads / 64; k++) s += buf[k];
-    return s;
+    T t = T(0);
+    if (threadIdx.x < KB * NV)
+        for (int i = 0; i < SL; i++) t += buf[i * NV * KB + threadIdx.x];
+    return t;
 }
 
-// f[i][k][3] (written) and e[i] = half the energy of core i's pairs
-template <typename T>
+// f[i][k][3] of the block's charges, and half the energy of its pairs into
+// eo: e[i] where the workgroup takes every block (gridDim.y = 1), else the
+// block's part work[i gridDim.y + block]
+template <typename T, int KB>
 __global__ void __launch_bounds__(kThreads) k_cc_fwd(int Nq, const T *__restrict__ Q, const T *__restrict__ q,
                                                      const int *__restrict__ off, const int *__restrict__ nbr,
-                                                     CCParams p, T *__restrict__ f, T *__restrict__ e) {
-    __shared__ T sQ[3 * kMaxSites], sq[kMaxSites], red[kThreads / 64];
-    const int i = blockIdx.x;
-    constexpr int KP = (kMaxSites + kThreads - 1) / kThreads;
-    T fx[KP], fy[KP], fz[KP], qk[KP], px[KP], py[KP], pz[KP];
+                                                     CCParams p, T *__restrict__ f, T *__restrict__ eo) {
+    constexpr int SL = kThreads / KB;
+    __shared__ Rec4<T> S[kTile];
+    const int i = blockIdx.x, slot = threadIdx.x / KB, s0 = off[i], M = (off[i + 1] - s0) * Nq;
+    static_assert(sizeof(S) >= kThreads * 4 * sizeof(T), "the slots' sums take the records' place");
     T en = T(0);
-    for (int t = 0; t < KP; t++) {
-        const int k = threadIdx.x + t * kThreads;
-        fx[t] = fy[t] = fz[t] = T(0);
-        if (k < Nq) {
-            const T *src = Q + ((size_t)i * Nq + k) * 3;
-            px[t] = src[0]; py[t] = src[1]; pz[t] = src[2];
-            qk[t] = q[k];
-        } else {
-            px[t] = py[t] = pz[t] = qk[t] = T(0);
-        }
-    }
-    for (int s = off[i]; s < off[i + 1]; s++) {
-        const int j = nbr[s];
-        __syncthreads();
-        for (int x = threadIdx.x; x < 3 * Nq; x += kThreads) sQ[x] = Q[(size_t)j * Nq * 3 + x];
-        for (int x = threadIdx.x; x < Nq; x += kThreads) sq[x] = q[x];
-        __syncthreads();
-        for (int t = 0; t < KP; t++) {
-            const int k = threadIdx.x + t * kThreads;
-            if (k >= Nq) continue;
-            for (int l = 0; l < Nq; l++) {
-                const T zx = px[t] - sQ[3 * l], zy = py[t] - sQ[3 * l + 1], zz = pz[t] - sQ[3 * l + 2];
-                const T d = sqrt(zx * zx + zy * zy + zz * zz);
-                const PairTerms<T> r = pair_terms<T>(d, qk[t] * sq[l], p);
-                const T gi = r.g / d;
-                fx[t] += gi * zx;
-                fy[t] += gi * zy;
-                fz[t] += gi * zz;
-                en += T(0.5) * r.e;
+    for (int k0 = blockIdx.y * KB; k0 < Nq; k0 += gridDim.y * KB) {
+        const int k = min(k0 + (int)threadIdx.x % KB, Nq - 1);
+        const T *src = Q + ((size_t)i * Nq + k) * 3;
+        const T px = src[0], py = src[1], pz = src[2], qk = q[k];
+        T v[4] = {T(0), T(0), T(0), T(0)};
+        for (int t0 = 0; t0 < M; t0 += kTile) {
+            const int R = min(M - t0, kTile);
+            __syncthreads();
+            for (int r = threadIdx.x; r < R; r += kThreads) {
+                const int m = t0 + r, l = m % Nq;
+                const T *o = Q + ((size_t)nbr[s0 + m / Nq] * Nq + l) * 3;
+                S[r] = Rec4<T>{o[0], o[1], o[2], q[l]};
+            }
+            __syncthreads();
+#pragma unroll 2
+            for (int r = slot; r < R; r += SL) {
+                const Rec4<T> o = S[r];
+                const T zx = px - o.x, zy = py - o.y, zz = pz - o.z;
+                const PairTerms<T> t = pair_terms<T, false>(zx * zx + zy * zy + zz * zz, qk * o.w, p);
+                const T gi = t.g * t.id;
+                v[0] += gi * zx;
+                v[1] += gi * zy;
+                v[2] += gi * zz;
+                v[3] += t.e;
             }
         }
+        const T sum = slot_sum<T, KB, 4>(v, reinterpret_cast<T *>(S));
+        const int u = threadIdx.x / KB, kk = k0 + threadIdx.x % KB;
+        if (threadIdx.x < 3 * KB && kk < Nq) f[((size_t)i * Nq + kk) * 3 + u] = sum;
+        if (u == 3 && kk < Nq) en += T(0.5) * sum;
     }
-    for (int t = 0; t < KP; t++) {
-        const int k = threadIdx.x + t * kThreads;
-        if (k < Nq) {
-            T *dst = f + ((size_t)i * Nq + k) * 3;
-            dst[0] = fx[t]; dst[1] = fy[t]; dst[2] = fz[t];
-        }
+    // the energy sits in the KB lanes of value 3
+    if (threadIdx.x >= 3 * KB && threadIdx.x < 4 * KB) {
+        for (int o = KB / 2; o > 0; o >>= 1) en += __shfl_down(en, o, KB);
+        if (threadIdx.x == 3 * KB) eo[(size_t)i * gridDim.y + blockIdx.y] = en;
     }
-    const T tot = block_sum(en, red);
-    if (threadIdx.x == 0) e[i] = tot;
+}
+
+// e[i] = the parts of core i in order
+template <typename T>
+__global__ void k_cc_esum(int n_c, int parts, const T *__restrict__ work, T *__restrict__ e) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_c) return;
+    T t = T(0);
+    for (int b = 0; b < parts; b++) t += work[(size_t)i * parts + b];
+    e[i] = t;
 }
 
 // gQ[i][k][3] and gq[i][k] (per-site charge gradient; the template
 // gradient is its sum over cores), both written
-template <typename T>
+template <typename T, int KB>
 __global__ void __launch_bounds__(kThreads) k_cc_bwd(int Nq, const T *__restrict__ Q, const T *__restrict__ q,
                                                      const int *__restrict__ off, const int *__restrict__ nbr,
                                                      CCParams p, const T *__restrict__ gf, const T *__restrict__ ge,
                                                      T *__restrict__ gQ, T *__restrict__ gqs) {
-    __shared__ T sQ[3 * kMaxSites], sL[3 * kMaxSites], sq[kMaxSites];
-    const int i = blockIdx.x;
-    constexpr int KP = (kMaxSites + kThreads - 1) / kThreads;
-    T gx[KP], gy[KP], gz[KP], gqk[KP], qk[KP], px[KP], py[KP], pz[KP], lx[KP], ly[KP], lz[KP];
+    constexpr int SL = kThreads / KB;
+    __shared__ Rec4<T> S[2 * kTile];
+    const int i = blockIdx.x, slot = threadIdx.x / KB, s0 = off[i], M = (off[i + 1] - s0) * Nq;
+    const int k0 = blockIdx.y * KB, k = min(k0 + (int)threadIdx.x % KB, Nq - 1);
+    const size_t ok = ((size_t)i * Nq + k) * 3;
+    const T px = Q[ok], py = Q[ok + 1], pz = Q[ok + 2], lx = gf[ok], ly = gf[ok + 1], lz = gf[ok + 2], qk = q[k];
     const T ei = ge[i];
-    for (int t = 0; t < KP; t++) {
-        const int k = threadIdx.x + t * kThreads;
-        gx[t] = gy[t] = gz[t] = gqk[t] = T(0);
-        if (k < Nq) {
-            const size_t o = ((size_t)i * Nq + k) * 3;
-            px[t] = Q[o]; py[t] = Q[o + 1]; pz[t] = Q[o + 2];
-            lx[t] = gf[o]; ly[t] = gf[o + 1]; lz[t] = gf[o + 2];
-            qk[t] = q[k];
-        } else {
-            px[t] = py[t] = pz[t] = lx[t] = ly[t] = lz[t] = qk[t] = T(0);
-        }
-    }
-    for (int s = off[i]; s < off[i + 1]; s++) {
-        const int j = nbr[s];
-        const T eps = T(0.5) * (ei + ge[j]);
+    T v[4] = {T(0), T(0), T(0), T(0)};
+    for (int t0 = 0; t0 < M; t0 += kTile) {
+        const int R = min(M - t0, kTile);
         __syncthreads();
-        for (int x = threadIdx.x; x < 3 * Nq; x += kThreads) {
-            sQ[x] = Q[(size_t)j * Nq * 3 + x];
-            sL[x] = gf[(size_t)j * Nq * 3 + x];
+        for (int r = threadIdx.x; r < R; r += kThreads) {
+            const int m = t0 + r, l = m % Nq, j = nbr[s0 + m / Nq];
+            const size_t o = ((size_t)j * Nq + l) * 3;
+            S[2 * r] = Rec4<T>{Q[o], Q[o + 1], Q[o + 2], q[l]};
+            S[2 * r + 1] = Rec4<T>{gf[o], gf[o + 1], gf[o + 2], T(0.5) * (ei + ge[j])};
         }
-        for (int x = threadIdx.x; x < Nq; x += kThreads) sq[x] = q[x];
         __syncthreads();
-        for (int t = 0; t < KP; t++) {
-            const int k = threadIdx.x + t * kThreads;
-            if (k >= Nq) continue;
-            for (int l = 0; l < Nq; l++) {
-                const T zx = px[t] - sQ[3 * l], zy = py[t] - sQ[3 * l + 1], zz = pz[t] - sQ[3 * l + 2];
-                const T d = sqrt(zx * zx + zy * zy + zz * zz), id = T(1) / d;
-                const T ux = lx[t] - sL[3 * l], uy = ly[t] - sL[3 * l + 1], uz_ = lz[t] - sL[3 * l + 2];
-                const T hx = zx * id, hy = zy * id, hz = zz * id;
-                const T uz = ux * hx + uy * hy + uz_ * hz;
-                const PairTerms<T> r = pair_terms<T>(d, qk[t] * sq[l], p);
-                const T a = r.gp * uz - eps * r.g - r.g * uz * id, b = r.g * id;
-                gx[t] += a * hx + b * ux;
-                gy[t] += a * hy + b * uy;
-                gz[t] += a * hz + b * uz_;
-                gqk[t] += sq[l] * (uz * r.gh + eps * r.eh);
-            }
+        for (int r = slot; r < R; r += SL) {
+            const Rec4<T> o = S[2 * r], w = S[2 * r + 1];
+            const T zx = px - o.x, zy = py - o.y, zz = pz - o.z;
+            const PairTerms<T> t = pair_terms<T, true>(zx * zx + zy * zy + zz * zz, qk * o.w, p);
+            const T ux = lx - w.x, uy = ly - w.y, uz_ = lz - w.z;
+            const T hx = zx * t.id, hy = zy * t.id, hz = zz * t.id;
+            const T uz = ux * hx + uy * hy + uz_ * hz;
+            const T b = t.g * t.id, a = t.gp * uz - w.w * t.g - b * uz;
+            v[0] += a * hx + b * ux;
+            v[1] += a * hy + b * uy;
+            v[2] += a * hz + b * uz_;
+            v[3] += o.w * (uz * t.gh + w.w * t.eh);
         }
     }
-    for (int t = 0; t < KP; t++) {
-        const int k = threadIdx.x + t * kThreads;
-        if (k < Nq) {
-            const size_t o = ((size_t)i * Nq + k) * 3;
-            gQ[o] = gx[t]; gQ[o + 1] = gy[t]; gQ[o + 2] = gz[t];
-            gqs[(size_t)i * Nq + k] = gqk[t];
-        }
+    const T sum = slot_sum<T, KB, 4>(v, reinterpret_cast<T *>(S));
+    const int u = threadIdx.x / KB, kk = k0 + threadIdx.x % KB;
+    if (kk < Nq) {
+        if (u < 3) gQ[((size_t)i * Nq + kk) * 3 + u] = sum;
+        else if (u == 3) gqs[(size_t)i * Nq + kk] = sum;
     }
+}
+
+// charges per block: 16, with fewer idle lanes in the last block (300 charges:
+// 304 lanes against 320) and more workgroups, until the blocks of 64 alone
+// are several rounds of workgroups, which then read half the records from
+// LDS.  Forward and backward with 64 / 16, us: 20 cores FP32 142 / 110, FP64
+// 270 / 158; 50 cores 158 / 152, 306 / 334; 120 cores 382 / 332, 826 / 731;
+// 300 cores 741 / 760, 1629 / 1726.
+int block_charges(int n_c, int Nq) { return n_c * ((Nq + 63) / 64) >= 1000 ? 64 : 16; }
+
+template <typename T>
+void cc_fwd(int n_c, int Nq, const void *Q, const void *q, const int *off, const int *nbr, const CCParams &p, void *f,
+            void *e, void *work, hipStream_t s) {
+    const int KB = work ? block_charges(n_c, Nq) : 64, nb = work ? (Nq + KB - 1) / KB : 1;
+    auto *eo = static_cast<T *>(work ? work : e);
+    if (KB == 64)
+        k_cc_fwd<T, 64><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (T *)f, eo);
+    else
+        k_cc_fwd<T, 16><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (T *)f, eo);
+    if (work) k_cc_esum<T><<<(n_c + 255) / 256, 256, 0, s>>>(n_c, nb, eo, (T *)e);
+}
+
+template <typename T>
+void cc_bwd(int n_c, int Nq, const void *Q, const void *q, const int *off, const int *nbr, const CCParams &p,
+            const void *gf, const void *ge, void *gQ, void *gqs, hipStream_t s) {
+    const int KB = block_charges(n_c, Nq), nb = (Nq + KB - 1) / KB;
+    if (KB == 64)
+        k_cc_bwd<T, 64><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (const T *)gf,
+                                                           (const T *)ge, (T *)gQ, (T *)gqs);
+    else
+        k_cc_bwd<T, 16><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (const T *)gf,
+                                                           (const T *)ge, (T *)gQ, (T *)gqs);
 }
 
 int cc_fail(int code, const char *fmt, ...) {
@@ -223,22 +294,24 @@ using namespace bd;
 
 extern "C" {
 
-int bd_cc_forward(int fp64, int n_c, int Nq, const void *Q, const void *q, const int *nbr_off, const int *nbr,
-                  double ke, double kappa, double kex, double sigma, void *f, void *e, void *stream) {
+int bd_cc_forward_work(int fp64, int n_c, int Nq, const void *Q, const void *q, const int *nbr_off, const int *nbr,
+                       double ke, double kappa, double kex, double sigma, void *f, void *e, void *work,
+                       void *stream) {
     int r = cc_check(n_c, Nq, Q, q, nbr_off, nbr);
     if (r) return r;
     if (!f || !e) return cc_fail(BD_E_ARG, "null output");
-    const CCParams p{ke, kappa, kex, sigma, 8.0};
+    const CCParams p{ke, kappa, kex, sigma};
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (fp64)
-        k_cc_fwd<double><<<n_c, kThreads, 0, s>>>(Nq, (const double *)Q, (const double *)q, nbr_off, nbr, p,
-                                                  (double *)f, (double *)e);
-    else
-        k_cc_fwd<float><<<n_c, kThreads, 0, s>>>(Nq, (const float *)Q, (const float *)q, nbr_off, nbr, p,
-                                                 (float *)f, (float *)e);
+    if (fp64) cc_fwd<double>(n_c, Nq, Q, q, nbr_off, nbr, p, f, e, work, s);
+    else cc_fwd<float>(n_c, Nq, Q, q, nbr_off, nbr, p, f, e, work, s);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return cc_fail(BD_E_HIP, "k_cc_fwd: %s", hipGetErrorString(err));
     return BD_OK;
+}
+
+int bd_cc_forward(int fp64, int n_c, int Nq, const void *Q, const void *q, const int *nbr_off, const int *nbr,
+                  double ke, double kappa, double kex, double sigma, void *f, void *e, void *stream) {
+    return bd_cc_forward_work(fp64, n_c, Nq, Q, q, nbr_off, nbr, ke, kappa, kex, sigma, f, e, nullptr, stream);
 }
 
 int bd_cc_backward(int fp64, int n_c, int Nq, const void *Q, const void *q, const int *nbr_off, const int *nbr,
@@ -247,16 +320,10 @@ int bd_cc_backward(int fp64, int n_c, int Nq, const void *Q, const void *q, cons
     int r = cc_check(n_c, Nq, Q, q, nbr_off, nbr);
     if (r) return r;
     if (!gf || !ge || !gQ || !gq_sites) return cc_fail(BD_E_ARG, "null argument");
-    const CCParams p{ke, kappa, kex, sigma, 8.0};
+    const CCParams p{ke, kappa, kex, sigma};
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (fp64)
-        k_cc_bwd<double><<<n_c, kThreads, 0, s>>>(Nq, (const double *)Q, (const double *)q, nbr_off, nbr, p,
-                                                  (const double *)gf, (const double *)ge, (double *)gQ,
-                                                  (double *)gq_sites);
-    else
-        k_cc_bwd<float><<<n_c, kThreads, 0, s>>>(Nq, (const float *)Q, (const float *)q, nbr_off, nbr, p,
-                                                 (const float *)gf, (const float *)ge, (float *)gQ,
-                                                 (float *)gq_sites);
+    if (fp64) cc_bwd<double>(n_c, Nq, Q, q, nbr_off, nbr, p, gf, ge, gQ, gq_sites, s);
+    else cc_bwd<float>(n_c, Nq, Q, q, nbr_off, nbr, p, gf, ge, gQ, gq_sites, s);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return cc_fail(BD_E_HIP, "k_cc_bwd: %s", hipGetErrorString(err));
     return BD_OK;

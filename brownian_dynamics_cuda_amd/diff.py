@@ -98,7 +98,7 @@ def _body(f, a, b, c):
 
 class CoreCorePairs(torch.autograd.Function):
     """Core-core charge forces and energies (func.cpp:1489-1566) on the HIP
-    kernels of bd_adjoint.hip: forward bd_cc_forward, backward the adjoint
+    kernels of bd_adjoint.hip: forward bd_cc_forward_work, backward the adjoint
     kernel bd_cc_backward (gradients with respect to the charge positions
     and the charge template)."""
 
@@ -110,10 +110,12 @@ class CoreCorePairs(torch.autograd.Function):
         n_c, nq = Q.shape[0], Q.shape[1]
         f = torch.empty_like(Q)
         e = torch.empty(n_c, dtype=Q.dtype, device=Q.device)
+        work = torch.empty(n_c, (nq + 15) // 16, dtype=Q.dtype, device=Q.device)
         fp64 = 1 if Q.dtype == torch.float64 else 0
         stream = C.c_void_p(torch.cuda.current_stream(Q.device).cuda_stream)
-        rc = lib.bd_cc_forward(fp64, n_c, nq, Q.data_ptr(), q.data_ptr(), off.data_ptr(),
-                               nbr.data_ptr(), *consts, f.data_ptr(), e.data_ptr(), stream)
+        rc = lib.bd_cc_forward_work(fp64, n_c, nq, Q.data_ptr(), q.data_ptr(), off.data_ptr(),
+                                    nbr.data_ptr(), *consts, f.data_ptr(), e.data_ptr(),
+                                    work.data_ptr(), stream)
         if rc:
             raise E.BDError(f"bd_cc_forward: {lib.bd_last_error().decode()}")
         ctx.save_for_backward(Q, q, off, nbr)

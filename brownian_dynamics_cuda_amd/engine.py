@@ -87,6 +87,8 @@ API = {
     "bd_set_refine": ([C.c_void_p, C.c_int], C.c_int),
     "bd_cc_forward": ([C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
                       + [C.c_double] * 4 + [C.c_void_p] * 3, C.c_int),
+    "bd_cc_forward_work": ([C.c_int, C.c_int, C.c_int] + [C.c_void_p] * 4 + [C.c_double] * 4
+                           + [C.c_void_p] * 4, C.c_int),
     "bd_cc_backward": ([C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
                        + [C.c_double] * 4 + [C.c_void_p] * 5, C.c_int),
     "bd_cholesky": ([C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int, _ip, C.c_void_p],

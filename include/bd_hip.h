@@ -241,6 +241,13 @@ int bd_cholesky_noalloc(int m, const double *D, int ldd, double *L, int ldl, int
 int bd_cc_forward(int fp64, int n_c, int Nq, const void *Q, const void *q, const int *nbr_off,
                   const int *nbr, double ke, double kappa, double kex, double sigma, void *f,
                   void *e, void *stream);
+/* The same with a work buffer of n_c * BD_CC_WORK(Nq) numbers of the
+ * arithmetic (device memory, not read before it is written), with which the
+ * charges of a core spread over several workgroups; NULL: bd_cc_forward. */
+#define BD_CC_WORK(Nq) (((Nq) + 15) / 16)
+int bd_cc_forward_work(int fp64, int n_c, int Nq, const void *Q, const void *q, const int *nbr_off,
+                       const int *nbr, double ke, double kappa, double kex, double sigma, void *f,
+                       void *e, void *work, void *stream);
 int bd_cc_backward(int fp64, int n_c, int Nq, const void *Q, const void *q, const int *nbr_off,
                    const int *nbr, double ke, double kappa, double kex, double sigma,
                    const void *gf, const void *ge, void *gQ, void *gq_sites, void *stream);

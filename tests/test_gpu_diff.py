@@ -95,6 +95,48 @@ def test_core_core_kernel_and_adjoint():
     assert rel_err(e32.double().cpu().numpy(), outs["dense"][1]) <= 1e-5
 
 
+@pytest.mark.parametrize("n_c,nq", [(1, 1), (2, 16), (3, 17), (3, 64), (2, 65), (4, 300), (2, 640), (200, 5)])
+def test_core_core_blocks(n_c, nq):
+    """Sizes around the blocks of 16 and 64 charges and the record tiles of
+    the core-core kernels, cores without partners among them, with and
+    without a work buffer, against the dense sums in FP64."""
+    import ctypes as C
+    from brownian_dynamics_cuda_amd import diff as Df
+    g = torch.Generator().manual_seed(100 * n_c + nq)
+    dev = torch.device("cuda")
+    r = torch.stack([9.0 * torch.arange(n_c, dtype=torch.float64)] + 2 * [torch.zeros(n_c, dtype=torch.float64)], 1)
+    Q0 = (r[:, None] + 3.0 * torch.rand(n_c, nq, 3, generator=g, dtype=torch.float64)).to(dev)
+    q0 = (2.0 * torch.rand(nq, generator=g, dtype=torch.float64) - 1.0).to(dev)
+    pairs = [(i, i + 1) for i in range(n_c - 1) if i % 3 != 2]
+    nb = [[] for _ in range(n_c)]
+    for i, j in pairs:
+        nb[i].append(j)
+        nb[j].append(i)
+    off = torch.tensor(np.r_[0, np.cumsum([len(x) for x in nb])], dtype=torch.int32, device=dev)
+    nbr = torch.tensor([v for x in nb for v in sorted(x)] or [0], dtype=torch.int32, device=dev)
+    consts = (0.7, 1.2, 0.03, 1.8)
+    gf = torch.randn(Q0.shape, generator=g, dtype=torch.float64).to(dev)
+    ge = torch.randn(n_c, generator=g, dtype=torch.float64).to(dev)
+    outs = {}
+    for name, fn in (("hip", lambda Q, q: Df.CoreCorePairs.apply(Q, q, off, nbr, consts)),
+                     ("dense", lambda Q, q: dense_cc(Q, q, pairs, consts))):
+        Q = Q0.clone().requires_grad_(True)
+        q = q0.clone().requires_grad_(True)
+        f, e = fn(Q, q)
+        gQ, gq = torch.autograd.grad((f * gf).sum() + (e * ge).sum() + 0.0 * q.sum(), [Q, q], allow_unused=True)
+        outs[name] = [(torch.zeros_like(Q) if t is None else t).detach().cpu().numpy() for t in (f, e, gQ, gq)]
+    for k_, (x, y) in enumerate(zip(outs["hip"], outs["dense"])):
+        assert rel_err(x, y) <= 1e-12, k_
+    # bd_cc_forward, without a work buffer
+    f, e = torch.empty_like(Q0), torch.empty(n_c, dtype=torch.float64, device=dev)
+    rc = E.load_library().bd_cc_forward(1, n_c, nq, Q0.data_ptr(), q0.data_ptr(), off.data_ptr(), nbr.data_ptr(),
+                                        *consts, f.data_ptr(), e.data_ptr(),
+                                        C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    assert rel_err(f.cpu().numpy(), outs["dense"][0]) <= 1e-12
+    assert rel_err(e.cpu().numpy(), outs["dense"][1]) <= 1e-12
+
+
 def thermalized(fib, st, steps, seed=777):
     """positions and frames `steps` oracle steps into a trajectory, and the
     generator to continue it"""
