@@ -92,6 +92,7 @@ __device__ __forceinline__ void tri_index(int idx, int &i, int &j) {
     j = idx - r * (r + 1) / 2;
 }
 
+constexpr int kDiagLds = 5376;  // LDS of diag_factor_inv, doubles
 __device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, double *A, int ld, int d0, double *Linv,
                                                 int *neg);
 
@@ -102,7 +103,7 @@ template <bool FACTOR>
 __global__ void __launch_bounds__(256) k_rpy(Stat s, Geo g, const double *rad_all, double *A, int m, int ld,
                                              double a1, double a2, int *neg, double *Linv) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *neg = 0;  // negative-pivot count of the factor that follows
-    __shared__ double T[(FACTOR ? 2 : 1) * TB * LDP];
+    __shared__ double T[FACTOR ? kDiagLds : TB * LDP];
     int ti, tj;
     tri_index(blockIdx.x, ti, tj);
     const int r0 = ti * TB, c0 = tj * TB, nhi = m / 3;
@@ -576,21 +577,21 @@ __device__ __forceinline__ void below_rows(double (&x)[16], const double (&u)[4]
                    [c3] "n"(pos16(K + 3)));
 }
 
-// LDS of the elimination: two tiles of pitch LDP, the second of which may
-// hold the tile itself until it is in registers
+// LDS of the elimination; the tile itself may lie anywhere in it until it is
+// in registers
 struct DiagLds {
     double *base;
-    // panel buffers W(b, j), j >= b, and E(b, j), j <= b, 256 each
+    // panel buffers W(b, j), j >= b, and E(b, j), j <= b, 256 each; the last
+    // block row's E takes the place of the blocks handed to it
     __device__ __forceinline__ double *W(int b, int j) const { return base + (b * (9 - b) / 2 + j - b) * 256; }
     __device__ __forceinline__ double *E(int b, int j) const { return base + (10 + b * (b + 1) / 2 + j) * 256; }
     // blocks of the next block row, element [18 c + row]: lane group q of
-    // wavefront 1, q = 4 wavefront 0
-    __device__ __forceinline__ double *next(int q) const { return base + 5120 + 288 * q; }
-    __device__ __forceinline__ double *R() const { return base + 6560; }  // 1/|f|, 64
-    __device__ __forceinline__ double *S() const { return base + 6624; }  // 1/sqrt(|f|), 64
+    // wavefront 1, q = 3 wavefront 0
+    __device__ __forceinline__ double *next(int q) const { return base + 4096 + 288 * q; }
+    __device__ __forceinline__ double *R() const { return base + 5248; }  // 1/|f|, 64
+    __device__ __forceinline__ double *S() const { return base + 5312; }  // 1/sqrt(|f|), 64
 };
 constexpr int kNextPitch = 18;
-static_assert(6688 <= 2 * TB * LDP, "the elimination fits two tiles");
 
 // the operand register of a panel: lane (k, c) holds row k, column c
 __device__ __forceinline__ double panel_op(const double *S, int p) {
@@ -740,7 +741,7 @@ __device__ __forceinline__ void below_row(dbl4 (&Z)[6], const DiagLds &l) {
     __syncthreads();
     below_panel<B, U, B + 1, B + 1>(Z, l, 3);
     if constexpr (U == 0) {
-        put_next(l, 4, Z[B == 0 ? 0 : B == 1 ? 2 : 4]);
+        put_next(l, 3, Z[B == 0 ? 0 : B == 1 ? 2 : 4]);
         put_next(l, B == 2 ? 1 : 0, Z[B == 0 ? 1 : B == 1 ? 3 : 5]);
     } else {
         put_next(l, B == 2 ? 0 : 1, Z[B == 0 ? 0 : B == 1 ? 2 : 4]);
@@ -750,8 +751,9 @@ __device__ __forceinline__ void below_row(dbl4 (&Z)[6], const DiagLds &l) {
     if constexpr (B < 2) below_panel<B, U, B + 2, 3>(Z, l, 3);
 }
 
-// Called by all four wavefronts.  lds: two tiles; T, one of them, holds the
-// tile (pitch LDP) at (d0, d0), of which the lower triangle is read.  L goes
+// Called by all four wavefronts.  lds: kDiagLds doubles; T, LDS that may
+// overlap it, holds the tile (pitch LDP) at (d0, d0), of which the lower
+// triangle is read.  L goes
 // to A (lower triangle), inv(L), row-major 64x64 with zeros above its
 // diagonal, to Linv.
 __device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, double *A, int ld, int d0, double *Linv,
@@ -766,7 +768,7 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, do
         __syncthreads();
 #pragma unroll 1
         for (int b = 0; b < 4; b++) {
-            if (b) load_rows(w, l.next(4) + kNextPitch * c);
+            if (b) load_rows(w, l.next(3) + kNextPitch * c);
             double y = 0.0, f = 0.0, n = 0.0;
             pivot_panel<0>(w, r, y, f, n, l, b);
             pivot_panel<1>(w, r, y, f, n, l, b);
@@ -884,26 +886,28 @@ __device__ __forceinline__ void tile_update(const double *Pi, const double *Pj, 
                 C[(size_t)r * ld + c] = cv[mi][ni][v] + -1.0 * (double)acc[mi][ni][v];
             }
 }
-// C -= P P^T for a diagonal tile: read into T (LDS) first, left there for the
-// factor (keep) or stored, its lower triangle
+// C -= P P^T for a diagonal tile in LDS
 template <int MODE>
-__device__ __forceinline__ void diag_tile_update(const double *P, double *T, double *C, int ld, bool keep) {
-    dbl2 v[PERT];
-    tile_to_regs(C, ld, v);
-    regs_to_lds(v, T);
-    __syncthreads();
+__device__ __forceinline__ void diag_tile_update(const double *P, double *C) {
     if (MODE == 0) {
-        syrk_lower(P, T);
+        syrk_lower(P, C);
     } else {
         typename AccOf<MODE>::T acc[2][2];
         for (int a = 0; a < 2; a++)
             for (int b = 0; b < 2; b++) acc[a][b] = {};
         tile_mma<MODE>(P, P, acc);
-        acc_to_lds(T, acc, -1.0, false);
+        acc_to_lds(C, acc, -1.0, false);
     }
-    if (keep) return;
-    __syncthreads();
-    store_tile(C, ld, 0, 0, T, true);
+}
+// A tile from LDS by wavefronts 2 and 3, which have two of syrk_lower's
+// blocks where 0 and 1 have three
+__device__ __forceinline__ void store_tile_half(double *dst, int ld, const double *S) {
+    if (threadIdx.x < NTHR / 2) return;
+#pragma unroll
+    for (int i = 0; i < 2 * PERT; i++) {
+        const int e = threadIdx.x - NTHR / 2 + i * (NTHR / 2), r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        *reinterpret_cast<dbl2 *>(dst + (size_t)r * ld + c) = dbl2{S[r * LDP + c], S[r * LDP + c + 1]};
+    }
 }
 
 // Trailing tiles of block column kb restricted to the first jcols trailing
@@ -959,7 +963,8 @@ __global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int 
         dbl2 vw[PERT];
         tile_to_regs(Linv + (size_t)kb * TB * TB, TB, vw);
         tile_to_regs(A + (size_t)ib * TB * ld + kb * TB, ld, vi);
-        if (!diag) tile_to_regs(A + (size_t)jb * TB * ld + kb * TB, ld, vj);
+        // the column's panel block, or the diagonal target tile
+        tile_to_regs(diag ? A + (size_t)ib * TB * ld + jb * TB : A + (size_t)jb * TB * ld + kb * TB, ld, vj);
         regs_to_lds(vw, S0);
         regs_to_lds(vi, S1);
     }
@@ -970,13 +975,15 @@ __global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int 
     __syncthreads();
     if (diag) {
         panel_to_lds(S1, pi);
+        regs_to_lds(vj, S0);
         __syncthreads();
-        if (jj == 0) store_tile(A, ld, kb * TB, ib * TB, S1, false);
-        diag_tile_update<MODE>(S1, S0, A + (size_t)ib * TB * ld + jb * TB, ld, ii == 0);
-        if (ii == 0) {
-            __syncthreads();
+        diag_tile_update<MODE>(S1, S0);
+        if (jj == 0) store_tile_half(A + (size_t)kb * TB * ld + ib * TB, ld, S1);
+        __syncthreads();
+        if (ii == 0)
             diag_factor_inv(S, S0, A, ld, ib * TB, Linv + (size_t)ib * TB * TB, neg);
-        }
+        else
+            store_tile(A, ld, ib * TB, jb * TB, S0, true);
         return;
     }
     regs_to_lds(vj, S1);
@@ -1035,22 +1042,24 @@ __global__ void __launch_bounds__(256, 2) k_update(double *A, int ld, int kb, in
     if (lb == 0) __builtin_amdgcn_s_setprio(3);
     {
         // the parked panel tiles L_ib,kb and L_jb,kb
+        // (the target tile in place of the second on the diagonal)
         dbl2 vi[PERT], vj[PERT];
         tile_to_regs(A + (size_t)kb * TB * ld + ib * TB, ld, vi);
-        if (!diag) tile_to_regs(A + (size_t)kb * TB * ld + jb * TB, ld, vj);
+        tile_to_regs(diag ? A + (size_t)ib * TB * ld + jb * TB : A + (size_t)kb * TB * ld + jb * TB, ld, vj);
         regs_to_lds(vi, S1);
-        if (!diag) regs_to_lds(vj, S0);
+        regs_to_lds(vj, S0);
     }
     __syncthreads();
     if (!diag) {
         tile_update<MODE>(S1, S0, A + (size_t)ib * TB * ld + jb * TB, ld);
         return;
     }
-    diag_tile_update<MODE>(S1, S0, A + (size_t)ib * TB * ld + jb * TB, ld, ii == 0);
-    if (ii == 0) {
-        __syncthreads();
+    diag_tile_update<MODE>(S1, S0);
+    __syncthreads();
+    if (ii == 0)
         diag_factor_inv(S, S0, A, ld, ib * TB, Linv + (size_t)ib * TB * TB, neg);
-    }
+    else
+        store_tile(A, ld, ib * TB, jb * TB, S0, true);
 }
 
 // Trailing update of a super-panel: block columns k0 .. k0+nb-1 are
@@ -1063,9 +1072,15 @@ __global__ void __launch_bounds__(256, 2) k_update(double *A, int ld, int kb, in
 // Workgroups are grouped in 8x8 blocks of tiles, 64 consecutive workgroups
 // per block, so the panel tiles of a block's 8 rows and 8 columns are
 // shared through the L2; workgroups past the triangle or the edge exit.
+// Workgroup 0, dispatched first, goes on to factor and invert its tile
+// (j0, j0), which the next panel begins with, beside the others' updates (a
+// launch of its own took 21 us per super-panel: 0.39 of 12.1 ms a step at 500
+// nucleosomes).  k_trail_pk and k_trail_bf do the same.
 template <int MODE>
-__global__ void __launch_bounds__(256, 2) k_trail(double *A, int ld, int k0, int nb, int j0, int nt) {
-    __shared__ double As[TB * LDP], Bs[TB * LDP];
+__global__ void __launch_bounds__(256, 2) k_trail(double *A, int ld, int k0, int nb, int j0, int nt, double *Linv,
+                                                  int *neg) {
+    __shared__ double S[2 * TB * LDP];
+    double *As = S, *Bs = S + TB * LDP;
     int SI, SJ;
     tri_index(blockIdx.x >> 6, SI, SJ);
     const int ib = j0 + 8 * SI + ((blockIdx.x >> 3) & 7), jb = j0 + 8 * SJ + (blockIdx.x & 7);
@@ -1096,7 +1111,8 @@ __global__ void __launch_bounds__(256, 2) k_trail(double *A, int ld, int k0, int
     __syncthreads();
     acc_to_lds(As, acc, -1.0, false);
     __syncthreads();
-    store_tile(A, ld, ib * TB, jb * TB, As, diag);
+    if (blockIdx.x == 0) diag_factor_inv(S, As, A, ld, j0 * TB, Linv + (size_t)j0 * TB * TB, neg);
+    else store_tile(A, ld, ib * TB, jb * TB, As, diag);
 }
 
 // Three-slice BF16 trailing update with the panel tiles split once.  Split
@@ -1244,7 +1260,8 @@ __device__ __forceinline__ void bf_body(const __bf16 *sp, int ra, int rbw, int n
 // Workgroups go round-robin over the eight XCDs (b % 8); XCD x takes groups
 // x, x + 8, ... of 8x8 blocks, 64 consecutive workgroups of its own per
 // group, so a group's 16 row and 16 column panel tiles are read into one L2.
-__global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __bf16 *sp, int nb, int j0, int nt) {
+__global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __bf16 *sp, int nb, int j0, int nt,
+                                                     double *Linv, int *neg) {
     __shared__ __attribute__((aligned(16))) __bf16 S[48 * 512];
     const int S2 = (nt - j0 + 1) / 2, SG = (S2 + 7) / 8, l = blockIdx.x >> 3, G = (l >> 6) * 8 + (blockIdx.x & 7);
     if (G >= SG * (SG + 1) / 2) return;
@@ -1263,10 +1280,15 @@ __global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __
         for (int b = 0; b < 4; b++) acc[a][b] = flt4{0.f, 0.f, 0.f, 0.f};
     if (IB == JB) bf_body<true>(sp, ra, rbw, nb, nrow, S, w, lane, active, acc);
     else bf_body<false>(sp, ra, rbw, nb, nrow, S, w, lane, active, acc);
-    if (!active) return;
+    if (!active && blockIdx.x) return;
     const int i16 = lane & 15, k4 = lane >> 4;
     // C -= acc in place, a row of 16x16 blocks at a time: loads, then stores
-    // (a diagonal tile keeps its upper triangle)
+    // (a diagonal tile keeps its upper triangle; the first tile goes to LDS,
+    // for its factor)
+    double *T = reinterpret_cast<double *>(S);
+    const bool keep = blockIdx.x == 0 && w == 0;
+    static_assert(sizeof(S) >= kDiagLds * sizeof(double) && sizeof(S) >= TB * LDP * sizeof(double), "LDS of the factor");
+    if (active)
 #pragma unroll
     for (int mi = 0; mi < 4; mi++) {
         double cv[4][4];
@@ -1283,8 +1305,14 @@ __global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __
             for (int v = 0; v < 4; v++) {
                 const int r = 16 * mi + 4 * k4 + v, c = 16 * ni + i16;
                 if (ib == jb && c > r) continue;
-                A[(size_t)(ib * TB + r) * ld + jb * TB + c] = cv[ni][v] + -1.0 * (double)acc[mi][ni][v];
+                const double x = cv[ni][v] + -1.0 * (double)acc[mi][ni][v];
+                if (keep) T[r * LDP + c] = x;
+                else A[(size_t)(ib * TB + r) * ld + jb * TB + c] = x;
             }
+    }
+    if (blockIdx.x == 0) {
+        __syncthreads();
+        diag_factor_inv(T, T, A, ld, j0 * TB, Linv + (size_t)j0 * TB * TB, neg);
     }
 }
 
@@ -1400,7 +1428,8 @@ __device__ __forceinline__ void pk_body(const double *pk, int ra, int rbw, int n
     }
 }
 template <int MODE>
-__global__ void __launch_bounds__(256, 2) k_trail_pk(double *A, int ld, const double *pk, int nb, int j0, int nt) {
+__global__ void __launch_bounds__(256, 2) k_trail_pk(double *A, int ld, const double *pk, int nb, int j0, int nt,
+                                                     double *Linv, int *neg) {
     __shared__ __attribute__((aligned(16))) double S[2 * 32 * 128];
     const int S2 = (nt - j0 + 1) / 2, SG = (S2 + 7) / 8, l = blockIdx.x >> 3, G = (l >> 6) * 8 + (blockIdx.x & 7);
     if (G >= SG * (SG + 1) / 2) return;
@@ -1420,10 +1449,12 @@ __global__ void __launch_bounds__(256, 2) k_trail_pk(double *A, int ld, const do
         for (int b = 0; b < 4; b++) acc[a][b] = V{};
     if (IB == JB) pk_body<MODE, true>(pk, ra, rbw, nb, nrow, S, w, lane, active, acc);
     else pk_body<MODE, false>(pk, ra, rbw, nb, nrow, S, w, lane, active, acc);
-    if (!active) return;
+    if (!active && blockIdx.x) return;
     const int i16 = lane & 15, k4 = lane >> 4;
     // C -= acc in place (row of register v: l/16 + 4v for the FP64 MFMA,
     // 4(l/16) + v for the FP32 one), a row of 16x16 blocks at a time
+    const bool keep = blockIdx.x == 0 && w == 0;  // the first tile goes to LDS, for its factor
+    if (active)
 #pragma unroll
     for (int mi = 0; mi < 4; mi++) {
         double cv[4][4];
@@ -1440,16 +1471,22 @@ __global__ void __launch_bounds__(256, 2) k_trail_pk(double *A, int ld, const do
             for (int v = 0; v < 4; v++) {
                 const int r = 16 * mi + (MODE == 0 ? k4 + 4 * v : 4 * k4 + v), c = 16 * ni + i16;
                 if (ib == jb && c > r) continue;
-                A[(size_t)(ib * TB + r) * ld + jb * TB + c] = cv[ni][v] + -1.0 * (double)acc[mi][ni][v];
+                const double x = cv[ni][v] + -1.0 * (double)acc[mi][ni][v];
+                if (keep) S[r * LDP + c] = x;
+                else A[(size_t)(ib * TB + r) * ld + jb * TB + c] = x;
             }
+    }
+    static_assert(sizeof(S) >= kDiagLds * sizeof(double), "LDS of the factor");
+    if (blockIdx.x == 0) {
+        __syncthreads();
+        diag_factor_inv(S, S, A, ld, j0 * TB, Linv + (size_t)j0 * TB * TB, neg);
     }
 }
 
 // Factor and inverse of the diagonal tile (d, d) by one workgroup (the
-// tile after a super-panel's trailing update, or the first tile of a
-// caller's matrix); clear != 0 also restarts the negative-pivot count.
+// first tile of a large or a caller's matrix); clear != 0 also restarts the negative-pivot count.
 __global__ void __launch_bounds__(256) k_diag(double *A, int ld, int d, double *Linv, int *neg, int clear) {
-    __shared__ double T[2 * TB * LDP];
+    __shared__ double T[kDiagLds];
     if (clear && threadIdx.x == 0) *neg = 0;
     load_tile(A, ld, d * TB, d * TB, T);
     __syncthreads();
@@ -1668,16 +1705,16 @@ void chol_trail(const CholWork &c, int k0, int nb, hipStream_t q) {
         if constexpr (MODE == 2) {
             __bf16 *sp = static_cast<__bf16 *>(c.sp);
             k_split3<<<(nt - j0) * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, sp);
-            k_trail_bf<<<grid, 256, 0, q>>>(c.A, c.ld, sp, nb, j0, nt);
+            k_trail_bf<<<grid, 256, 0, q>>>(c.A, c.ld, sp, nb, j0, nt, c.Linv, c.neg);
         } else {
             double *pk = static_cast<double *>(c.sp);
             k_pack64<<<(nt - j0) * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, pk);
-            k_trail_pk<MODE><<<grid, 256, 0, q>>>(c.A, c.ld, pk, nb, j0, nt);
+            k_trail_pk<MODE><<<grid, 256, 0, q>>>(c.A, c.ld, pk, nb, j0, nt, c.Linv, c.neg);
         }
         return;
     }
     const int SM = (nt - j0 + 7) / 8;
-    k_trail<MODE><<<SM * (SM + 1) / 2 * 64, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, nt);
+    k_trail<MODE><<<SM * (SM + 1) / 2 * 64, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, nt, c.Linv, c.neg);
 }
 }  // namespace
 
@@ -1686,11 +1723,16 @@ size_t split_bytes(int ld, int nb) {
                     (size_t)(ld / TB) * nb * kPackTile * sizeof(double));
 }
 
+// Super-panels from 84 block columns in FP64 (us a step without / with them,
+// panels of 8: 66 block columns 2129 / 2237, 76 2666 / 2680, 86 3347 / 3351,
+// 99 4471 / 4287, 115 6161 / 5690).  In the reduced modes from 64, where the
+// panel's own columns also gain FP64 arithmetic (FP32 66 block columns 2276 /
+// 2341, 76 2827 / 2804; BF16 66 2506 / 2278).
 int chol_panel_tiles(const CholWork &c) {
     const int nt = c.mpad / TB;
     if (c.panel_tiles > 0) return c.panel_tiles >= 2 && nt > c.panel_tiles ? c.panel_tiles : 0;
     if (c.panel_tiles < 0) return 0;
-    return nt >= 64 ? 8 : 0;
+    return nt >= (c.mode == 0 ? 84 : 64) ? 8 : 0;
 }
 
 void launch_cholesky(const CholWork &c, hipStream_t q, MarkFn mark, void *mark_arg, hipEvent_t gate, int gate_kb) {
@@ -1718,9 +1760,6 @@ void launch_cholesky(const CholWork &c, hipStream_t q, MarkFn mark, void *mark_a
             else if (c.mode == 1) chol_trail<1>(c, k0, NB, q);
             else chol_trail<2>(c, k0, NB, q);
             M_(K_CHOL_TRAIL, 1);
-            M_(K_CHOL_DIAG, 0);
-            k_diag<<<1, 256, 0, q>>>(c.A, c.ld, kend, c.Linv, c.neg, 0);
-            M_(K_CHOL_DIAG, 1);
         }
     }
     // one launch (or two) per block column, each updating the whole trailing matrix

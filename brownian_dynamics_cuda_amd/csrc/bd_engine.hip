@@ -56,7 +56,7 @@ int fail(int code, const char *fmt, ...) {
 const char *kKernelNames[K_COUNT] = {
     "sites", "mech", "linker", "tail", "lh", "core", "cc_list", "cc_work", "rpy",
     "chol_step", "noise", "frames", "betas", "translate",
-    "commit", "energy_reduce", "cc_gather", "chol_trail", "chol_diag", "refine"};
+    "commit", "energy_reduce", "cc_gather", "chol_trail", "refine"};
 
 }  // namespace
 

@@ -32,7 +32,7 @@ void launch_sites(const Stat &s, const Geo &g, const Sites &st, int *cc_count, h
 // (phase 0 before, 1 after); ids are the K_* values below.
 enum KernelId { K_SITES, K_MECH, K_LINKER, K_TAIL, K_LH, K_CORE, K_CCLIST, K_CCWORK,
                 K_RPY, K_CHOL_STEP, K_NOISE, K_FRAMES, K_BETAS, K_TRANSLATE,
-                K_COMMIT, K_EREDUCE, K_CCGATHER, K_CHOL_TRAIL, K_CHOL_DIAG, K_REFINE, K_COUNT };
+                K_COMMIT, K_EREDUCE, K_CCGATHER, K_CHOL_TRAIL, K_REFINE, K_COUNT };
 typedef void (*MarkFn)(void *, int, int);
 // Extra streams of a force pass: after the charge sites, the tail, the
 // linker-histone (then, once mechanics is done, linker) and the core-core
@@ -78,8 +78,9 @@ struct CholWork {
     // two-launch form (k_panel + k_update): about two rounds of workgroups
     // at one per CU
     int split_tiles;
-    // super-panel width in block columns: 0 chooses (8 from 64 block
-    // columns up, none below), -1 never, k >= 2 always k
+    // super-panel width in block columns: 0 chooses (8 from 84 block columns
+    // up in FP64, from 64 in the reduced modes, none below), -1 never, k >= 2
+    // always k
     int panel_tiles;
     // FP64 refinement of B xi in the FP32 / BF16 modes (1: on): xs, the
     // hydrodynamic-set positions D was last assembled from (ld doubles);

@@ -184,9 +184,10 @@ int bd_set_refine(bd_context *ctx, int enable);
 
 /* Schedule of the blocked factor (no counterpart in the reference, which
  * calls cusolverDnDpotrf, func_cuda.cu:3526-3529).  panel_tiles = 0 (the
- * default) chooses: super-panels of 8 block columns of 64 from 64 block
- * columns (D of 4096 rows) up, one block column per launch below; -1 always
- * one block column per launch; k >= 2 super-panels of k block columns
+ * default) chooses: super-panels of 8 block columns of 64 from 84 block
+ * columns (D of 5313 rows) up, from 64 (4033 rows) in the FP32 and BF16
+ * modes, one block column per launch below; -1 always one block column per
+ * launch; k >= 2 super-panels of k block columns
  * whenever the matrix has more than k.  In a super-panel the panel columns
  * are factored with their updates restricted to the panel, then the
  * trailing matrix takes the panel's K = 64k update in one pass.  The

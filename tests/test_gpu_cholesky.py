@@ -69,8 +69,24 @@ def test_blocks_of_the_diagonal_tile(m):
         assert np.array_equal(Ls, np.ldexp(Lg, k // 2))
 
 
+@pytest.mark.parametrize("m,mode", [(5312, E.CHOL_FP64), (5313, E.CHOL_FP64), (4033, E.CHOL_FP32), (4033, E.CHOL_BF16)])
+def test_ends_of_the_super_panels(m, mode):
+    """The first sizes with super-panels (84 and 64 block columns) and the last
+    without: 64 = 7 8 + 8 and 84 = 10 8 + 4 block columns, whose trailing
+    updates go on to factor the next panel's first tile.  |L L^T - D| is at
+    most (m + 1) u |L| |L^T|, with u = 2^-53 in FP64 and 2^-24 for the products
+    of the reduced modes."""
+    D = spd(m, 3)
+    L, neg = E.cholesky_device(D, mode)
+    u = 2.0 ** (-53 if mode == E.CHOL_FP64 else -24)
+    v = np.random.default_rng(1).standard_normal((m, 4))
+    bound = (m + 1) * u * (np.abs(L) @ (np.abs(L.T) @ np.abs(v)))
+    assert neg == 0
+    assert np.all(np.abs(L @ (L.T @ v) - D @ v) <= bound + (m + 1) * 2.0 ** -53 * (np.abs(D) @ np.abs(v)))
+
+
 def test_super_panel_size_and_mixed_modes():
-    """4500 rows: 71 block columns, factored in super-panels of 8."""
+    """4500 rows: 71 block columns, super-panels of 8 in the reduced modes."""
     D = spd(4500, 7)
     L0 = np.linalg.cholesky(D)
     L, neg = E.cholesky_device(D)
