@@ -1115,6 +1115,29 @@ __global__ void __launch_bounds__(256, 2) k_trail(double *A, int ld, int k0, int
     else store_tile(A, ld, ib * TB, jb * TB, As, diag);
 }
 
+// A triangle of S x S blocks (tiles, or 2x2 tiles) over the eight XCDs, which
+// workgroups take round-robin (blockIdx % 8): XCD x takes the x-th eighth of
+// the blocks in the order 8x8 group by 8x8 group, a group row by row.  False
+// for the workgroups past the triangle.
+__device__ __forceinline__ bool group_index(int b, int S, int &IB, int &JB) {
+    const int n = S * (S + 1) / 2, per = (n + 7) / 8, lin = (b & 7) * per + (b >> 3);
+    if (lin >= n) return false;
+    int r, c;
+    tri_index(lin, r, c);  // r: the block row in row-by-row order, in the same group row
+    const int GI = r >> 3, h = min(8, S - 8 * GI), o = lin - 4 * GI * (8 * GI + 1);
+    if (o < 8 * h * GI) {
+        const int GJ = o / (8 * h), q = o - 8 * h * GJ;
+        IB = 8 * GI + (q >> 3);
+        JB = 8 * GJ + (q & 7);
+    } else {
+        tri_index(o - 8 * h * GI, r, c);
+        IB = 8 * GI + r;
+        JB = 8 * GI + c;
+    }
+    return true;
+}
+inline int group_grid(int S) { return (S * (S + 1) / 2 + 7) / 8 * 8; }
+
 // Three-slice BF16 trailing update with the panel tiles split once.  Split
 // on the fly (k_trail<2>), every workgroup converts every operand fragment it
 // multiplies, so each panel tile is split by all the workgroups of its tile
@@ -1257,18 +1280,13 @@ __device__ __forceinline__ void bf_body(const __bf16 *sp, int ra, int rbw, int n
         }
     }
 }
-// Workgroups go round-robin over the eight XCDs (b % 8); XCD x takes groups
-// x, x + 8, ... of 8x8 blocks, 64 consecutive workgroups of its own per
-// group, so a group's 16 row and 16 column panel tiles are read into one L2.
+// The blocks of an XCD follow each other in 8x8 groups (group_index), so a
+// group's 16 row and 16 column panel tiles are read into one L2.
 __global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __bf16 *sp, int nb, int j0, int nt,
                                                      double *Linv, int *neg) {
     __shared__ __attribute__((aligned(16))) __bf16 S[48 * 512];
-    const int S2 = (nt - j0 + 1) / 2, SG = (S2 + 7) / 8, l = blockIdx.x >> 3, G = (l >> 6) * 8 + (blockIdx.x & 7);
-    if (G >= SG * (SG + 1) / 2) return;
-    int GI, GJ;
-    tri_index(G, GI, GJ);
-    const int IB = 8 * GI + ((l >> 3) & 7), JB = 8 * GJ + (l & 7);
-    if (IB >= S2 || JB > IB) return;
+    int IB, JB;
+    if (!group_index(blockIdx.x, (nt - j0 + 1) / 2, IB, JB)) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wr = w >> 1, wc = w & 1;
     const int nrow = nt - j0, ra = 2 * IB, rbw = 2 * JB;  // tile rows relative to j0
     const int ib = j0 + ra + wr, jb = j0 + rbw + wc;
@@ -1319,164 +1337,143 @@ __global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __
 // FP64 / FP32 trailing update of a super-panel from panel tiles packed once.
 // k_pack64 copies each parked panel tile of the super-panel into the operand
 // order of v_mfma_f64_16x16x4f64 (v_mfma_f32_16x16x4f32 has the same lane
-// layout): unit (rb, kp) of a tile is 64 lanes x 16 bytes, lane l holding
-// row 16 rb + l % 16 at K = 8 kp + l / 16 and 8 kp + 4 + l / 16, the
-// operands of K steps 2 kp and 2 kp + 1.  The tile of row block i and panel
-// column t sits at pk[((i - j0) nb + t) TB TB].
-constexpr size_t kPackTile = (size_t)TB * TB;  // doubles
-__device__ __forceinline__ size_t pk_off(int rb, int kp, int lane) { return (size_t)((rb * 8 + kp) * 64 + lane) * 2; }
+// layout): unit (u, rb) of a tile is 64 lanes x 16 bytes, lane l holding
+// row 16 rb + l % 16 at K = Q u + 4 q + l / 16, q = 0, 1 in doubles (Q = 8)
+// or q = 0 .. 3 rounded to floats (Q = 16).  A row block's units follow each
+// other through the whole K of the super-panel: unit (u, rb) of the tile of
+// row block i and panel column t is the one numbered
+// 4 (((i - j0) nb + t) TB / Q + u) + rb.
+template <int MODE> struct PackOf { typedef dbl2 T; static constexpr int kUnits = 8; };
+template <> struct PackOf<1> { typedef flt4 T; static constexpr int kUnits = 4; };
 
 // one workgroup per (row block, panel column) tile; wavefront w writes the
-// units of row block w
-__global__ void __launch_bounds__(256) k_pack64(const double *A, int ld, int k0, int nb, int j0, double *pk) {
+// units of rows 16 w
+template <int MODE>
+__global__ void __launch_bounds__(256) k_pack64(const double *A, int ld, int k0, int nb, int j0, void *pk) {
+    typedef typename PackOf<MODE>::T T;
+    constexpr int U = PackOf<MODE>::kUnits, Q = 16 / U;
     const int i = j0 + blockIdx.x / nb, t = blockIdx.x % nb;
-    const double *src = A + (size_t)(k0 + t) * TB * ld + (size_t)i * TB;
-    double *dst = pk + (size_t)blockIdx.x * kPackTile;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r = 16 * w + (lane & 15), k4 = lane >> 4;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double *src = A + (size_t)((k0 + t) * TB + 16 * w + (lane & 15)) * ld + (size_t)i * TB + (lane >> 4);
+    T *dst = static_cast<T *>(pk) + ((size_t)blockIdx.x * U * 4 + w) * 64 + lane;
 #pragma unroll
-    for (int kp = 0; kp < 8; kp++) {
-        dbl2 v;
-        v.x = src[(size_t)r * ld + 8 * kp + k4];
-        v.y = src[(size_t)r * ld + 8 * kp + 4 + k4];
-        *reinterpret_cast<dbl2 *>(dst + pk_off(w, kp, lane)) = v;
+    for (int u = 0; u < U; u++) {
+        T v;
+#pragma unroll
+        for (int q = 0; q < Q; q++) v[q] = src[4 * (Q * u + q)];
+        dst[256 * u] = v;
     }
 }
 
-// k_trail_pk: a workgroup takes a 2x2 block of trailing tiles (128x128),
-// wavefront (wr, wc) the whole tile (ib0 + wr, jb0 + wc), as k_trail_bf
-// does.  A stage is 16 of a panel column's K: units (rb, kp) of the
-// block's two row and two column tiles, 32 KB in slots (op, tile, rb, kp),
-// copied straight from global memory into LDS.  Two stages per workgroup:
-// the copy of stage s + 1 is issued before the products of stage s, so it
-// has a whole stage to land; two workgroups per CU (2 x 64 KB of LDS).
+// k_trail_pk: a workgroup takes one trailing tile and each wavefront a 32x32
+// quarter of it, reading its operands (two row and two column units a step)
+// from global memory straight into registers, the next step's while the
+// matrix cores work on the current one's.  No LDS, no barrier, and a
+// quarter that lies above the diagonal costs nothing.  What bounds it is the
+// matrix cores: 64 to 66 TF in FP64, of 78 that a loop of nothing but
+// products reaches, and 97 to 100 of 157 in FP32, where reading and writing
+// the tile takes its share.  A CU reads 32 bytes of operands a cycle, half of
+// what its L1 gives.  The form before (128x128 blocks staged through LDS by
+// direct copies, two barriers per 16 of K) reached in FP64 60.0 / 54.0 / 48.2
+// TF at 320 / 156 / 80 trailing block rows, this one 64.1 / 65.3 / 65.0;
+// 64x64 per wavefront in this form reached 64.4 / 62.0 / 52.8 (as few as 3
+// such blocks per CU) and in FP32 66 against 97 TF.  Three workgroups share a
+// CU (the LDS of the first tile's factor); a fourth changed nothing.
+//
+// Workgroups go round-robin over the eight XCDs (b % 8).  Each XCD takes an
+// eighth of the triangle's tiles in the order of group_index, so the tiles in
+// flight on it share their 8 row and 8 column panels in its L2 and all eight
+// end together (whole groups dealt to XCDs in turn left up to 28% of the chip
+// idle at 120 block rows).
+//
 // Every accumulator takes the MFMAs of k_trail<MODE> in the same order (panel
 // column, then K step), so the update is the same bit for bit.
-__device__ __forceinline__ int pk_slot(int op, int tile, int rb, int kpl) { return ((op * 2 + tile) * 4 + rb) * 2 + kpl; }
-template <bool DIAG>
-__device__ __forceinline__ void pk_issue(const double *pk, int ra, int rbw, int nb, int nrow, int st, double *S, int w,
-                                         int lane) {
-    const int t = st >> 2, h = st & 3;
-    if (DIAG) {
-        const int tile = w >> 1, half = w & 1;
-        if (ra + tile >= nrow) return;
-        const double *src = pk + (size_t)((ra + tile) * nb + t) * kPackTile;
+template <typename T>
+__device__ __forceinline__ void pk_read(const T *A, const T *B, T (&a)[2], T (&b)[2]) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int rb = 2 * half + (j >> 1), kpl = j & 1;
-            __builtin_amdgcn_global_load_lds(src + pk_off(rb, 2 * h + kpl, lane),
-                                             (lds_void *)(S + (size_t)pk_slot(0, tile, rb, kpl) * 128), 16, 0, 0);
-        }
-    } else {
-        const int op = w >> 1, tile = w & 1, row = (op ? rbw : ra) + tile;
-        if (row >= nrow) return;
-        const double *src = pk + (size_t)(row * nb + t) * kPackTile;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int rb = j >> 1, kpl = j & 1;
-            __builtin_amdgcn_global_load_lds(src + pk_off(rb, 2 * h + kpl, lane),
-                                             (lds_void *)(S + (size_t)pk_slot(op, tile, rb, kpl) * 128), 16, 0, 0);
-        }
+    for (int q = 0; q < 2; q++) {
+        a[q] = A[64 * q];
+        b[q] = B[64 * q];
     }
 }
-template <int MODE, typename V>
-__device__ __forceinline__ V pk_mfma(double a, double b, V c) {
-    if constexpr (MODE == 0) return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_16x16x4f32((float)a, (float)b, c, 0, 0, 0);
+__device__ __forceinline__ dbl4 pk_mfma(double a, double b, dbl4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
-template <int MODE, bool DIAG, typename V>
-__device__ __forceinline__ void pk_body(const double *pk, int ra, int rbw, int nb, int nrow, double *S, int w, int lane,
-                                        bool active, V (&acc)[4][4]) {
-    constexpr int BOP = DIAG ? 0 : 1;
-    const int wr = w >> 1, wc = w & 1, ns = 4 * nb;
-    pk_issue<DIAG>(pk, ra, rbw, nb, nrow, 0, S, w, lane);
-    for (int st = 0; st < ns; st++) {
-        const double *B = S + (size_t)(st & 1) * 32 * 128;
-        if (st + 1 < ns) {
-            pk_issue<DIAG>(pk, ra, rbw, nb, nrow, st + 1, S + (size_t)((st + 1) & 1) * 32 * 128, w, lane);
-            // this wavefront's copies of stage st are done, those of st + 1
-            // may be in flight (vector memory counts retire in order)
-            if (DIAG) __builtin_amdgcn_s_waitcnt(0xF74);  // vmcnt(4)
-            else __builtin_amdgcn_s_waitcnt(0xF78);       // vmcnt(8)
-        } else {
-            __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
-        }
-        __builtin_amdgcn_s_barrier();
-        if (active) {
-            dbl2 a[2][4], b[2][4];
+__device__ __forceinline__ flt4 pk_mfma(float a, float b, flt4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+template <int Q, typename T, typename V>
+__device__ __forceinline__ void pk_products(const T (&a)[2], const T (&b)[2], V (&acc)[2][2]) {
+    // between the reads before and after it, so that these are in flight
+    // beside the products
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int kpl = 0; kpl < 2; kpl++)
+    for (int q = 0; q < Q; q++)
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    a[kpl][q] = *reinterpret_cast<const dbl2 *>(B + (size_t)pk_slot(0, wr, q, kpl) * 128 + lane * 2);
-                    b[kpl][q] = *reinterpret_cast<const dbl2 *>(B + (size_t)pk_slot(BOP, wc, q, kpl) * 128 + lane * 2);
-                }
+        for (int mi = 0; mi < 2; mi++)
 #pragma unroll
-            for (int kpl = 0; kpl < 2; kpl++) {
-#pragma unroll
-                for (int mi = 0; mi < 4; mi++)
-#pragma unroll
-                    for (int ni = 0; ni < 4; ni++) acc[mi][ni] = pk_mfma<MODE>(a[kpl][mi].x, b[kpl][ni].x, acc[mi][ni]);
-#pragma unroll
-                for (int mi = 0; mi < 4; mi++)
-#pragma unroll
-                    for (int ni = 0; ni < 4; ni++) acc[mi][ni] = pk_mfma<MODE>(a[kpl][mi].y, b[kpl][ni].y, acc[mi][ni]);
-            }
-        }
-        // every wavefront has read stage st before its slots take stage st + 2
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-        __builtin_amdgcn_s_barrier();
-    }
+            for (int ni = 0; ni < 2; ni++) acc[mi][ni] = pk_mfma(a[mi][q], b[ni][q], acc[mi][ni]);
+    __builtin_amdgcn_sched_barrier(0);
 }
 template <int MODE>
-__global__ void __launch_bounds__(256, 2) k_trail_pk(double *A, int ld, const double *pk, int nb, int j0, int nt,
+__global__ void __launch_bounds__(256, 3) k_trail_pk(double *A, int ld, const void *pk, int nb, int j0, int nt,
                                                      double *Linv, int *neg) {
-    __shared__ __attribute__((aligned(16))) double S[2 * 32 * 128];
-    const int S2 = (nt - j0 + 1) / 2, SG = (S2 + 7) / 8, l = blockIdx.x >> 3, G = (l >> 6) * 8 + (blockIdx.x & 7);
-    if (G >= SG * (SG + 1) / 2) return;
-    int GI, GJ;
-    tri_index(G, GI, GJ);
-    const int IB = 8 * GI + ((l >> 3) & 7), JB = 8 * GJ + (l & 7);
-    if (IB >= S2 || JB > IB) return;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wr = w >> 1, wc = w & 1;
-    const int nrow = nt - j0, ra = 2 * IB, rbw = 2 * JB;  // tile rows relative to j0
-    const int ib = j0 + ra + wr, jb = j0 + rbw + wc;
-    const bool active = ib < nt && jb <= ib;
+    typedef typename PackOf<MODE>::T T;
     typedef typename AccOf<MODE>::T V;
-    V acc[4][4];
+    __shared__ __attribute__((aligned(16))) double S[kDiagLds];
+    static_assert(kDiagLds >= TB * LDP, "the first tile");
+    constexpr int U = PackOf<MODE>::kUnits;
+    int IB, JB;
+    if (!group_index(blockIdx.x, nt - j0, IB, JB)) return;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wr = w >> 1, wc = w & 1;
+    const bool diag = IB == JB && wr == wc, active = IB > JB || wr >= wc;
+    const bool keep = blockIdx.x == 0;  // the first tile goes to LDS, for its factor
+    if (active) {
+        const T *a = static_cast<const T *>(pk) + ((size_t)IB * nb * U * 4 + 2 * wr) * 64 + lane;
+        const T *b = static_cast<const T *>(pk) + ((size_t)JB * nb * U * 4 + 2 * wc) * 64 + lane;
+        V acc[2][2];
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+        for (int mi = 0; mi < 2; mi++)
 #pragma unroll
-        for (int b = 0; b < 4; b++) acc[a][b] = V{};
-    if (IB == JB) pk_body<MODE, true>(pk, ra, rbw, nb, nrow, S, w, lane, active, acc);
-    else pk_body<MODE, false>(pk, ra, rbw, nb, nrow, S, w, lane, active, acc);
-    if (!active && blockIdx.x) return;
-    const int i16 = lane & 15, k4 = lane >> 4;
-    // C -= acc in place (row of register v: l/16 + 4v for the FP64 MFMA,
-    // 4(l/16) + v for the FP32 one), a row of 16x16 blocks at a time
-    const bool keep = blockIdx.x == 0 && w == 0;  // the first tile goes to LDS, for its factor
-    if (active)
+            for (int ni = 0; ni < 2; ni++) acc[mi][ni] = V{};
+        T a0[2], b0[2], a1[2], b1[2];
+        pk_read(a, b, a0, b0);
+        for (int u = U * nb; u > 0; u -= 2) {
+            pk_read(a + 256, b + 256, a1, b1);
+            pk_products<16 / U>(a0, b0, acc);
+            const int st = u > 2 ? 512 : 0;  // the last pass reads its own units again
+            a += st;
+            b += st;
+            pk_read(a, b, a0, b0);
+            pk_products<16 / U>(a1, b1, acc);
+        }
+        // C -= acc in place (row of register v: l/16 + 4v for the FP64 MFMA,
+        // 4(l/16) + v for the FP32 one), loads before stores
+        const int i16 = lane & 15, k4 = lane >> 4;
+        double *C = A + (size_t)((j0 + IB) * TB + 32 * wr) * ld + (j0 + JB) * TB + 32 * wc;
+        double *T0 = S + 32 * wr * LDP + 32 * wc;
+        double cv[2][2][4];
+        auto row = [&](int mi, int v) { return 16 * mi + (MODE == 0 ? k4 + 4 * v : 4 * k4 + v); };
 #pragma unroll
-    for (int mi = 0; mi < 4; mi++) {
-        double cv[4][4];
+        for (int mi = 0; mi < 2; mi++)
 #pragma unroll
-        for (int ni = 0; ni < 4; ni++)
+            for (int ni = 0; ni < 2; ni++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = 16 * mi + (MODE == 0 ? k4 + 4 * v : 4 * k4 + v), c = 16 * ni + i16;
-                cv[ni][v] = A[(size_t)(ib * TB + r) * ld + jb * TB + c];
-            }
+                for (int v = 0; v < 4; v++) cv[mi][ni][v] = C[(size_t)row(mi, v) * ld + 16 * ni + i16];
 #pragma unroll
-        for (int ni = 0; ni < 4; ni++)
+        for (int mi = 0; mi < 2; mi++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = 16 * mi + (MODE == 0 ? k4 + 4 * v : 4 * k4 + v), c = 16 * ni + i16;
-                if (ib == jb && c > r) continue;
-                const double x = cv[ni][v] + -1.0 * (double)acc[mi][ni][v];
-                if (keep) S[r * LDP + c] = x;
-                else A[(size_t)(ib * TB + r) * ld + jb * TB + c] = x;
-            }
+            for (int ni = 0; ni < 2; ni++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int r = row(mi, v), c = 16 * ni + i16;
+                    if (diag && c > r) continue;
+                    const double x = cv[mi][ni][v] + -1.0 * (double)acc[mi][ni][v];
+                    if (keep) T0[r * LDP + c] = x;
+                    else C[(size_t)r * ld + c] = x;
+                }
     }
-    static_assert(sizeof(S) >= kDiagLds * sizeof(double), "LDS of the factor");
     if (blockIdx.x == 0) {
         __syncthreads();
         diag_factor_inv(S, S, A, ld, j0 * TB, Linv + (size_t)j0 * TB * TB, neg);
@@ -1694,22 +1691,20 @@ void chol_column(const CholWork &c, int kb, int jcols, hipStream_t q) {
 template <int MODE>
 void chol_trail(const CholWork &c, int k0, int nb, hipStream_t q) {
     const int nt = c.mpad / TB, j0 = k0 + nb;
-    // the 128x128 blocks pay in FP64 from 192 trailing block rows, in FP32
-    // from about 96 (fewer blocks than workgroup slots below that); in BF16
-    // always (the direct form splits every operand fragment in every
-    // workgroup)
-    const int min_rows = c.pack_min_rows >= 0 ? c.pack_min_rows : MODE == 0 ? 192 : MODE == 1 ? 96 : 0;
-    if (c.sp && nb <= c.sp_nb && nt - j0 >= min_rows) {
-        // panel tiles packed (split) once, 128x128 blocks in 8x8 groups
-        const int S2 = (nt - j0 + 1) / 2, SG = (S2 + 7) / 8, grid = (SG * (SG + 1) / 2 + 7) / 8 * 512;
+    // packed wherever the buffer holds the panel: with its packing pass FP64
+    // takes 80 us against 87 at 40 trailing block rows, 39 against 45 at 20
+    // (FP32 56 and 29), and in BF16 the direct form splits every operand
+    // fragment in every workgroup
+    if (c.sp && nb <= c.sp_nb && nt - j0 >= c.pack_min_rows) {
+        // panel tiles packed (split) once, tiles in 8x8 groups over the XCDs
+        const int R = nt - j0;
         if constexpr (MODE == 2) {
             __bf16 *sp = static_cast<__bf16 *>(c.sp);
-            k_split3<<<(nt - j0) * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, sp);
-            k_trail_bf<<<grid, 256, 0, q>>>(c.A, c.ld, sp, nb, j0, nt, c.Linv, c.neg);
+            k_split3<<<R * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, sp);
+            k_trail_bf<<<group_grid((R + 1) / 2), 256, 0, q>>>(c.A, c.ld, sp, nb, j0, nt, c.Linv, c.neg);
         } else {
-            double *pk = static_cast<double *>(c.sp);
-            k_pack64<<<(nt - j0) * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, pk);
-            k_trail_pk<MODE><<<grid, 256, 0, q>>>(c.A, c.ld, pk, nb, j0, nt, c.Linv, c.neg);
+            k_pack64<MODE><<<R * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, c.sp);
+            k_trail_pk<MODE><<<group_grid(R), 256, 0, q>>>(c.A, c.ld, c.sp, nb, j0, nt, c.Linv, c.neg);
         }
         return;
     }
@@ -1720,7 +1715,7 @@ void chol_trail(const CholWork &c, int k0, int nb, hipStream_t q) {
 
 size_t split_bytes(int ld, int nb) {
     return std::max((size_t)(ld / TB) * nb * 3 * kSplitTile * sizeof(__bf16),
-                    (size_t)(ld / TB) * nb * kPackTile * sizeof(double));
+                    (size_t)(ld / TB) * nb * TB * TB * sizeof(double));
 }
 
 // Super-panels from 84 block columns in FP64 (us a step without / with them,

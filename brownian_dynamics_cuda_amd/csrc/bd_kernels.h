@@ -93,8 +93,7 @@ struct CholWork {
     // parked tiles directly
     void *sp;
     int sp_nb;
-    // smallest trailing matrix (block rows) that takes the packed form; -1:
-    // the mode's default
+    // smallest trailing matrix (block rows) that takes the packed form
     int pack_min_rows;
 };
 // bytes of the packed / split panel buffer for leading dimension ld and

@@ -56,26 +56,42 @@ int split_tiles_of_current_device() {
     return ncu * 19 / 10;
 }
 
+CholWork work_of(int m, int mode) {
+    CholWork c{};
+    c.m = m;
+    c.mpad = (m + 63) / 64 * 64;
+    c.ld = c.mpad;
+    c.mode = mode;
+    return c;
+}
+
 // Work of one factor in the workspace at ws (doubles): the padded matrix
 // (mpad x mpad), the inverses of the diagonal factors (one 64x64 tile per
-// block column) and the negative-pivot counter.
+// block column) and the negative-pivot counter; behind these, where packed,
+// the packed panel tiles of the super-panels (pack_bytes, 0 for a matrix that
+// has none).
 size_t workspace_doubles(int m) {
     const size_t mpad = ((size_t)m + 63) / 64 * 64;
     return mpad * mpad + (mpad / 64) * 64 * 64 + 32;
 }
 
+size_t pack_bytes(int m, int mode) {
+    const CholWork c = work_of(m, mode);
+    const int nb = chol_panel_tiles(c);
+    return nb ? split_bytes(c.ld, nb) : 0;
+}
+
 int run_factor(int m, const double *D, int ldd, double *L, int ldl, int mode, int *neg, hipStream_t q,
-               double *ws) {
-    CholWork c{};
-    c.m = m;
-    c.mpad = (m + 63) / 64 * 64;
-    c.ld = c.mpad;
+               double *ws, bool packed) {
+    CholWork c = work_of(m, mode);
     c.A = ws;
     c.Linv = ws + (size_t)c.mpad * c.mpad;
     c.neg = reinterpret_cast<int *>(c.Linv + (size_t)(c.mpad / 64) * 64 * 64);
-    c.mode = mode;
+    if (packed) {
+        c.sp = ws + workspace_doubles(m);
+        c.sp_nb = chol_panel_tiles(c);
+    }
     c.split_tiles = split_tiles_of_current_device();
-    c.panel_tiles = 0;
     launch_pack(D, ldd, c, q);
     launch_diag(c, 0, true, q);
     launch_cholesky(c, q);
@@ -128,8 +144,14 @@ int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, i
     if (r) return r;
     hipStream_t q = static_cast<hipStream_t>(stream);
     double *ws = nullptr;
-    POTRF_CHK(hipMalloc((void **)&ws, workspace_doubles(m) * sizeof(double)));
-    r = run_factor(m, D, ldd, L, ldl, mode, neg, q, ws);
+    // without room for the packed panel tiles the factor does without them
+    const size_t bytes = workspace_doubles(m) * sizeof(double), pack = pack_bytes(m, mode);
+    const bool packed = pack && hipMalloc((void **)&ws, bytes + pack) == hipSuccess;
+    if (!packed) {
+        if (pack) (void)hipGetLastError();
+        POTRF_CHK(hipMalloc((void **)&ws, bytes));
+    }
+    r = run_factor(m, D, ldd, L, ldl, mode, neg, q, ws, packed);
     hipError_t e = hipFree(ws);
     if (r) return r;
     if (e != hipSuccess) return fail(BD_E_HIP, "hipFree: %s", hipGetErrorString(e));
@@ -145,7 +167,7 @@ int bd_cholesky_noalloc(int m, const double *D, int ldd, double *L, int ldl, int
     double *ws = nullptr;
     r = scratch_of_current_device(&ws);
     if (r) return r;
-    return run_factor(m, D, ldd, L, ldl, mode, neg, static_cast<hipStream_t>(stream), ws);
+    return run_factor(m, D, ldd, L, ldl, mode, neg, static_cast<hipStream_t>(stream), ws, false);
 }
 
 }  // extern "C"
