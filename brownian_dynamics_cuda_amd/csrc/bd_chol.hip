@@ -21,13 +21,17 @@
 // and the trailing matrix then receives the whole panel in one launch
 // (k_trail: each tile accumulates K = 64 NB in registers before its one
 // read-modify-write), so the trailing matrix streams through HBM once per
-// NB block columns rather than once per block column.  On large trailing
-// matrices the panel tiles are first copied once into the operand order of
-// the matrix cores (k_pack64; k_split3 splits them into BF16 slices) and
-// the update takes 128x128 blocks fed by global-to-LDS copies (k_trail_pk,
-// k_trail_bf).  In the FP32 and BF16 modes only that trailing update takes
+// NB block columns rather than once per block column.  The panel tiles lie
+// once more in the operand order of the matrix cores for it (k_trail_pk; in
+// BF16 split into slices, k_trail_bf).  Panels of eight in FP64 and FP32
+// (chol_panels) factor only their diagonal block column by column, beside
+// tiles of the trailing update before it (k_block_step), and solve the rows
+// below in one launch (k_panel_rows).  In the FP32 and BF16 modes only the
+// trailing update takes
 // the reduced precision; the panel's own columns stay FP64.
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "bd_dev.h"
 #include "bd_kernels.h"
@@ -910,6 +914,20 @@ __device__ __forceinline__ void store_tile_half(double *dst, int ld, const doubl
     }
 }
 
+// A panel tile from LDS, negated, in the operand order of k_panel_rows: 16
+// bytes of lane l of unit u = 2 b + h of wavefront w are row 16 w +
+// row_pi(l % 16), K = 16 b + 4 (l / 16) + 2 h and the next
+__device__ __forceinline__ int row_pi(int i16) { return 4 * (i16 & 3) + (i16 >> 2); }
+__device__ __forceinline__ void store_operand(double *dst, const double *S) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double *src = S + (16 * w + row_pi(lane & 15)) * LDP + 4 * (lane >> 4);
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const int c = 16 * (u >> 1) + 2 * (u & 1);
+        *reinterpret_cast<dbl2 *>(dst + (w * 8 + u) * 128 + 2 * lane) = dbl2{-src[c], -src[c + 1]};
+    }
+}
+
 // Trailing tiles of block column kb restricted to the first jcols trailing
 // block columns, row-major: rows ii = 0..M-1, columns jj <= min(ii, jcols-1)
 // (jcols = M: the whole trailing triangle, in tri_index order).
@@ -940,19 +958,14 @@ __device__ __forceinline__ void trap_index(int idx, int jcols, int &i, int &j) {
 // The panel products are repeated by the workgroups of a block row, in
 // exchange for one launch (and one kernel boundary) per block column.
 // jcols < M restricts the update to the columns of a super-panel.
+constexpr int kStepLds = 2 * TB * LDP;
 template <int MODE>
-__global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int jcols, double *Linv, int *neg) {
-    // two tiles of LDS (two workgroups per CU): first inv(L_kb,kb) and the
-    // row's panel block, then the column's panel block in place of the row's,
-    // then the two panel tiles; the target tile stays in registers
-    __shared__ double S[2 * TB * LDP];
+__device__ __forceinline__ void step_tile(double *S, double *A, int ld, int kb, int jcols, int lb, double *Linv, int *neg,
+                                          double *Lp) {
+    // two tiles of LDS: first inv(L_kb,kb) and the row's panel block, then the
+    // column's panel block in place of the row's, then the two panel tiles;
+    // the target tile stays in registers
     double *S0 = S, *S1 = S + TB * LDP;
-    // workgroups go round-robin over the eight XCDs (b % 8); XCD x takes a
-    // contiguous run of tiles, so the tiles of a block row, which read the
-    // same panel tile, share an L2 (workgroup 0, the diagonal tile, stays 0)
-    int lb = blockIdx.x;
-    const int G8 = gridDim.x / 8;
-    if (lb < 8 * G8) lb = (lb % 8) * G8 + lb / 8;
     int ii, jj;
     trap_index(lb, jcols, ii, jj);
     const int ib = kb + 1 + ii, jb = kb + 1 + jj;
@@ -979,6 +992,7 @@ __global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int 
         __syncthreads();
         diag_tile_update<MODE>(S1, S0);
         if (jj == 0) store_tile_half(A + (size_t)kb * TB * ld + ib * TB, ld, S1);
+        if (Lp && jcols == 1) store_operand(Lp, S1);
         __syncthreads();
         if (ii == 0)
             diag_factor_inv(S, S0, A, ld, ib * TB, Linv + (size_t)ib * TB * TB, neg);
@@ -997,8 +1011,25 @@ __global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int 
         panel_to_lds(S1, pj);
     }
     __syncthreads();
-    if (jj == 0) store_tile(A, ld, kb * TB, ib * TB, S0, false);
+    if (jj == 0) {
+        store_tile(A, ld, kb * TB, ib * TB, S0, false);
+        if (Lp) {
+            store_operand(Lp + ii * TB * TB, S0);
+            if (ii == 1) store_operand(Lp, S1);  // L_kb+1,kb, which workgroup 0 has no time for
+        }
+    }
     tile_update<MODE>(S0, S1, A + (size_t)ib * TB * ld + jb * TB, ld);
+}
+template <int MODE>
+__global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int jcols, double *Linv, int *neg) {
+    __shared__ double S[kStepLds];  // two workgroups per CU
+    // workgroups go round-robin over the eight XCDs (b % 8); XCD x takes a
+    // contiguous run of tiles, so the tiles of a block row, which read the
+    // same panel tile, share an L2 (workgroup 0, the diagonal tile, stays 0)
+    int lb = blockIdx.x;
+    const int G8 = gridDim.x / 8;
+    if (lb < 8 * G8) lb = (lb % 8) * G8 + lb / 8;
+    step_tile<MODE>(S, A, ld, kb, jcols, lb, Linv, neg, nullptr);
 }
 
 // The same block column in two launches, for wide trailing matrices (many
@@ -1115,29 +1146,34 @@ __global__ void __launch_bounds__(256, 2) k_trail(double *A, int ld, int k0, int
     else store_tile(A, ld, ib * TB, jb * TB, As, diag);
 }
 
-// A triangle of S x S blocks (tiles, or 2x2 tiles) over the eight XCDs, which
-// workgroups take round-robin (blockIdx % 8): XCD x takes the x-th eighth of
-// the blocks in the order 8x8 group by 8x8 group, a group row by row.  False
-// for the workgroups past the triangle.
-__device__ __forceinline__ bool group_index(int b, int S, int &IB, int &JB) {
-    const int n = S * (S + 1) / 2, per = (n + 7) / 8, lin = (b & 7) * per + (b >> 3);
-    if (lin >= n) return false;
+constexpr int kPanel = 8;  // super-panel width of chol_panels
+
+// Block lin of a triangle of S x S blocks (tiles, or 2x2 tiles) in the order
+// GxG group by GxG group, a group row by row.
+template <int G>
+__device__ __forceinline__ void group_index(int lin, int S, int &IB, int &JB) {
     int r, c;
     tri_index(lin, r, c);  // r: the block row in row-by-row order, in the same group row
-    const int GI = r >> 3, h = min(8, S - 8 * GI), o = lin - 4 * GI * (8 * GI + 1);
-    if (o < 8 * h * GI) {
-        const int GJ = o / (8 * h), q = o - 8 * h * GJ;
-        IB = 8 * GI + (q >> 3);
-        JB = 8 * GJ + (q & 7);
+    const int GI = r / G, h = min(G, S - G * GI), o = lin - G * GI * (G * GI + 1) / 2;
+    if (o < G * h * GI) {
+        const int GJ = o / (G * h), q = o - G * h * GJ;
+        IB = G * GI + q / G;
+        JB = G * GJ + q % G;
     } else {
-        tri_index(o - 8 * h * GI, r, c);
-        IB = 8 * GI + r;
-        JB = 8 * GI + c;
+        tri_index(o - G * h * GI, r, c);
+        IB = G * GI + r;
+        JB = G * GI + c;
     }
-    return true;
+    IB = __builtin_amdgcn_readfirstlane(IB);
+    JB = __builtin_amdgcn_readfirstlane(JB);
 }
-inline int group_grid(int S) { return (S * (S + 1) / 2 + 7) / 8 * 8; }
-
+// Blocks lin0 .. lin0 + n - 1 over the eight XCDs, which workgroups take
+// round-robin (b % 8): XCD x takes the x-th eighth of them.  -1 past the end.
+__device__ __forceinline__ int xcd_index(int b, int lin0, int n) {
+    const int per = (n + 7) / 8, l = (b & 7) * per + (b >> 3);
+    return l < n ? lin0 + l : -1;
+}
+inline int xcd_grid(int n) { return (n + 7) / 8 * 8; }
 // Three-slice BF16 trailing update with the panel tiles split once.  Split
 // on the fly (k_trail<2>), every workgroup converts every operand fragment it
 // multiplies, so each panel tile is split by all the workgroups of its tile
@@ -1282,11 +1318,10 @@ __device__ __forceinline__ void bf_body(const __bf16 *sp, int ra, int rbw, int n
 }
 // The blocks of an XCD follow each other in 8x8 groups (group_index), so a
 // group's 16 row and 16 column panel tiles are read into one L2.
-__global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __bf16 *sp, int nb, int j0, int nt,
-                                                     double *Linv, int *neg) {
-    __shared__ __attribute__((aligned(16))) __bf16 S[48 * 512];
-    int IB, JB;
-    if (!group_index(blockIdx.x, (nt - j0 + 1) / 2, IB, JB)) return;
+constexpr int kBfLds = 48 * 512;  // of BF16
+__device__ __forceinline__ void trail_bf_block(__bf16 *S, double *A, int ld, const __bf16 *sp, int nb, int j0, int nt, int IB,
+                                               int JB, double *Linv, int *neg) {
+    const bool first = IB == 0;  // the block of the next panel's first tile
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, wr = w >> 1, wc = w & 1;
     const int nrow = nt - j0, ra = 2 * IB, rbw = 2 * JB;  // tile rows relative to j0
     const int ib = j0 + ra + wr, jb = j0 + rbw + wc;
@@ -1298,14 +1333,13 @@ __global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __
         for (int b = 0; b < 4; b++) acc[a][b] = flt4{0.f, 0.f, 0.f, 0.f};
     if (IB == JB) bf_body<true>(sp, ra, rbw, nb, nrow, S, w, lane, active, acc);
     else bf_body<false>(sp, ra, rbw, nb, nrow, S, w, lane, active, acc);
-    if (!active && blockIdx.x) return;
+    if (!active && !first) return;
     const int i16 = lane & 15, k4 = lane >> 4;
     // C -= acc in place, a row of 16x16 blocks at a time: loads, then stores
     // (a diagonal tile keeps its upper triangle; the first tile goes to LDS,
     // for its factor)
     double *T = reinterpret_cast<double *>(S);
-    const bool keep = blockIdx.x == 0 && w == 0;
-    static_assert(sizeof(S) >= kDiagLds * sizeof(double) && sizeof(S) >= TB * LDP * sizeof(double), "LDS of the factor");
+    const bool keep = first && w == 0;
     if (active)
 #pragma unroll
     for (int mi = 0; mi < 4; mi++) {
@@ -1328,10 +1362,20 @@ __global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __
                 else A[(size_t)(ib * TB + r) * ld + jb * TB + c] = x;
             }
     }
-    if (blockIdx.x == 0) {
+    if (first) {
         __syncthreads();
         diag_factor_inv(T, T, A, ld, j0 * TB, Linv + (size_t)j0 * TB * TB, neg);
     }
+}
+__global__ void __launch_bounds__(256, 3) k_trail_bf(double *A, int ld, const __bf16 *sp, int nb, int j0, int nt, int n,
+                                                     double *Linv, int *neg) {
+    __shared__ __attribute__((aligned(16))) __bf16 S[kBfLds];
+    static_assert(sizeof(S) >= kDiagLds * sizeof(double) && sizeof(S) >= TB * LDP * sizeof(double), "LDS of the factor");
+    const int lin = xcd_index(blockIdx.x, 0, n);
+    if (lin < 0) return;
+    int IB, JB;
+    group_index<4>(lin, (nt - j0 + 1) / 2, IB, JB);
+    trail_bf_block(S, A, ld, sp, nb, j0, nt, IB, JB, Linv, neg);
 }
 
 // FP64 / FP32 trailing update of a super-panel from panel tiles packed once.
@@ -1370,15 +1414,17 @@ __global__ void __launch_bounds__(256) k_pack64(const double *A, int ld, int k0,
 // from global memory straight into registers, the next step's while the
 // matrix cores work on the current one's.  No LDS, no barrier, and a
 // quarter that lies above the diagonal costs nothing.  What bounds it is the
-// matrix cores: 64 to 66 TF in FP64, of 78 that a loop of nothing but
-// products reaches, and 97 to 100 of 157 in FP32, where reading and writing
-// the tile takes its share.  A CU reads 32 bytes of operands a cycle, half of
-// what its L1 gives.  The form before (128x128 blocks staged through LDS by
-// direct copies, two barriers per 16 of K) reached in FP64 60.0 / 54.0 / 48.2
-// TF at 320 / 156 / 80 trailing block rows, this one 64.1 / 65.3 / 65.0;
-// 64x64 per wavefront in this form reached 64.4 / 62.0 / 52.8 (as few as 3
-// such blocks per CU) and in FP32 66 against 97 TF.  Three workgroups share a
-// CU (the LDS of the first tile's factor); a fourth changed nothing.
+// matrix cores: 67 TF in FP64, of 78 that a loop of nothing but products
+// reaches, and 112 of 157 in FP32, where reading and writing the tile takes
+// its share.  A CU reads 32 bytes of operands a cycle, half of what its L1
+// gives.  The form before (128x128 blocks staged through LDS by direct copies,
+// two barriers per 16 of K) reached in FP64 60.0 / 54.0 / 48.2 TF at 320 / 156
+// / 80 trailing block rows, this one 64 / 66.9 / 67.5; 64x64 per wavefront in
+// this form reached 64.4 / 62.0 / 52.8 (as few as 3 such blocks per CU) and in
+// FP32 66 against 97 TF.  With the operand addresses in vector registers it
+// was 65 and 100 TF.  Three workgroups share a CU (the LDS of the first tile's
+// factor); a fourth changed nothing, nor did the tile's own loads before the
+// loop (FP32 slower by a fifth: the registers).
 //
 // Workgroups go round-robin over the eight XCDs (b % 8).  Each XCD takes an
 // eighth of the triangle's tiles in the order of group_index, so the tiles in
@@ -1388,12 +1434,19 @@ __global__ void __launch_bounds__(256) k_pack64(const double *A, int ld, int k0,
 //
 // Every accumulator takes the MFMAs of k_trail<MODE> in the same order (panel
 // column, then K step), so the update is the same bit for bit.
+// one step's units from the uniform addresses A and B, which the empty asm
+// keeps in scalar registers: an FP64 matrix product and a vector ALU
+// instruction do not overlap, so the loop holds no address arithmetic in
+// vector registers
 template <typename T>
-__device__ __forceinline__ void pk_read(const T *A, const T *B, T (&a)[2], T (&b)[2]) {
+__device__ __forceinline__ void pk_read(const T *A, const T *B, unsigned lane, T (&a)[2], T (&b)[2]) {
+    typedef const T __attribute__((address_space(1))) *Global;
+    Global pa = (Global)A, pb = (Global)B;
+    asm volatile("" : "+s"(pa), "+s"(pb));
 #pragma unroll
     for (int q = 0; q < 2; q++) {
-        a[q] = A[64 * q];
-        b[q] = B[64 * q];
+        a[q] = pa[lane + 64u * q];
+        b[q] = pb[lane + 64u * q];
     }
 }
 __device__ __forceinline__ dbl4 pk_mfma(double a, double b, dbl4 c) {
@@ -1415,38 +1468,38 @@ __device__ __forceinline__ void pk_products(const T (&a)[2], const T (&b)[2], V 
             for (int ni = 0; ni < 2; ni++) acc[mi][ni] = pk_mfma(a[mi][q], b[ni][q], acc[mi][ni]);
     __builtin_amdgcn_sched_barrier(0);
 }
-template <int MODE>
-__global__ void __launch_bounds__(256, 3) k_trail_pk(double *A, int ld, const void *pk, int nb, int j0, int nt,
-                                                     double *Linv, int *neg) {
+// D: steps in the operand ring (divides 4 nb)
+template <int MODE, int D>
+__device__ __forceinline__ void trail_pk_tile(double *S, double *A, int ld, const void *pk, int nb, int j0, int IB, int JB,
+                                              double *Linv, int *neg) {
     typedef typename PackOf<MODE>::T T;
     typedef typename AccOf<MODE>::T V;
-    __shared__ __attribute__((aligned(16))) double S[kDiagLds];
-    static_assert(kDiagLds >= TB * LDP, "the first tile");
     constexpr int U = PackOf<MODE>::kUnits;
-    int IB, JB;
-    if (!group_index(blockIdx.x, nt - j0, IB, JB)) return;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = w >> 1, wc = w & 1;
     const bool diag = IB == JB && wr == wc, active = IB > JB || wr >= wc;
-    const bool keep = blockIdx.x == 0;  // the first tile goes to LDS, for its factor
+    const bool first = IB == 0;  // the first tile goes to LDS, for its factor
     if (active) {
-        const T *a = static_cast<const T *>(pk) + ((size_t)IB * nb * U * 4 + 2 * wr) * 64 + lane;
-        const T *b = static_cast<const T *>(pk) + ((size_t)JB * nb * U * 4 + 2 * wc) * 64 + lane;
+        const T *a = static_cast<const T *>(pk) + ((size_t)IB * nb * U * 4 + 2 * wr) * 64;
+        const T *b = static_cast<const T *>(pk) + ((size_t)JB * nb * U * 4 + 2 * wc) * 64;
         V acc[2][2];
 #pragma unroll
         for (int mi = 0; mi < 2; mi++)
 #pragma unroll
             for (int ni = 0; ni < 2; ni++) acc[mi][ni] = V{};
-        T a0[2], b0[2], a1[2], b1[2];
-        pk_read(a, b, a0, b0);
-        for (int u = U * nb; u > 0; u -= 2) {
-            pk_read(a + 256, b + 256, a1, b1);
-            pk_products<16 / U>(a0, b0, acc);
-            const int st = u > 2 ? 512 : 0;  // the last pass reads its own units again
+        T ra[D][2], rb[D][2];
+#pragma unroll
+        for (int d = 0; d < D - 1; d++) pk_read(a + 256 * d, b + 256 * d, lane, ra[d], rb[d]);
+        for (int u = U * nb; u > 0; u -= D) {
+            pk_read(a + 256 * (D - 1), b + 256 * (D - 1), lane, ra[D - 1], rb[D - 1]);
+            const int st = u > D ? 256 * D : 0;  // the last pass reads its own units again
             a += st;
             b += st;
-            pk_read(a, b, a0, b0);
-            pk_products<16 / U>(a1, b1, acc);
+#pragma unroll
+            for (int d = 0; d < D; d++) {
+                pk_products<16 / U>(ra[d], rb[d], acc);
+                if (d + 1 < D) pk_read(a + 256 * d, b + 256 * d, lane, ra[d], rb[d]);
+            }
         }
         // C -= acc in place (row of register v: l/16 + 4v for the FP64 MFMA,
         // 4(l/16) + v for the FP32 one), loads before stores
@@ -1470,14 +1523,207 @@ __global__ void __launch_bounds__(256, 3) k_trail_pk(double *A, int ld, const vo
                     const int r = row(mi, v), c = 16 * ni + i16;
                     if (diag && c > r) continue;
                     const double x = cv[mi][ni][v] + -1.0 * (double)acc[mi][ni][v];
-                    if (keep) T0[r * LDP + c] = x;
+                    if (first) T0[r * LDP + c] = x;
                     else C[(size_t)r * ld + c] = x;
                 }
     }
-    if (blockIdx.x == 0) {
+    if (first) {
         __syncthreads();
         diag_factor_inv(S, S, A, ld, j0 * TB, Linv + (size_t)j0 * TB * TB, neg);
     }
+}
+template <int MODE>
+__global__ void __launch_bounds__(256, 3) k_trail_pk(double *A, int ld, const void *pk, int nb, int j0, int nt, int lin0,
+                                                     int n, double *Linv, int *neg) {
+    __shared__ __attribute__((aligned(16))) double S[kDiagLds];
+    static_assert(kDiagLds >= TB * LDP, "the first tile");
+    const int lin = xcd_index(blockIdx.x, lin0, n);
+    if (lin < 0) return;
+    int IB, JB;
+    group_index<kPanel>(lin, nt - j0, IB, JB);
+    trail_pk_tile<MODE, 2>(S, A, ld, pk, nb, j0, IB, JB, Linv, neg);
+}
+
+// One block column inside the diagonal block of a super-panel (step_tile, the
+// jcols (jcols + 1) / 2 workgroups before the others) beside n tiles of the
+// trailing update that is under way.  The column's launch is a chain of
+// latencies (13.0 us, of which 6.2 the next diagonal tile), at most 28
+// workgroups of it, so the other CUs take a tile of K = 512 each: 21.5 us with
+// 228 of them, where a launch of their own would cost 14.5 us more than the
+// chain alone.  jcols = 0: tiles only, the first of them the next panel's
+// first, which workgroup 0 goes on to factor.  The FP64 vector arithmetic of a
+// diagonal tile stands still beside another workgroup's matrix products, so a
+// workgroup asks for more than half of the LDS and has its CU to itself.
+constexpr int kOwnCu = 10368;  // doubles, more than half of a CU's LDS
+template <int MODE>
+__global__ void __launch_bounds__(256, 1) k_block_step(double *A, int ld, int kb, int jcols, const void *pk, int nb, int j0,
+                                                       int nt, int lin0, int n, double *Linv, int *neg, double *Lp) {
+    __shared__ __attribute__((aligned(16))) double S[kOwnCu];
+    static_assert(kOwnCu >= kStepLds && kOwnCu >= kDiagLds, "LDS");
+    const int G = jcols * (jcols + 1) / 2;
+    if ((int)blockIdx.x < G) {
+        step_tile<0>(S, A, ld, kb, jcols, blockIdx.x, Linv, neg, Lp);
+        return;
+    }
+    const int lin = xcd_index(blockIdx.x - G, lin0, n);
+    if (lin < 0) return;
+    int IB, JB;
+    group_index<kPanel>(lin, nt - j0, IB, JB);
+    trail_pk_tile<MODE, 4>(S, A, ld, pk, nb, j0, IB, JB, Linv, neg);
+}
+
+// The rows below the diagonal block of a super-panel of kPanel columns, once
+// the block is factored: X_k = (B_k - sum_{j<k} X_j L_kj^T) inv(L_kk)^T, 16
+// rows per workgroup and 16 of a column's 64 rows of L per wavefront, the
+// rows' eight column blocks in the accumulators.  The tiles go to their parked
+// places and, where the trailing update takes them packed (pk), there too.
+// Each wavefront multiplies L (as left operands, negated and in operand order
+// from k_block_step) with the transposed rows: a product's result layout is
+// then the next one's right operand, and the two exchanges per column, of the
+// updated and of the solved block, are two LDS writes and eight reads of a
+// wavefront, run between the updates that do not need them.  27 us up to 256
+// workgroups (64 block rows; 16 of them the products at the matrix cores'
+// rate), 50 up to 512, where column by column beside the block's own steps the
+// rows took 3 to 11 us per column, with the trailing update's tiles left
+// outside.  Operands in other layouts, with a transposition through LDS on
+// either side of each column: 31 and 56 us.
+constexpr int kPanelTiles = kPanel * (kPanel + 1) / 2;
+// Order of the products of k_panel_rows: the solve of column 0, then for each
+// column k its updates of columns k + 1, k + 2, k + 3, the solve of column
+// k + 1, and the rest of the updates.
+struct PanelTile { int k, t; };  // inv(L_kk) where t == k, else L_tk
+constexpr PanelTile panel_tile(int e) {
+    if (e == 0) return {0, 0};
+    int n = 1;
+    for (int k = 0; k + 1 < kPanel; k++) {
+        const int before = kPanel - 1 - k < 3 ? kPanel - 1 - k : 3;  // updates before the solve
+        const int count = kPanel - k;
+        if (e < n + count) {
+            const int j = e - n;
+            if (j < before) return {k, k + 1 + j};
+            if (j == before) return {k + 1, k + 1};
+            return {k, k + j};
+        }
+        n += count;
+    }
+    return {-1, -2};
+}
+template <typename F, int... I>
+__device__ __forceinline__ void static_steps(F f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+// Operands of the 16 matrix products of a 64x64 tile, by wavefront w its rows
+// 16 w ..: row 16 w + pi(l % 16), K = 16 b + 4 (l / 16) + s, s = 0 .. 3, in
+// o[2 b + s / 2]; off: this lane's first element, step: between its pairs
+template <int S1, int S2>
+__device__ __forceinline__ void read_operand(const double *base, unsigned off, dbl2 (&o)[8]) {
+    typedef const double __attribute__((address_space(1))) *Global;
+    typedef const dbl2 __attribute__((address_space(1))) *Global2;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        Global p = (Global)base + 2 * S2 * h;
+        asm volatile("" : "+s"(p));  // in scalar registers, as in pk_read
+#pragma unroll
+        for (int u = 0; u < 4; u++) o[4 * h + u] = *(Global2)(p + off + S1 * (u & 1) + S2 * (u >> 1));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int MODE>
+__global__ void __launch_bounds__(256, 2) k_panel_rows(double *A, int ld, int k0, const double *Linv, const double *Lp,
+                                                       void *pk) {
+    __shared__ __attribute__((aligned(16))) dbl2 Bs[512], Xs[512];  // [2 b + h][lane]
+    const int ri = blockIdx.x / 4, rb = blockIdx.x & 3, i = k0 + kPanel + ri;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+    // column blocks, transposed: lane l holds row l % 16, columns
+    // 64 t + 16 w + 4 (l / 16) + v, in the MFMA's result layout with its rows
+    // taken by row_pi, which is also the layout of a product's right operand
+    dbl4 acc[kPanel];
+    dbl2 op[3][8], x[8], y[8];
+    const unsigned inv_off = (16 * w + row_pi(i16)) * TB + 4 * k4, tile_off = w * 1024 + 2 * lane;
+    auto fetch = [&](auto E) {
+        constexpr PanelTile q = panel_tile(E);
+        if constexpr (q.t == q.k) read_operand<2, 16>(Linv + (size_t)(k0 + q.k) * TB * TB, inv_off, op[E % 3]);
+        else read_operand<128, 256>(Lp + (q.k * kPanel + q.t) * TB * TB, tile_off, op[E % 3]);
+    };
+    auto products = [&](const dbl2 (&a)[8], const dbl2 (&b)[8], dbl4 c) {
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][q], b[u][q], c, 0, 0, 0);
+        return c;
+    };
+    auto put = [&](dbl2 *S, const dbl4 &v) {
+        S[128 * w + lane] = dbl2{v[0], v[1]};
+        S[128 * w + 64 + lane] = dbl2{v[2], v[3]};
+    };
+    auto get = [&](const dbl2 *S, dbl2 (&v)[8]) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = S[64 * u + lane];
+    };
+    double *row = A + (size_t)(i * TB + 16 * rb + i16) * ld + k0 * TB + 16 * w + 4 * k4;
+    double *park = A + (size_t)(k0 * TB + 16 * rb + i16) * ld + i * TB + 16 * w + 4 * k4;
+    // column t's block of this wavefront, solved: to the others and to memory
+    auto store = [&](int t, const dbl4 &v) {
+        put(Xs, v);
+        dbl2 *d = reinterpret_cast<dbl2 *>(park + (size_t)t * TB * ld);
+        d[0] = dbl2{v[0], v[1]};
+        d[1] = dbl2{v[2], v[3]};
+    };
+    // the packed (split) form of column t, from all four blocks
+    auto pack = [&](int t) {
+        if (!pk) return;
+        const double *X = reinterpret_cast<const double *>(Xs);
+        // column c of row i16
+        auto at = [&](int c) { return X[((c >> 4) * 128 + ((c >> 1) & 1) * 64 + i16 + 16 * ((c >> 2) & 3)) * 2 + (c & 1)]; };
+        typedef typename PackOf<MODE>::T T;
+        constexpr int U = PackOf<MODE>::kUnits, Q = 16 / U;
+        T *dst = static_cast<T *>(pk) + ((size_t)(ri * kPanel + t) * U * 4 + rb) * 64 + lane;
+#pragma unroll
+        for (int uu = 0; uu < U / 4; uu++) {
+            const int u = U / 4 * w + uu;
+            T v;
+#pragma unroll
+            for (int q = 0; q < Q; q++) v[q] = at(4 * (Q * u + q) + k4);
+            dst[256 * u] = v;
+        }
+    };
+#pragma unroll
+    for (int t = 0; t < kPanel; t++) {
+        const dbl2 *src = reinterpret_cast<const dbl2 *>(row + t * TB);
+        const dbl2 lo = src[0], hi = src[1];
+        acc[t] = dbl4{lo.x, lo.y, hi.x, hi.y};
+    }
+    fetch(std::integral_constant<int, 0>{});
+    fetch(std::integral_constant<int, 1>{});
+    put(Bs, acc[0]);
+    __syncthreads();
+    get(Bs, y);
+    auto step = [&](auto E) {
+        constexpr PanelTile q = panel_tile(E);
+        if constexpr (E + 2 < kPanelTiles) fetch(std::integral_constant<int, E + 2>{});
+        if constexpr (q.t == q.k) {
+            const dbl4 v = products(op[E % 3], y, dbl4{0.0, 0.0, 0.0, 0.0});
+            store(q.k, v);
+        } else {
+            acc[q.t] = products(op[E % 3], x, acc[q.t]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // the exchanges: column k + 1 once updated by k, read one update
+        // later; the solved column after the last update by the one before
+        constexpr PanelTile n = panel_tile(E + 1);
+        if constexpr (q.t == q.k + 1) put(Bs, acc[q.t]);
+        if constexpr (q.t != q.k && (q.t == q.k + 2 || n.t == q.k + 1) && q.t < q.k + 3) {
+            __syncthreads();
+            get(Bs, y);
+        }
+        if constexpr (n.t == n.k + 1 || E == kPanelTiles - 1) {
+            constexpr int k = E == kPanelTiles - 1 ? kPanel - 1 : n.k;
+            __syncthreads();
+            get(Xs, x);
+            pack(k);
+        }
+    };
+    static_steps(step, std::make_integer_sequence<int, kPanelTiles>{});
 }
 
 // Factor and inverse of the diagonal tile (d, d) by one workgroup (the
@@ -1688,28 +1934,90 @@ void chol_column(const CholWork &c, int kb, int jcols, hipStream_t q) {
         k_step<MODE><<<grid, 256, 0, q>>>(c.A, c.ld, kb, jcols, c.Linv, c.neg);
     }
 }
+// tiles lin .. lin + n - 1 of the trailing update from packed panels
+template <int MODE>
+void trail_tiles(const CholWork &c, int nb, int j0, int lin, int n, hipStream_t q) {
+    k_trail_pk<MODE><<<xcd_grid(n), 256, 0, q>>>(c.A, c.ld, c.sp, nb, j0, c.mpad / TB, lin, n, c.Linv, c.neg);
+}
+template <int MODE>
+void trail_direct(const CholWork &c, int k0, int nb, hipStream_t q) {
+    const int nt = c.mpad / TB, j0 = k0 + nb, SM = (nt - j0 + 7) / 8;
+    k_trail<MODE><<<SM * (SM + 1) / 2 * 64, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, nt, c.Linv, c.neg);
+}
 template <int MODE>
 void chol_trail(const CholWork &c, int k0, int nb, hipStream_t q) {
-    const int nt = c.mpad / TB, j0 = k0 + nb;
-    // packed wherever the buffer holds the panel: with its packing pass FP64
-    // takes 80 us against 87 at 40 trailing block rows, 39 against 45 at 20
-    // (FP32 56 and 29), and in BF16 the direct form splits every operand
-    // fragment in every workgroup
-    if (c.sp && nb <= c.sp_nb && nt - j0 >= c.pack_min_rows) {
-        // panel tiles packed (split) once, tiles in 8x8 groups over the XCDs
-        const int R = nt - j0;
+    const int nt = c.mpad / TB, j0 = k0 + nb, R = nt - j0;
+    if (c.sp && nb <= c.sp_nb && R >= c.pack_min_rows) {
         if constexpr (MODE == 2) {
             __bf16 *sp = static_cast<__bf16 *>(c.sp);
+            const int S = (R + 1) / 2, n = S * (S + 1) / 2;
             k_split3<<<R * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, sp);
-            k_trail_bf<<<group_grid((R + 1) / 2), 256, 0, q>>>(c.A, c.ld, sp, nb, j0, nt, c.Linv, c.neg);
+            k_trail_bf<<<xcd_grid(n), 256, 0, q>>>(c.A, c.ld, sp, nb, j0, nt, n, c.Linv, c.neg);
         } else {
             k_pack64<MODE><<<R * nb, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, c.sp);
-            k_trail_pk<MODE><<<group_grid(R), 256, 0, q>>>(c.A, c.ld, c.sp, nb, j0, nt, c.Linv, c.neg);
+            trail_tiles<MODE>(c, nb, j0, 0, R * (R + 1) / 2, q);
         }
-        return;
+    } else {
+        trail_direct<MODE>(c, k0, nb, q);
     }
-    const int SM = (nt - j0 + 7) / 8;
-    k_trail<MODE><<<SM * (SM + 1) / 2 * 64, 256, 0, q>>>(c.A, c.ld, k0, nb, j0, nt, c.Linv, c.neg);
+}
+// Factor in super-panels of kPanel block columns, FP64 and FP32 updates: per
+// panel the columns of its diagonal block with the tiles of the last trailing
+// update (one round of the CUs each), what is left of these tiles, the
+// panel's rows, and the first tiles of its trailing update, among them the
+// next diagonal block's.  The last block's columns are factored in c.mode's
+// arithmetic, as they are without panels.  Against whole panels column by column and the
+// trailing update in one launch (us, FP64): 200 nucleosomes 1449 -> 1375, 300
+// 2920 -> 2670, 500 8730 -> 8100, 1000 55200 -> 52100; FP32 300 2400 -> 2140,
+// 1000 37500 -> 32600.  In BF16, whose 128x128 blocks make poor company (300
+// nucleosomes 2210 -> 2330), the panels stay whole.
+template <int MODE>
+void chol_panels(const CholWork &c, hipStream_t q, MarkFn mark, void *mark_arg, hipEvent_t gate, int gate_kb) {
+    const int nt = c.mpad / TB, ncu = c.ncu;
+    auto M_ = [&](int id, int ph) { if (mark) mark(mark_arg, id, ph); };
+    auto done = [&](int kb) { if (gate && kb == gate_kb) (void)hipEventRecord(gate, q); };
+    int j0 = 0, lin = 0, end = 0;  // the trailing update in progress: blocks lin .. end - 1 left
+    for (int k0 = 0;; k0 += kPanel) {
+        const int kend = std::min(k0 + kPanel, nt);
+        for (int kb = k0; kb + 1 < kend; kb++) {
+            if (kend == nt) {
+                M_(K_CHOL_STEP, 0);
+                chol_column<MODE>(c, kb, nt - kb - 1, q);
+                M_(K_CHOL_STEP, 1);
+                done(kb);
+                continue;
+            }
+            const int jcols = kend - 1 - kb, G = jcols * (jcols + 1) / 2, n = std::min(end - lin, std::max(0, ncu - G) / 8 * 8);
+            M_(K_CHOL_STEP, 0);
+            k_block_step<MODE><<<G + xcd_grid(n), 256, 0, q>>>(c.A, c.ld, kb, jcols, c.sp, kPanel, j0, nt, lin, n, c.Linv, c.neg,
+                                                              c.Lp + ((kb - k0) * kPanel + kb - k0 + 1) * TB * TB);
+            M_(K_CHOL_STEP, 1);
+            lin += n;
+            done(kb);
+        }
+        if (kend == nt) break;
+        if (lin < end) {
+            M_(K_CHOL_TRAIL, 0);
+            trail_tiles<MODE>(c, kPanel, j0, lin, end - lin, q);
+            M_(K_CHOL_TRAIL, 1);
+        }
+        j0 = kend;
+        const bool packed = c.sp && c.sp_nb >= kPanel && nt - j0 >= c.pack_min_rows;
+        M_(K_CHOL_STEP, 0);
+        k_panel_rows<MODE><<<4 * (nt - j0), 256, 0, q>>>(c.A, c.ld, k0, c.Linv, c.Lp, packed ? c.sp : nullptr);
+        M_(K_CHOL_STEP, 1);
+        done(kend - 1);
+        M_(K_CHOL_TRAIL, 0);
+        if (packed) {
+            end = (nt - j0) * (nt - j0 + 1) / 2;
+            lin = std::min(end, std::max(kPanel * (kPanel + 1) / 2, ncu / 8 * 8));
+            k_block_step<MODE><<<xcd_grid(lin), 256, 0, q>>>(c.A, c.ld, 0, 0, c.sp, kPanel, j0, nt, 0, lin, c.Linv, c.neg, nullptr);
+        } else {
+            trail_direct<MODE>(c, k0, kPanel, q);
+            lin = end = 0;
+        }
+        M_(K_CHOL_TRAIL, 1);
+    }
 }
 }  // namespace
 
@@ -1718,16 +2026,16 @@ size_t split_bytes(int ld, int nb) {
                     (size_t)(ld / TB) * nb * TB * TB * sizeof(double));
 }
 
-// Super-panels from 84 block columns in FP64 (us a step without / with them,
-// panels of 8: 66 block columns 2129 / 2237, 76 2666 / 2680, 86 3347 / 3351,
-// 99 4471 / 4287, 115 6161 / 5690).  In the reduced modes from 64, where the
-// panel's own columns also gain FP64 arithmetic (FP32 66 block columns 2276 /
-// 2341, 76 2827 / 2804; BF16 66 2506 / 2278).
+// Super-panels from 60 block columns in FP64 (us a factor without / with them:
+// 56 block columns 1086 / 1088, 59 1181 / 1176, 63 1321 / 1263, 72 1703 /
+// 1515).  In the reduced modes from 64: FP32 would gain from 52 (53 952 / 938,
+// 63 1233 / 1110), but a panel's own columns are FP64, so the line also says
+// which rounding errors a factor has.
 int chol_panel_tiles(const CholWork &c) {
     const int nt = c.mpad / TB;
     if (c.panel_tiles > 0) return c.panel_tiles >= 2 && nt > c.panel_tiles ? c.panel_tiles : 0;
     if (c.panel_tiles < 0) return 0;
-    return nt >= (c.mode == 0 ? 84 : 64) ? 8 : 0;
+    return nt >= (c.mode == 0 ? 60 : 64) ? kPanel : 0;
 }
 
 void launch_cholesky(const CholWork &c, hipStream_t q, MarkFn mark, void *mark_arg, hipEvent_t gate, int gate_kb) {
@@ -1743,6 +2051,12 @@ void launch_cholesky(const CholWork &c, hipStream_t q, MarkFn mark, void *mark_a
     };
     const int NB = chol_panel_tiles(c);
     int k0 = 0;
+    if (NB == kPanel && c.mode != 2) {
+        if (c.mode == 0) chol_panels<0>(c, q, mark, mark_arg, gate, gate_kb);
+        else chol_panels<1>(c, q, mark, mark_arg, gate, gate_kb);
+        if (gate && gate_kb >= nt - 1) (void)hipEventRecord(gate, q);
+        return;
+    }
     if (NB > 0) {
         // super-panels while a whole one and a trailing matrix remain; the
         // panel's own columns are factored in FP64 in every mode (the

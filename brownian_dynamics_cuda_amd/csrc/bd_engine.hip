@@ -590,9 +590,11 @@ int bd_create(const bd_system *sys, const bd_options *opt, bd_context **out) {
             ncu = prop.multiProcessorCount;
         c->ncu = ncu;
         c->chol.split_tiles = ncu * 19 / 10;
+        c->chol.ncu = ncu;
     }
     r |= c->alloc(&c->chol.A, (size_t)c->chol.ld * c->chol.ld);
     r |= c->alloc(&c->chol.Linv, (size_t)(c->chol.ld / 64) * 64 * 64);
+    r |= c->alloc(&c->chol.Lp, kPanelDoubles);
     r |= c->alloc(&c->chol.neg, 1);
     c->chol.refine = 1;
     if (const char *ev = getenv("BD_REFINE")) c->chol.refine = atoi(ev) != 0;

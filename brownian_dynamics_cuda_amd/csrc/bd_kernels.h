@@ -78,7 +78,11 @@ struct CholWork {
     // two-launch form (k_panel + k_update): about two rounds of workgroups
     // at one per CU
     int split_tiles;
-    // super-panel width in block columns: 0 chooses (8 from 84 block columns
+    int ncu;         // CUs of the device
+    // the panel tiles of a super-panel's diagonal block in operand order,
+    // kPanelDoubles doubles
+    double *Lp;
+    // super-panel width in block columns: 0 chooses (8 from 60 block columns
     // up in FP64, from 64 in the reduced modes, none below), -1 never, k >= 2
     // always k
     int panel_tiles;
@@ -96,6 +100,7 @@ struct CholWork {
     // smallest trailing matrix (block rows) that takes the packed form
     int pack_min_rows;
 };
+constexpr size_t kPanelDoubles = 64 * 64 * 64;
 // bytes of the packed / split panel buffer for leading dimension ld and
 // panels of nb
 size_t split_bytes(int ld, int nb);

@@ -47,13 +47,13 @@ int check_args(int m, const double *D, int ldd, const double *L, int ldl, int mo
     return BD_OK;
 }
 
-int split_tiles_of_current_device() {
+int cus_of_current_device() {
     int dev = 0, ncu = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
         int v = 0;
         if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) ncu = v;
     }
-    return ncu * 19 / 10;
+    return ncu;
 }
 
 CholWork work_of(int m, int mode) {
@@ -87,11 +87,13 @@ int run_factor(int m, const double *D, int ldd, double *L, int ldl, int mode, in
     c.A = ws;
     c.Linv = ws + (size_t)c.mpad * c.mpad;
     c.neg = reinterpret_cast<int *>(c.Linv + (size_t)(c.mpad / 64) * 64 * 64);
+    c.Lp = ws + workspace_doubles(m);
     if (packed) {
-        c.sp = ws + workspace_doubles(m);
+        c.sp = c.Lp + kPanelDoubles;
         c.sp_nb = chol_panel_tiles(c);
     }
-    c.split_tiles = split_tiles_of_current_device();
+    c.ncu = cus_of_current_device();
+    c.split_tiles = c.ncu * 19 / 10;
     launch_pack(D, ldd, c, q);
     launch_diag(c, 0, true, q);
     launch_cholesky(c, q);
@@ -145,7 +147,7 @@ int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, i
     hipStream_t q = static_cast<hipStream_t>(stream);
     double *ws = nullptr;
     // without room for the packed panel tiles the factor does without them
-    const size_t bytes = workspace_doubles(m) * sizeof(double), pack = pack_bytes(m, mode);
+    const size_t pack = pack_bytes(m, mode), bytes = (workspace_doubles(m) + (pack ? kPanelDoubles : 0)) * sizeof(double);
     const bool packed = pack && hipMalloc((void **)&ws, bytes + pack) == hipSuccess;
     if (!packed) {
         if (pack) (void)hipGetLastError();

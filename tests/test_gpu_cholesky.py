@@ -85,6 +85,26 @@ def test_ends_of_the_super_panels(m, mode):
     assert np.all(np.abs(L @ (L.T @ v) - D @ v) <= bound + (m + 1) * 2.0 ** -53 * (np.abs(D) @ np.abs(v)))
 
 
+@pytest.mark.parametrize("mode, nt", [(E.CHOL_FP64, 59), (E.CHOL_FP64, 60), (E.CHOL_FP64, 65), (E.CHOL_FP64, 71),
+                                      (E.CHOL_FP64, 81), (E.CHOL_FP32, 63), (E.CHOL_FP32, 64), (E.CHOL_FP32, 73)])
+def test_panels_solved_in_one_launch(mode, nt):
+    """The first sizes whose super-panels factor their diagonal block beside
+    the trailing update and solve their rows in one launch (60 and 64 block
+    columns) and the last without; last panels of one (65, 73, 81), four and
+    seven (71) block columns; 65 and more trailing block rows (two workgroups
+    per CU) and more tiles than the steps take (71, 73, 81); two rows of padding.
+    |L L^T - D| at most (m + 1) u |L| |L^T|, with u = 2^-53 in FP64 and 2^-24
+    for the products of FP32."""
+    m = 64 * nt - 2
+    D = spd(m, 3)
+    L, neg = E.cholesky_device(D, mode)
+    u = 2.0 ** (-53 if mode == E.CHOL_FP64 else -24)
+    v = np.random.default_rng(1).standard_normal((m, 4))
+    bound = (m + 1) * u * (np.abs(L) @ (np.abs(L.T) @ np.abs(v)))
+    assert neg == 0
+    assert np.all(np.abs(L @ (L.T @ v) - D @ v) <= bound + (m + 1) * 2.0 ** -53 * (np.abs(D) @ np.abs(v)))
+
+
 def test_super_panel_size_and_mixed_modes():
     """4500 rows: 71 block columns, super-panels of 8 in the reduced modes."""
     D = spd(4500, 7)
