@@ -164,16 +164,19 @@ __global__ void __launch_bounds__(256) k_rpy(Stat s, Geo g, const double *rad_al
 // of a workgroup, 16-byte accesses, fully unrolled: all eight global loads
 // of a thread are in flight before the first LDS store waits on them.
 constexpr int NTHR = 256;
+// thread of the team of 256 that works on a tile (k_step2 has two teams in a
+// workgroup)
+__device__ __forceinline__ int tid() { return threadIdx.x & (NTHR - 1); }
 __device__ __forceinline__ void load_tile(const double *A, int ld, int r0, int c0, double *S) {
     dbl2 v[TB * TB / 2 / NTHR];
 #pragma unroll
     for (int i = 0; i < TB * TB / 2 / NTHR; i++) {
-        const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        const int e = tid() + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
         v[i] = *reinterpret_cast<const dbl2 *>(A + (size_t)(r0 + r) * ld + c0 + c);
     }
 #pragma unroll
     for (int i = 0; i < TB * TB / 2 / NTHR; i++) {
-        const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        const int e = tid() + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
         S[r * LDP + c] = v[i].x;
         S[r * LDP + c + 1] = v[i].y;
     }
@@ -181,7 +184,7 @@ __device__ __forceinline__ void load_tile(const double *A, int ld, int r0, int c
 __device__ __forceinline__ void store_tile(double *A, int ld, int r0, int c0, const double *S, bool lower_only) {
 #pragma unroll
     for (int i = 0; i < TB * TB / 2 / NTHR; i++) {
-        const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        const int e = tid() + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
         dbl2 v;
         v.x = (lower_only && c > r) ? 0.0 : S[r * LDP + c];
         v.y = (lower_only && c + 1 > r) ? 0.0 : S[r * LDP + c + 1];
@@ -194,7 +197,7 @@ __device__ __forceinline__ void store_tile(double *A, int ld, int r0, int c0, co
 // B^T[l/16][l%16]; result register v of lane l is C[l/16 + 4v][l%16]
 // (measured on gfx950; the FP32 16x16x4 form places it at C[4(l/16)+v]).
 __device__ __forceinline__ void mma_f64(const double *As, const double *Bs, dbl4 acc[2][2]) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid() & 63, w = tid() >> 6;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32, i16 = lane & 15, k4 = lane >> 4;
     // the operands of K step kk + 4 are read while the products of step kk run
     const double *pa0 = As + (wr + i16) * LDP + k4, *pa1 = pa0 + 16 * LDP;
@@ -219,7 +222,7 @@ __device__ __forceinline__ void mma_f64(const double *As, const double *Bs, dbl4
 // Same product with FP32 operands and FP32 accumulation
 // (v_mfma_f32_16x16x4f32, identical lane layout).
 __device__ __forceinline__ void mma_f32(const double *As, const double *Bs, flt4 acc[2][2]) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid() & 63, w = tid() >> 6;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32, i16 = lane & 15, k4 = lane >> 4;
     const double *pa0 = As + (wr + i16) * LDP + k4, *pa1 = pa0 + 16 * LDP;
     const double *pb0 = Bs + (wc + i16) * LDP + k4, *pb1 = pb0 + 16 * LDP;
@@ -263,7 +266,7 @@ __device__ __forceinline__ void split3(const double *src, bf8 &h, bf8 &m, bf8 &l
     }
 }
 __device__ __forceinline__ void mma_bf16x3(const double *As, const double *Bs, flt4 acc[2][2]) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid() & 63, w = tid() >> 6;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32, i16 = lane & 15, k8 = lane >> 4;
 #pragma unroll
     for (int kk = 0; kk < TB; kk += 32) {
@@ -303,7 +306,7 @@ template <> struct AccOf<0> { typedef dbl4 T; };
 // lane l: l/16 + 4v for the FP64 MFMA, 4(l/16) + v for the FP32 one)
 template <typename V>
 __device__ __forceinline__ void acc_to_lds(double *C, V acc[2][2], double sign, bool overwrite) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid() & 63, w = tid() >> 6;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32, i16 = lane & 15, k4 = lane >> 4;
     constexpr bool f64 = sizeof(acc[0][0][0]) == 8;
     for (int mi = 0; mi < 2; mi++)
@@ -319,7 +322,7 @@ __device__ __forceinline__ void acc_to_lds(double *C, V acc[2][2], double sign, 
 // A 16x16 output block of the FP64 matrix cores (mapping of mma_f64:
 // register v of lane l is element (l/16 + 4v, l%16) of the block) into C.
 __device__ __forceinline__ void blk_to_lds(double *C, int I, int J, dbl4 acc, double sign, bool overwrite) {
-    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
+    const int lane = tid() & 63, i16 = lane & 15, k4 = lane >> 4;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         double *c = C + (16 * I + k4 + 4 * v) * LDP + 16 * J + i16;
@@ -334,7 +337,7 @@ __device__ __forceinline__ void blk_to_lds(double *C, int I, int J, dbl4 acc, do
 // wavefront issues the same 40 products.  Skipping the zero blocks adds
 // nothing to any sum, so P is the full product bit for bit.
 __device__ __forceinline__ void mma_panel(const double *As, const double *Li, dbl4 (&acc)[4]) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i16 = lane & 15, k4 = lane >> 4;
+    const int lane = tid() & 63, w = tid() >> 6, i16 = lane & 15, k4 = lane >> 4;
     const double *pa = As + (16 * w + i16) * LDP + k4, *pl = Li + i16 * LDP + k4;
     double na = pa[0], nb[4];
 #pragma unroll
@@ -357,7 +360,7 @@ __device__ __forceinline__ void mma_panel(const double *As, const double *Li, db
     }
 }
 __device__ __forceinline__ void panel_to_lds(double *C, const dbl4 (&acc)[4]) {
-    const int w = threadIdx.x >> 6;
+    const int w = tid() >> 6;
 #pragma unroll
     for (int J = 0; J < 4; J++) blk_to_lds(C, w, J, acc[J], 1.0, true);
 }
@@ -370,7 +373,7 @@ __device__ __forceinline__ void panel_to_lds(double *C, const dbl4 (&acc)[4]) {
 template <int N, int I0, int J0, int I1, int J1, int I2, int J2>
 __device__ __forceinline__ void syrk_blocks(const double *P, double *C) {
     constexpr int I[3] = {I0, I1, I2}, J[3] = {J0, J1, J2};
-    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
+    const int lane = tid() & 63, i16 = lane & 15, k4 = lane >> 4;
     const double *p = P + i16 * LDP + k4;
     dbl4 acc[N];
     double na[N], nb[N];
@@ -401,7 +404,7 @@ __device__ __forceinline__ void syrk_blocks(const double *P, double *C) {
     for (int b = 0; b < N; b++) blk_to_lds(C, I[b], J[b], acc[b], -1.0, false);
 }
 __device__ __forceinline__ void syrk_lower(const double *P, double *C) {
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w = __builtin_amdgcn_readfirstlane(tid() >> 6);
     // (I, J) blocks of wavefront w: {00 10 11} {20 21 22} {30 31} {32 33}
     if (w == 0) syrk_blocks<3, 0, 0, 1, 0, 1, 1>(P, C);
     else if (w == 1) syrk_blocks<3, 2, 0, 2, 1, 2, 2>(P, C);
@@ -599,7 +602,7 @@ constexpr int kNextPitch = 18;
 
 // the operand register of a panel: lane (k, c) holds row k, column c
 __device__ __forceinline__ double panel_op(const double *S, int p) {
-    const int lane = threadIdx.x & 63;
+    const int lane = tid() & 63;
     return S[64 * p + 4 * (lane & 15) + (lane >> 4)];
 }
 __device__ __forceinline__ dbl4 rank4(double a, double b, dbl4 acc) {
@@ -608,7 +611,7 @@ __device__ __forceinline__ dbl4 rank4(double a, double b, dbl4 acc) {
 // rows 4P..4P+3 of w to a panel buffer (this lane's column)
 template <int P>
 __device__ __forceinline__ void put_rows(double *S, const double (&w)[16]) {
-    double2 *d = reinterpret_cast<double2 *>(S + 64 * P + 4 * (threadIdx.x & 15));
+    double2 *d = reinterpret_cast<double2 *>(S + 64 * P + 4 * (tid() & 15));
     d[0] = make_double2(w[4 * P], w[4 * P + 1]);
     d[1] = make_double2(w[4 * P + 2], w[4 * P + 3]);
 }
@@ -631,7 +634,7 @@ __device__ __forceinline__ void pivot_panel(double (&w)[16], double (&r)[16], do
     pivot<4 * P + 1>(w, r, y, f, n);
     pivot<4 * P + 2>(w, r, y, f, n);
     pivot<4 * P + 3>(w, r, y, f, n);
-    const int lane = threadIdx.x & 63;
+    const int lane = tid() & 63;
     if (lane < 16) put_rows<P>(l.W(b, b), w);
     if (lane == 16) {
         double2 *d = reinterpret_cast<double2 *>(l.R() + 16 * b + 4 * P);
@@ -647,7 +650,7 @@ __device__ __forceinline__ void pivot_panel(double (&w)[16], double (&r)[16], do
 template <int P>
 __device__ __forceinline__ void follow_panel(double (&x)[16], const DiagLds &l, double *Y, int b) {
     __syncthreads();
-    const double2 *u2 = reinterpret_cast<const double2 *>(l.W(b, b) + 64 * P + 4 * (threadIdx.x & 15));
+    const double2 *u2 = reinterpret_cast<const double2 *>(l.W(b, b) + 64 * P + 4 * (tid() & 15));
     const double2 *r2 = reinterpret_cast<const double2 *>(l.R() + 16 * b + 4 * P);
     const double2 ua = u2[0], ub = u2[1], ra = r2[0], rb = r2[1];
     const double u[4] = {ua.x, ua.y, ub.x, ub.y}, r[4] = {ra.x, ra.y, rb.x, rb.y};
@@ -662,7 +665,7 @@ __device__ __forceinline__ void follow_panel(double (&x)[16], const DiagLds &l, 
 // L(b + q, b) for q < 4 - b, inv(L)(b, q - (4 - b)) after them: block q of
 // the five that block row b leaves, scaled by 1/sqrt(|f|) and stored.
 __device__ __forceinline__ void store_block(const DiagLds &l, int b, int q, double *A, int ld, int d0, double *Linv) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
+    const int lane = tid() & 63, g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
     const bool isl = q < 4 - b;
     const int j = isl ? b + q : q - (4 - b);
     const double2 *s = reinterpret_cast<const double2 *>((isl ? l.W(b, j) : l.E(b, j)) + 64 * g + 4 * c);
@@ -685,7 +688,7 @@ __device__ __forceinline__ void store_block(const DiagLds &l, int b, int q, doub
 
 // Block (i, j) of the tile, i <= j, in matrix-core result registers
 __device__ __forceinline__ dbl4 tile_block(const double *T, int i, int j) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
+    const int lane = tid() & 63, g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
     dbl4 x;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
@@ -696,7 +699,7 @@ __device__ __forceinline__ dbl4 tile_block(const double *T, int i, int j) {
 }
 // a finished block of block row b + 1 to its reader
 __device__ __forceinline__ void put_next(const DiagLds &l, int q, dbl4 x) {
-    const int lane = threadIdx.x & 63;
+    const int lane = tid() & 63;
     double2 *d = reinterpret_cast<double2 *>(l.next(q) + kNextPitch * (lane & 15) + 4 * (lane >> 4));
     d[0] = make_double2(x[0], x[1]);
     d[1] = make_double2(x[2], x[3]);
@@ -706,7 +709,7 @@ __device__ __forceinline__ void put_next(const DiagLds &l, int q, dbl4 x) {
 // I0 to I1: U = 0 has C11 C12 C22 C23 C33 E31, U = 1 has C13 E10 E20 E21 E30 E32.
 template <int B, int U, int I0, int I1>
 __device__ __forceinline__ void below_panel(dbl4 (&Z)[6], const DiagLds &l, int p) {
-    const int g = (threadIdx.x & 63) >> 4;
+    const int g = (tid() & 63) >> 4;
     const double rn = -l.R()[16 * B + 4 * p + g];
     double a[4], e[3];
 #pragma unroll
@@ -762,7 +765,7 @@ __device__ __forceinline__ void below_row(dbl4 (&Z)[6], const DiagLds &l) {
 // diagonal, to Linv.
 __device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, double *A, int ld, int d0, double *Linv,
                                                 int *neg) {
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = tid() & 63, wv = __builtin_amdgcn_readfirstlane(tid() >> 6);
     const int g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
     const DiagLds l = {lds};
     if (wv == 0) {
@@ -847,14 +850,14 @@ constexpr int PERT = TB * TB / 2 / NTHR;
 __device__ __forceinline__ void tile_to_regs(const double *src, int ld, dbl2 (&v)[PERT]) {
 #pragma unroll
     for (int i = 0; i < PERT; i++) {
-        const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        const int e = tid() + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
         v[i] = *reinterpret_cast<const dbl2 *>(src + (size_t)r * ld + c);
     }
 }
 __device__ __forceinline__ void regs_to_lds(const dbl2 (&v)[PERT], double *S) {
 #pragma unroll
     for (int i = 0; i < PERT; i++) {
-        const int e = threadIdx.x + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        const int e = tid() + i * NTHR, r = e / (TB / 2), c = 2 * (e % (TB / 2));
         S[r * LDP + c] = v[i].x;
         S[r * LDP + c + 1] = v[i].y;
     }
@@ -867,7 +870,7 @@ __device__ __forceinline__ void tile_update(const double *Pi, const double *Pj, 
     for (int a = 0; a < 2; a++)
         for (int b = 0; b < 2; b++) acc[a][b] = {};
     tile_mma<MODE>(Pi, Pj, acc);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid() & 63, w = tid() >> 6;
     const int wr = (w >> 1) * 32, wc = (w & 1) * 32, i16 = lane & 15, k4 = lane >> 4;
     constexpr bool f64 = MODE == 0;
     double cv[2][2][4];
@@ -906,10 +909,10 @@ __device__ __forceinline__ void diag_tile_update(const double *P, double *C) {
 // A tile from LDS by wavefronts 2 and 3, which have two of syrk_lower's
 // blocks where 0 and 1 have three
 __device__ __forceinline__ void store_tile_half(double *dst, int ld, const double *S) {
-    if (threadIdx.x < NTHR / 2) return;
+    if (tid() < NTHR / 2) return;
 #pragma unroll
     for (int i = 0; i < 2 * PERT; i++) {
-        const int e = threadIdx.x - NTHR / 2 + i * (NTHR / 2), r = e / (TB / 2), c = 2 * (e % (TB / 2));
+        const int e = tid() - NTHR / 2 + i * (NTHR / 2), r = e / (TB / 2), c = 2 * (e % (TB / 2));
         *reinterpret_cast<dbl2 *>(dst + (size_t)r * ld + c) = dbl2{S[r * LDP + c], S[r * LDP + c + 1]};
     }
 }
@@ -919,7 +922,7 @@ __device__ __forceinline__ void store_tile_half(double *dst, int ld, const doubl
 // row_pi(l % 16), K = 16 b + 4 (l / 16) + 2 h and the next
 __device__ __forceinline__ int row_pi(int i16) { return 4 * (i16 & 3) + (i16 >> 2); }
 __device__ __forceinline__ void store_operand(double *dst, const double *S) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid() & 63, w = tid() >> 6;
     const double *src = S + (16 * w + row_pi(lane & 15)) * LDP + 4 * (lane >> 4);
 #pragma unroll
     for (int u = 0; u < 8; u++) {
@@ -1030,6 +1033,32 @@ __global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int 
     const int G8 = gridDim.x / 8;
     if (lb < 8 * G8) lb = (lb % 8) * G8 + lb / 8;
     step_tile<MODE>(S, A, ld, kb, jcols, lb, Linv, neg, nullptr);
+}
+
+// The same with one workgroup of two teams per CU, for 257 to 511 tiles: tile
+// 0 has workgroup 0, and with it a CU, to itself, so that its factor, a chain
+// of FP64 vector arithmetic, does not stand still beside another workgroup's
+// matrix products; the others go in contiguous runs to the XCDs (workgroups go
+// round-robin over the eight), each XCD's as many as it has teams for.  The
+// teams share their barriers, which a team that has left no longer takes part
+// in.  17.0 us against 18.4 (253 tiles in k_step: 15.5); what is left are two
+// tiles' products on a CU, 10.2 us.  k_update in this form, its teams going
+// from tile to tile, took 18 to 28 us against 15 to 20.
+constexpr int kStep2Tiles(int grid) { return 2 * (grid - 1) + 1; }
+template <int MODE>
+__global__ void __launch_bounds__(512, 2) k_step2(double *A, int ld, int kb, int jcols, int n, double *Linv, int *neg) {
+    __shared__ double S[2 * kStepLds];
+    const int team = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int per = gridDim.x / 8, x = blockIdx.x & 7, all = 2 * ((int)gridDim.x - 1);
+    const int before = x ? 2 * (per - 1) + 2 * per * (x - 1) : 0, own = x ? 2 * per : 2 * (per - 1);
+    const int t0 = (n - 1) * before / all, t1 = (n - 1) * (before + own) / all;
+    int lb = t0 + 2 * ((blockIdx.x >> 3) - (x == 0)) + team, end = t1;
+    if (blockIdx.x == 0) {
+        lb = team - 1;
+        end = 0;
+    }
+    if (lb >= end) return;
+    step_tile<MODE>(S + team * kStepLds, A, ld, kb, jcols, lb + 1, Linv, neg, nullptr);
 }
 
 // The same block column in two launches, for wide trailing matrices (many
@@ -1930,6 +1959,8 @@ void chol_column(const CholWork &c, int kb, int jcols, hipStream_t q) {
     } else if (grid >= c.split_tiles) {
         k_panel<<<M, 256, 0, q>>>(c.A, c.ld, kb, c.Linv);
         k_update<MODE><<<grid, 256, 0, q>>>(c.A, c.ld, kb, jcols, c.Linv, c.neg);
+    } else if (grid > c.ncu && grid <= kStep2Tiles(c.ncu / 8 * 8)) {
+        k_step2<MODE><<<c.ncu / 8 * 8, 512, 0, q>>>(c.A, c.ld, kb, jcols, grid, c.Linv, c.neg);
     } else {
         k_step<MODE><<<grid, 256, 0, q>>>(c.A, c.ld, kb, jcols, c.Linv, c.neg);
     }
