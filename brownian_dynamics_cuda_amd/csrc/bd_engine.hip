@@ -64,6 +64,16 @@ namespace bd {
 void set_last_error(const char *msg) { g_err = msg; }
 }  // namespace bd
 
+// hipMalloc, with the workspaces bd_cholesky has kept given back where it fails
+static hipError_t device_malloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && release_workspaces()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 struct bd_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -118,7 +128,7 @@ struct bd_context {
     int alloc(T **p, size_t count) {
         size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
         void *q = nullptr;
-        hipError_t e = hipMalloc(&q, bytes);
+        hipError_t e = device_malloc(&q, bytes);
         if (e != hipSuccess) return fail(BD_E_HIP, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
         allocs.push_back(q);
         *p = static_cast<T *>(q);
@@ -864,7 +874,7 @@ int bd_run_steps(bd_context *c, int k, const double *rr, const double *p, double
         if (c->batch) (void)hipFree(c->batch);
         c->batch = nullptr;
         c->batch_cap = 0;
-        hipError_t e = hipMalloc((void **)&c->batch, need * sizeof(double));
+        hipError_t e = device_malloc((void **)&c->batch, need * sizeof(double));
         if (e != hipSuccess) return fail(BD_E_HIP, "hipMalloc(%zu): %s", need * sizeof(double), hipGetErrorString(e));
         c->batch_cap = need;
     }
@@ -1069,7 +1079,7 @@ int bd_get_work_counts(bd_context *c, bd_work_counts *w) {
 
 int bd_device_alloc(size_t bytes, void **ptr) {
     if (!ptr) return fail(BD_E_ARG, "null argument");
-    HIPCHK(hipMalloc(ptr, bytes));
+    HIPCHK(device_malloc(ptr, bytes));
     return BD_OK;
 }
 int bd_device_free(void *ptr) {

@@ -104,6 +104,8 @@ constexpr size_t kPanelDoubles = 64 * 64 * 64;
 // bytes of the packed / split panel buffer for leading dimension ld and
 // panels of nb
 size_t split_bytes(int ld, int nb);
+// frees the workspaces bd_cholesky has kept (false: there were none)
+bool release_workspaces();
 // super-panel width the factor of c uses (0: one block column at a time)
 int chol_panel_tiles(const CholWork &c);
 // D into c.A; also clears the negative-pivot count of the factor that

@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <mutex>
 #include <string>
+#include <utility>
 
 #include "../../include/bd_hip.h"
 #include "bd_kernels.h"
@@ -106,6 +107,46 @@ int run_factor(int m, const double *D, int ldd, double *L, int ldl, int mode, in
     return BD_OK;
 }
 
+constexpr int kMaxDevices = 64;
+
+// The workspace of the last bd_cholesky call on each device, kept for the
+// next one: hipMalloc and hipFree took 360 of the 1240 us of a 3001-row factor.
+// A call takes the workspace out and puts it back when its stream is done with
+// it, so calls that overlap (threads, streams) never share one, and at most one
+// workspace of at most kKeepBytes stays per device.  It is given back by
+// bd_cholesky_release, by a call that needs a larger one and when an allocation
+// of the library fails.
+constexpr size_t kKeepBytes = (size_t)256 << 20;
+struct Workspace {
+    void *ptr;
+    size_t bytes;
+};
+std::mutex g_kept_mu;
+Workspace g_kept[kMaxDevices] = {};
+
+Workspace exchange_kept(int dev, Workspace w) {
+    if (dev < 0 || dev >= kMaxDevices) return w;
+    std::lock_guard<std::mutex> lock(g_kept_mu);
+    std::swap(g_kept[dev], w);
+    return w;
+}
+
+// at least bytes on the current device dev: the kept workspace if it is large
+// enough, else a new one in its place
+hipError_t take_workspace(int dev, size_t bytes, Workspace *w) {
+    *w = exchange_kept(dev, {});
+    if (w->bytes >= bytes) return hipSuccess;
+    if (w->ptr) (void)hipFree(w->ptr);
+    *w = {nullptr, bytes};
+    const hipError_t e = hipMalloc(&w->ptr, bytes);
+    if (e != hipSuccess) *w = {};
+    return e;
+}
+hipError_t give_workspace(int dev, Workspace w, bool keep) {
+    if (keep && w.bytes <= kKeepBytes) w = exchange_kept(dev, w);
+    return w.ptr ? hipFree(w.ptr) : hipSuccess;
+}
+
 // Workspace of bd_cholesky_noalloc: a static device array of the library,
 // sized for matrices of up to kNoallocMaxM rows (33 block columns; the
 // 2082-row tensor of the 100-nucleosome fiber fits): 36.8 MB that every GPU
@@ -117,7 +158,6 @@ constexpr size_t kNoallocDoubles =
     (size_t)kNoallocMaxM * kNoallocMaxM + (size_t)(kNoallocMaxM / 64) * 64 * 64 + 32;
 static __device__ __align__(256) double scratch[kNoallocDoubles];
 
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double *g_scratch[kMaxDevices] = {};
 
@@ -139,24 +179,43 @@ int scratch_of_current_device(double **out) {
 
 }  // namespace
 
+bool bd::release_workspaces() {
+    bool any = false;
+    for (int dev = 0; dev < kMaxDevices; dev++) {
+        const Workspace w = exchange_kept(dev, {});
+        if (!w.ptr) continue;
+        any = true;
+        (void)hipFree(w.ptr);
+    }
+    return any;
+}
+
 extern "C" {
 
 int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, int *neg, void *stream) {
     int r = check_args(m, D, ldd, L, ldl, mode);
     if (r) return r;
     hipStream_t q = static_cast<hipStream_t>(stream);
-    double *ws = nullptr;
+    int dev = 0;
+    POTRF_CHK(hipGetDevice(&dev));
+    Workspace ws{};
     // without room for the packed panel tiles the factor does without them
     const size_t pack = pack_bytes(m, mode), bytes = (workspace_doubles(m) + (pack ? kPanelDoubles : 0)) * sizeof(double);
-    const bool packed = pack && hipMalloc((void **)&ws, bytes + pack) == hipSuccess;
+    const bool packed = pack && take_workspace(dev, bytes + pack, &ws) == hipSuccess;
     if (!packed) {
         if (pack) (void)hipGetLastError();
-        POTRF_CHK(hipMalloc((void **)&ws, bytes));
+        POTRF_CHK(take_workspace(dev, bytes, &ws));
     }
-    r = run_factor(m, D, ldd, L, ldl, mode, neg, q, ws, packed);
-    hipError_t e = hipFree(ws);
+    r = run_factor(m, D, ldd, L, ldl, mode, neg, q, static_cast<double *>(ws.ptr), packed);
+    // a call that failed may have left work on the stream: nothing is kept
+    const hipError_t e = give_workspace(dev, ws, r == BD_OK);
     if (r) return r;
     if (e != hipSuccess) return fail(BD_E_HIP, "hipFree: %s", hipGetErrorString(e));
+    return BD_OK;
+}
+
+int bd_cholesky_release(void) {
+    release_workspaces();
     return BD_OK;
 }
 

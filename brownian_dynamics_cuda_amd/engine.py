@@ -93,6 +93,7 @@ API = {
                        + [C.c_double] * 4 + [C.c_void_p] * 5, C.c_int),
     "bd_cholesky": ([C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int, _ip, C.c_void_p],
                     C.c_int),
+    "bd_cholesky_release": ([], C.c_int),
     "bd_cholesky_noalloc": ([C.c_int, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_int, _ip,
                              C.c_void_p], C.c_int),
     "bd_get_chol_schedule": ([C.c_void_p, _ip], C.c_int),

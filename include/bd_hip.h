@@ -206,10 +206,13 @@ int bd_get_chol_schedule(bd_context *ctx, int *panel_tiles_used);
  * and L may be the same buffer when ldd == ldl.  mode: BD_CHOL_*.  neg: host
  * int for the count of negative pivots (may be NULL).  stream: a hipStream_t
  * (NULL: the default stream); the call returns once the factor is done.
- * The workspace, (64 ceil(m/64))^2 + 4096 ceil(m/64) doubles, is allocated
- * and freed by the call. */
+ * The workspace, (64 ceil(m/64))^2 + 4096 ceil(m/64) doubles and from 60
+ * block columns about 1.4 % more, is allocated by the call.  One of at most 256
+ * MiB per device is kept for the next call; calls that overlap have one each.
+ * bd_cholesky_release frees what is kept. */
 int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, int *neg,
                 void *stream);
+int bd_cholesky_release(void);
 
 /* bd_cholesky without any allocation: no counterpart in the reference; for
  * callers that cannot allocate device memory (code under HIP graph capture,

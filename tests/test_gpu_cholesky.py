@@ -3,6 +3,7 @@
 C-ABI, against the compiled reference's factor (the |f| rule of
 func.cpp:825-835), LAPACK, and the factor the step itself takes."""
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -115,6 +116,35 @@ def test_super_panel_size_and_mixed_modes():
         Lm, neg = E.cholesky_device(D, mode)
         err = np.linalg.norm(Lm @ Lm.T - D) / np.linalg.norm(D)
         assert neg == 0 and err <= 1e-6, (mode, err)
+
+
+@pytest.mark.parametrize("threads", [1, 3])
+def test_kept_workspace(threads):
+    """The workspace kept between calls: sizes that need a larger one, fit the
+    kept one and leave most of it unused, from one thread and from three at
+    once, with a release in between; each call's factor as the first one's."""
+    lib = E.load_library()
+    sizes = [65, 700, 130, 1, 700, 900, 64]
+    mats = {m: spd(m, m) for m in sizes}
+    assert lib.bd_cholesky_release() == 0
+    ref = {m: np.linalg.cholesky(D) for m, D in mats.items()}
+    bad = []
+
+    def work(first):
+        for rep in range(2):
+            for m in sizes[first:] + sizes[:first]:
+                L, neg = E.cholesky_device(mats[m])
+                if neg != 0 or rel_err(L, ref[m]) > 1e-12:
+                    bad.append((first, m))
+            lib.bd_cholesky_release()
+
+    ts = [threading.Thread(target=work, args=(2 * i,)) for i in range(threads)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
+    assert lib.bd_cholesky_release() == 0 and lib.bd_cholesky_release() == 0
 
 
 def test_same_factor_as_the_step():
