@@ -1734,7 +1734,10 @@ __global__ void __launch_bounds__(256, 2) k_panel_rows(double *A, int ld, int k0
             const dbl4 v = products(op[E % 3], y, dbl4{0.0, 0.0, 0.0, 0.0});
             store(q.k, v);
         } else {
-            acc[q.t] = products(op[E % 3], x, acc[q.t]);
+            // summed apart, as column by column: chained onto the block the 512
+            // products leave a residual L L^T - D 1.5 times as large
+            acc[q.t] += products(op[E % 3], x, dbl4{0.0, 0.0, 0.0, 0.0});
+            asm volatile("" : "+v"(acc[q.t]));  // added here, not where it is next read
         }
         __builtin_amdgcn_sched_barrier(0);
         // the exchanges: column k + 1 once updated by k, read one update
