@@ -92,6 +92,7 @@ __host__ __device__ inline int nchunks(int n) { return (n + kChunk - 1) / kChunk
 // each cell are the partner indices in increasing order, cells in x-fastest
 // order, so a run of cells along x is one contiguous range of members.
 constexpr int kCellMax = 1 << 17;
+constexpr int kCellBoxes = 32;  // shares of a set's points in the build
 struct CellGrid {
     // the set's points for the build, set per pass by launch_sites:
     // point k is at pos + 3 idx[k] (idx NULL: pos + 3 k)
@@ -101,9 +102,10 @@ struct CellGrid {
     double *hdr;   // 4: origin x, y, z and 1 / edge
     int *dim;      // 3: nx, ny, nz (0 for an empty set)
     int *start;    // kCellMax + 1: first member of each cell
-    int *cursor;   // kCellMax: fill cursor of the build
+    double *box;   // 6 kCellBoxes: lowest and highest coordinates of the shares
     int *members;  // partner indices, cell by cell
     int *cid;      // cell of each partner
+    int *rank;     // its place in arrival order among the cell's partners
 };
 // partner sets of the culled loops
 enum { SET_TAIL = 0, SET_LH = 1, SET_HEAD = 2, SET_LINKER = 3, NSETS = 4 };

@@ -553,9 +553,10 @@ int bd_create(const bd_system *sys, const bd_options *opt, bd_context **out) {
             r |= c->alloc(&cg.hdr, 4);
             r |= c->alloc(&cg.dim, 3);
             r |= c->alloc(&cg.start, (size_t)kCellMax + 1);
-            r |= c->alloc(&cg.cursor, (size_t)kCellMax);
+            r |= c->alloc(&cg.box, (size_t)6 * kCellBoxes);
             r |= c->alloc(&cg.members, cap[k]);
             r |= c->alloc(&cg.cid, cap[k]);
+            r |= c->alloc(&cg.rank, cap[k]);
         }
         // the grid build costs more than it saves on small fibers (measured:
         // 100 nucleosomes 987 steps/s with chunk spheres, 923 with cells);

@@ -319,22 +319,23 @@ __device__ __forceinline__ int block_excl_scan(int v, int *wsum, int *tot) {
     return off + x - v;
 }
 
-// One workgroup per partner set: bounding box, grid, counts, offsets and
-// the fill (atomic cursors; k_cell_sort orders each cell afterwards).
-constexpr int kCellThreads = 1024;
-__global__ void __launch_bounds__(kCellThreads) k_cells(Sites st) {
+// The grids, a set's points over many workgroups (blockIdx.y: the set): boxes
+// of shares of the points; the grid from the boxes, each point's cell and its
+// place among the cell's points in arrival order (k_cell_sort orders each cell
+// afterwards); offsets; members.  One workgroup per set for all of it, a chain
+// of passes over the points at one CU's latency, took 77 us at 300 nucleosomes
+// and 145 at 1000; these four launches take 19 at 300 (a force pass 976 -> 911
+// us, at 1000 2750 -> 2363).
+constexpr int kCellThreads = 256, kScanThreads = 1024;
+__global__ void __launch_bounds__(kCellThreads) k_cell_box(Sites st) {
     __shared__ double red[6 * (kCellThreads / 64)];
-    __shared__ double s_hdr[4];
-    __shared__ int s_dim[3], s_wsum[kCellThreads / 64];
-    const int set = blockIdx.x, tid = threadIdx.x;
-    const CellGrid cg = st.cg[set];
-    const int n = cg.n;
-    if (n == 0) {
-        if (tid < 3) cg.dim[tid] = 0;
-        return;
-    }
+    const CellGrid cg = st.cg[blockIdx.y];
+    const int n = cg.n, tid = threadIdx.x;
+    if (n == 0) return;
+    // no counts yet
+    for (int c = blockIdx.x * kCellThreads + tid; c <= kCellMax; c += kCellBoxes * kCellThreads) cg.start[c] = 0;
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int k = tid; k < n; k += kCellThreads) {
+    for (int k = blockIdx.x * kCellThreads + tid; k < n; k += kCellBoxes * kCellThreads) {
         const double3 p = grid_point(cg, k);
         lo[0] = fmin(lo[0], p.x); lo[1] = fmin(lo[1], p.y); lo[2] = fmin(lo[2], p.z);
         hi[0] = fmax(hi[0], p.x); hi[1] = fmax(hi[1], p.y); hi[2] = fmax(hi[2], p.z);
@@ -349,17 +350,43 @@ __global__ void __launch_bounds__(kCellThreads) k_cells(Sites st) {
     if (lane == 0)
         for (int d = 0; d < 3; d++) { red[6 * w + d] = lo[d]; red[6 * w + 3 + d] = hi[d]; }
     __syncthreads();
-    if (tid == 0) {
-        for (int i = 1; i < kCellThreads / 64; i++)
-            for (int d = 0; d < 3; d++) {
-                red[d] = fmin(red[d], red[6 * i + d]);
-                red[3 + d] = fmax(red[3 + d], red[6 * i + 3 + d]);
+    if (tid < 6) {
+        double v = red[tid];
+        for (int i = 1; i < kCellThreads / 64; i++) v = tid < 3 ? fmin(v, red[6 * i + tid]) : fmax(v, red[6 * i + tid]);
+        cg.box[6 * blockIdx.x + tid] = v;
+    }
+}
+__global__ void __launch_bounds__(kCellThreads) k_cell_count(Sites st) {
+    __shared__ double box[6], s_hdr[4];
+    __shared__ int s_dim[3];
+    const CellGrid cg = st.cg[blockIdx.y];
+    const int n = cg.n, tid = threadIdx.x;
+    if (n == 0) {
+        if (blockIdx.x == 0 && tid < 3) cg.dim[tid] = 0;
+        return;
+    }
+    if (tid < 64) {
+        static_assert(kCellBoxes <= 64, "one box per lane");
+        double v[6];
+#pragma unroll
+        for (int d = 0; d < 6; d++) v[d] = cg.box[6 * min(tid, kCellBoxes - 1) + d];
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int d = 0; d < 6; d++) {
+                const double y = __shfl_xor(v[d], o, 64);
+                v[d] = d < 3 ? fmin(v[d], y) : fmax(v[d], y);
             }
+        if (tid == 0)
+#pragma unroll
+            for (int d = 0; d < 6; d++) box[d] = v[d];
+    }
+    __syncthreads();
+    if (tid == 0) {
         // a box that is not finite (a trajectory that blew up) takes one cell
         double ext[3];
         for (int d = 0; d < 3; d++) {
-            ext[d] = red[3 + d] - red[d];
-            if (!(ext[d] >= 0.0 && ext[d] < 1e12)) { ext[d] = 0.0; red[d] = 0.0; }
+            ext[d] = box[3 + d] - box[d];
+            if (!(ext[d] >= 0.0 && ext[d] < 1e12)) { ext[d] = 0.0; box[d] = 0.0; }
         }
         double edge = kReach;
         int nd[3] = {1, 1, 1};
@@ -372,42 +399,49 @@ __global__ void __launch_bounds__(kCellThreads) k_cells(Sites st) {
             if (tot <= kCellMax) break;
             edge *= 1.25;
         }
-        for (int d = 0; d < 3; d++) { s_hdr[d] = red[d]; s_dim[d] = nd[d]; cg.hdr[d] = red[d]; cg.dim[d] = nd[d]; }
+        for (int d = 0; d < 3; d++) { s_hdr[d] = box[d]; s_dim[d] = nd[d]; }
         s_hdr[3] = 1.0 / edge;
-        cg.hdr[3] = s_hdr[3];
+        if (blockIdx.x == 0) {
+            for (int d = 0; d < 3; d++) { cg.hdr[d] = s_hdr[d]; cg.dim[d] = nd[d]; }
+            cg.hdr[3] = s_hdr[3];
+        }
     }
     __syncthreads();
-    const int nx = s_dim[0], ny = s_dim[1], nz = s_dim[2], nc = nx * ny * nz;
+    const int nx = s_dim[0], ny = s_dim[1], nz = s_dim[2];
     const double inv = s_hdr[3];
-    // counts, offsets and cursors: plain stores complete (the barrier waits
-    // for them) before the atomics of the next phase act on the same words,
-    // and the counts are read back through atomics, where they were formed
-    for (int c = tid; c <= nc; c += kCellThreads) cg.start[c] = 0;
-    __syncthreads();
-    for (int k = tid; k < n; k += kCellThreads) {
+    for (int k = blockIdx.x * kCellThreads + tid; k < n; k += gridDim.x * kCellThreads) {
         const int c = cell_of(grid_point(cg, k), s_hdr, inv, nx, ny, nz);
         cg.cid[k] = c;
-        atomicAdd(cg.start + c, 1);
+        cg.rank[k] = atomicAdd(cg.start + c, 1);
     }
-    __syncthreads();
+}
+// counts to offsets, four cells per thread and round (the counts past the last
+// cell are 0)
+__global__ void __launch_bounds__(kScanThreads) k_cell_scan(Sites st) {
+    __shared__ int s_wsum[kScanThreads / 64];
+    const CellGrid cg = st.cg[blockIdx.x];
+    if (cg.n == 0) return;
+    const int nc = cg.dim[0] * cg.dim[1] * cg.dim[2];
+    int4 *start = reinterpret_cast<int4 *>(cg.start);
+    const int4 zero = make_int4(0, 0, 0, 0);
     int carry = 0;
-    for (int base = 0; base < nc; base += kCellThreads) {
-        const int c = base + tid;
-        const int v = c < nc ? atomicAdd(cg.start + c, 0) : 0;
+    int4 next = 4 * (int)threadIdx.x < nc ? start[threadIdx.x] : zero;
+    for (int base = 0; base < nc; base += 4 * kScanThreads) {
+        const int i = base / 4 + threadIdx.x, j = i + kScanThreads;
+        const int4 v = next;
+        next = 4 * j < nc ? start[j] : zero;
         int tot;
-        const int ex = block_excl_scan<kCellThreads>(v, s_wsum, &tot);
-        if (c < nc) {
-            cg.start[c] = carry + ex;
-            cg.cursor[c] = carry + ex;
-        }
+        int x = carry + block_excl_scan<kScanThreads>(v.x + v.y + v.z + v.w, s_wsum, &tot);
+        if (4 * i < nc) start[i] = make_int4(x, x + v.x, x + v.x + v.y, x + v.x + v.y + v.z);
         carry += tot;
     }
-    if (tid == 0) cg.start[nc] = carry;
     __syncthreads();
-    for (int k = tid; k < n; k += kCellThreads) {
-        const int slot = atomicAdd(cg.cursor + cg.cid[k], 1);
-        cg.members[slot] = k;
-    }
+    if (threadIdx.x == 0) cg.start[nc] = carry;
+}
+__global__ void __launch_bounds__(kCellThreads) k_cell_fill(Sites st) {
+    const CellGrid cg = st.cg[blockIdx.y];
+    for (int k = blockIdx.x * kCellThreads + threadIdx.x; k < cg.n; k += gridDim.x * kCellThreads)
+        cg.members[cg.start[cg.cid[k]] + cg.rank[k]] = k;
 }
 
 // Members of every cell in increasing index order, one wavefront per cell
@@ -1382,7 +1416,13 @@ void launch_sites(const Stat &s, const Geo &g, const Sites &st, int *cc_count, h
         sp.cg[SET_LINKER].pos = g.r;
         sp.cg[SET_LINKER].idx = s.lnk;
         sp.cg[SET_LINKER].n = s.n_lnk;
-        k_cells<<<NSETS, kCellThreads, 0, q>>>(sp);
+        int most = 1;
+        for (int k = 0; k < NSETS; k++) most = std::max(most, sp.cg[k].n);
+        const dim3 points(std::min(nblk(most, kCellThreads), 128), NSETS);
+        k_cell_box<<<dim3(kCellBoxes, NSETS), kCellThreads, 0, q>>>(sp);
+        k_cell_count<<<points, kCellThreads, 0, q>>>(sp);
+        k_cell_scan<<<NSETS, kScanThreads, 0, q>>>(sp);
+        k_cell_fill<<<points, kCellThreads, 0, q>>>(sp);
         k_cell_sort<<<512, 256, 0, q>>>(s, st);
     }
 }
