@@ -206,6 +206,42 @@ __host__ __device__ __forceinline__ double exp_neg_t(double x, const double *tab
     p = __builtin_fma(p, r, 1.0);
     return __builtin_ldexp(tab[im & 31] * p, im >> 5);
 }
+// e^(-kappa d) in the same form from y = k d, k = -kappa 32/ln2: m = rint(y)
+// comes out of the low bits of y + 1.5 2^52, f = y - m is exact, and the series
+// of e^(f ln2/32) takes the powers of ln2/32 into its coefficients: no reduction
+// in two parts and no rounding and converting instructions.  The one rounding
+// of k moves the exponent by at most 2^-53 of itself, as that of the product
+// kappa d does in the form above.  c0 is c[0] in a vector register, the one
+// coefficient that shares an instruction with another.
+struct ExpCoefF {
+    double c[6];  // (ln2/32)^i / i!, i = 6 .. 1
+    double k;
+};
+inline ExpCoefF exp_coef_f(double kappa) {
+    const long double q = 0.693147180559945309417232121458176568L / 32.0L;
+    ExpCoefF e;
+    long double p = 1.0L, n = 1.0L;
+    for (int i = 1; i <= 6; i++) {
+        p *= q / n;
+        e.c[6 - i] = (double)p;
+        n += 1.0L;
+    }
+    e.k = (double)(-(long double)kappa / q);
+    return e;
+}
+__host__ __device__ __forceinline__ double exp_neg_f(double d, double c0, const double *tab, const ExpCoefF &e) {
+    const double big = 6755399441055744.0;
+    const double t = __builtin_fma(d, e.k, big);
+    long long bits;
+    __builtin_memcpy(&bits, &t, sizeof bits);
+    const int im = (int)bits;
+    const double f = __builtin_fma(d, e.k, big - t);
+    double p = __builtin_fma(c0, f, e.c[1]);
+#pragma unroll
+    for (int i = 2; i < 6; i++) p = __builtin_fma(p, f, e.c[i]);
+    p = __builtin_fma(p, f, 1.0);
+    return __builtin_ldexp(tab[im & 31] * p, im >> 5);
+}
 // sin and cos of x for |x| < 2^19 (the frame angles here lie within
 // [-2 pi, 2 pi]), branch-free: x = n pi/2 + r with n = rint(2x/pi) and pi/2
 // in three parts (the published constants of fdlibm's e_rem_pio2.c: two
@@ -391,18 +427,49 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
     return t;  // valid on thread 0
 }
 
+// Sums of K doubles over a wavefront, each lane left with the one of index
+// wave_sum_index<K>(lane): a round over lane bit M exchanges half of the values
+// for the other half's lanes, so K sums take K/2 + K/4 + .. + 1 exchanges and
+// not 6 K (10 sums: 13).  Every sum adds the same pairs as a tree of
+// __shfl_down, in either order: the same value bit for bit.
+template <int K, int M = 32>
+__device__ __forceinline__ double wave_sum_n(const double (&v)[K]) {
+    if constexpr (K == 1) {
+        double t = v[0];
+#pragma unroll
+        for (int o = M; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+        return t;
+    } else {
+        static_assert(M > 0, "at most 64 sums");
+        const bool high = threadIdx.x & M;
+        double u[(K + 1) / 2];
+#pragma unroll
+        for (int i = 0; i < K / 2; i++) {
+            const double keep = high ? v[2 * i + 1] : v[2 * i], send = high ? v[2 * i] : v[2 * i + 1];
+            u[i] = keep + __shfl_xor(send, M, 64);
+        }
+        if constexpr (K & 1) u[K / 2] = v[K - 1] + __shfl_xor(v[K - 1], M, 64);
+        return wave_sum_n<(K + 1) / 2, M / 2>(u);
+    }
+}
+// the sum a lane holds, -1 where another lane answers for it
+template <int K>
+__device__ __forceinline__ int wave_sum_index(int lane) {
+    int idx = 0, o = 32;
+#pragma unroll
+    for (int k = 1; k < K; k *= 2, o >>= 1)
+        if (lane & o) idx += k;
+    return (lane & (2 * o - 1)) == 0 && idx < K ? idx : -1;
+}
+
 // Block-wide sums of K doubles at once (fixed order); results valid on
 // thread 0.  sh must hold K * (NT / 64) doubles.
 template <int NT, int K>
 __device__ __forceinline__ void block_sum_n(double (&v)[K], double *sh) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < K; q++)
-        for (int o = 32; o > 0; o >>= 1) v[q] += __shfl_down(v[q], o, 64);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, idx = wave_sum_index<K>(lane);
+    const double mine = wave_sum_n(v);
     __syncthreads();
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < K; q++) sh[q * (NT / 64) + w] = v[q];
+    if (idx >= 0) sh[idx * (NT / 64) + w] = mine;
     __syncthreads();
     if (threadIdx.x == 0)
 #pragma unroll

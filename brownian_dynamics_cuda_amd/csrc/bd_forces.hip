@@ -1292,16 +1292,22 @@ constexpr int kCCThreads = 256;   // four wavefronts, a work unit each
 // summed in world axes about its centre and turned into body components by
 // k_cc_gather (equal to the reference's body-frame sum for an orthonormal
 // frame).  Lanes past the last charge repeat it and are weighted by 0.
-// exp(-kappa d) is the table form exp_neg_t: 2^(j/32) comes in as a kernel
+// exp(-kappa d) is the table form exp_neg_f: 2^(j/32) comes in as a kernel
 // argument and is copied to LDS once (32 doubles over the 64 banks, so any
-// mix of lanes reads it without conflict); the Taylor coefficients of e^r
-// come in as a kernel argument too, so they sit in scalar registers and each
-// Horner step is one FMA with a scalar addend (compile-time constants end up
-// in vector registers, where every step first copies its addend).
+// mix of lanes reads it without conflict); the coefficients come in as a
+// kernel argument too, so they sit in scalar registers and each Horner step is
+// one FMA with a scalar addend (compile-time constants end up in vector
+// registers, where every step first copies its addend).
+// Bound by the vector instructions of a pair of charges: 38 and a reciprocal
+// root, 44 before k_e q_k left the loop and exp took this form.  With that and
+// the slot's ten sums in 13 exchanges instead of 60 a force pass takes at 250
+// nucleosomes 559 us (633), at 600 1430 (1540).  Eight wavefronts per SIMD,
+// though a few values of the unit's set-up then go through scratch: six left
+// part of the grid for a second round.
 template <bool WITH_E>
-__global__ void __launch_bounds__(kCCThreads) k_cc_work(Stat s, Geo g, const double *__restrict__ Qp,
+__global__ void __launch_bounds__(kCCThreads, 8) k_cc_work(Stat s, Geo g, const double *__restrict__ Qp,
                                                        const int *__restrict__ list, const int *__restrict__ count,
-                                                       int nkb, int nlc, double *__restrict__ slots, ExpCoef6 ec,
+                                                       int nkb, int nlc, double *__restrict__ slots, ExpCoefF ec,
                                                        Exp2Tab et) {
     __shared__ double etab[32];
     if (threadIdx.x < 32) etab[threadIdx.x] = et.t[threadIdx.x];
@@ -1311,6 +1317,9 @@ __global__ void __launch_bounds__(kCCThreads) k_cc_work(Stat s, Geo g, const dou
     const int nsub = nkb * nlc, nunits = (*count) * nsub, Nq = s.Nq;
     const int chunk = (Nq + nlc - 1) / nlc;
     const double kappa = s.debye, kex = s.k_ex, sg = s.sig_cc, c12 = 12.0 / sg, c6 = 6.0 / sg;
+    double c0 = ec.c[0];
+    asm volatile("" : "+v"(c0));
+    const int idx = wave_sum_index<10>(threadIdx.x & 63);
     for (int u = blockIdx.x * (kCCThreads / 64) + wv; u < nunits; u += gridDim.x * (kCCThreads / 64)) {
         const int pr = u / nsub, sub = u % nsub, kb = sub / nlc, lc = sub % nlc;
         const int k1 = list[2 * pr], k2 = list[2 * pr + 1];
@@ -1321,9 +1330,10 @@ __global__ void __launch_bounds__(kCCThreads) k_cc_work(Stat s, Geo g, const dou
         const double *pk = Qp + 4 * ((size_t)k1 * Nq + k);
         const double3 Qk = make_double3(pk[0], pk[1], pk[2]);
         const double keq = s.k_e * pk[3];
-        // Fk = sum_l f_l, f_l = g_l (Qk - Q_l)
-        double3 Fk = zero3();
-        double E = 0.0;
+        // Fk = sum_l f_l, f_l = g_l (Qk - Q_l): the Debye-Hueckel part over
+        // k_e q_k, the excluded volume apart, few pairs as it has
+        double3 Fk = zero3(), Fv = zero3();
+        double E = 0.0, Ev = 0.0;
         const double *pl = Qp + 4 * (size_t)k2 * Nq;
         for (int l = l0; l < l1; l++) {
             const double *d = pl + 4 * l;
@@ -1332,19 +1342,23 @@ __global__ void __launch_bounds__(kCCThreads) k_cc_work(Stat s, Geo g, const dou
             // with 1/d from a refined reciprocal square root
             const double r2s = dot(z, z);
             const double inv = rsqrt_f64(r2s);
-            const double dist = r2s * inv;
-            const double t = keq * d[3] * exp_neg_t(-kappa * dist, etab, ec);
+            const double t = d[3] * exp_neg_f(r2s * inv, c0, etab, ec);
             if (WITH_E) E += t * inv;
-            double g1d = t * (kappa + inv) * (inv * inv);  // (kappa d + 1) / d^3
+            const double g1d = t * (kappa + inv) * (inv * inv);  // (kappa d + 1) / d^3
             if (r2s <= kD8Sq) {  // the reference's d <= 8, exactly
                 const double x = sg * inv, x2 = x * x, x6 = x2 * x2 * x2, x7 = x6 * x, x13 = x6 * x7;
-                if (WITH_E) E += kex * (x6 * x6 - x6);
-                g1d += kex * (c12 * x13 - c6 * x7) * inv;
+                if (WITH_E) Ev += x6 * x6 - x6;
+                const double g = (c12 * x13 - c6 * x7) * inv;
+                Fv.x = __builtin_fma(g, z.x, Fv.x);
+                Fv.y = __builtin_fma(g, z.y, Fv.y);
+                Fv.z = __builtin_fma(g, z.z, Fv.z);
             }
             Fk.x = __builtin_fma(g1d, z.x, Fk.x);
             Fk.y = __builtin_fma(g1d, z.y, Fk.y);
             Fk.z = __builtin_fma(g1d, z.z, Fk.z);
         }
+        Fk = keq * Fk + kex * Fv;
+        E = keq * E + kex * Ev;
         Fk = act * Fk;
         const double3 a1 = ld3(g.a + 3 * b1), bb1 = ld3(g.b + 3 * b1), c1 = ld3(g.c + 3 * b1);
         const double3 T1 = torque_rel(Fk, ld3(s.cpos + 3 * k), a1, bb1, c1);
@@ -1352,15 +1366,9 @@ __global__ void __launch_bounds__(kCCThreads) k_cc_work(Stat s, Geo g, const dou
         // w = Qk - r2, z_l = Qk - Q_l: sum_l (w - z_l) x (-g_l z_l) = Fk x w,
         // since z_l x z_l = 0 -- the force sum alone gives it
         const double3 T2 = cross(Fk, Qk - ld3(g.r + 3 * s.core_bead[k2]));
-        double v[10] = {Fk.x, Fk.y, Fk.z, T1.x, T1.y, T1.z, T2.x, T2.y, T2.z, act * E};
-#pragma unroll
-        for (int q = 0; q < 10; q++)
-            for (int o = 32; o > 0; o >>= 1) v[q] += __shfl_down(v[q], o, 64);
-        if (lane == 0) {
-            double *slot = slots + 10 * ((size_t)(k1 * s.n_c + k2) * nsub + sub);
-#pragma unroll
-            for (int q = 0; q < 10; q++) slot[q] = v[q];
-        }
+        const double v[10] = {Fk.x, Fk.y, Fk.z, T1.x, T1.y, T1.z, T2.x, T2.y, T2.z, act * E};
+        const double mine = wave_sum_n(v);
+        if (idx >= 0) slots[10 * ((size_t)(k1 * s.n_c + k2) * nsub + sub) + idx] = mine;
     }
 }
 
@@ -1461,10 +1469,10 @@ void launch_forces(const Stat &s, const Geo &g, const Sites &st, const Frc &f, c
         M(K_CCWORK, 0);
         if (Epart)
             k_cc_work<true><<<w.cc_grid, kCCThreads, 0, qq>>>(s, g, st.Qp, w.cc_list, w.cc_count, w.cc_nkb,
-                                                              w.cc_nlc, w.cc_slots, kExpCoef6, kExp2Tab);
+                                                              w.cc_nlc, w.cc_slots, exp_coef_f(s.debye), kExp2Tab);
         else
             k_cc_work<false><<<w.cc_grid, kCCThreads, 0, qq>>>(s, g, st.Qp, w.cc_list, w.cc_count, w.cc_nkb,
-                                                               w.cc_nlc, w.cc_slots, kExpCoef6, kExp2Tab);
+                                                               w.cc_nlc, w.cc_slots, exp_coef_f(s.debye), kExp2Tab);
         M(K_CCWORK, 1);
     };
     auto mech = [&]() { M(K_MECH, 0); k_mech<<<nblk(s.n, 64), 64, 0, q>>>(s, g, f, E(off_mech), terms); M(K_MECH, 1); };

@@ -120,3 +120,43 @@ def test_squared_cutoffs_exact():
             assert np.array_equal(root < r, x < t), r
         else:
             assert np.array_equal(root <= r, x <= t), r
+
+
+PROG_F = r"""
+#include "bd_dev.h"
+#include <cmath>
+#include <cstdio>
+#include <random>
+int main(int, char **argv) {
+    const double kappa = atof(argv[1]), top = 60.0 / kappa;
+    const bd::ExpCoefF c = bd::exp_coef_f(kappa);
+    std::mt19937_64 gen(12345);
+    std::uniform_real_distribution<double> ud(0.0, top);
+    long double emax = -1;
+    for (int i = 0; i < 2000000; i++) {
+        // random points, and points at the edges of the reduction intervals
+        double d = (i % 4 == 3) ? (i / 4) * (0.69314718055994530942 / 64.0) / kappa : ud(gen);
+        if (d > top) d = ud(gen);
+        const long double x = (long double)kappa * d, ref = expl(-x);
+        const long double e = fabsl(((long double)bd::exp_neg_f(d, c.c[0], bd::kExp2Tab.t, c) - ref) / ref) - ldexpl(x, -53);
+        if (e > emax) emax = e;
+    }
+    printf("%.6Le\n", emax);
+    return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("kappa", [0.1, 1.04, 3.3])
+def test_exp_neg_f_accuracy(kappa, tmp_path):
+    """exp_neg_f, the core-core kernel's e^(-kappa d): off by the exponent's
+    rounding (2^-53 kappa d) and the few ulps of exp_neg_t at most."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    src, exe = tmp_path / "expf.cpp", tmp_path / "expf"
+    src.write_text(PROG_F)
+    r = subprocess.run([HIPCC, "-x", "hip", "--cuda-host-only", "-std=c++17", "-O2", "-I" + CSRC, str(src), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    out = subprocess.run([str(exe), str(kappa)], capture_output=True, text=True, check=True).stdout
+    assert float(out) <= 4e-16
