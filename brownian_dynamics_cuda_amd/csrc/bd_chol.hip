@@ -1919,10 +1919,11 @@ __global__ void __launch_bounds__(256) k_dmul(const double *xs, const double *ra
 #pragma unroll
             for (int k = 0; k < 3; k++) acc[k] += d * uj[k];
         } else {
-            double M[3][3];
-            rpy_block(ri, make_double3(xs[3 * j], xs[3 * j + 1], xs[3 * j + 2]), radi, rad_all[j], a1, a2, M);
-#pragma unroll
-            for (int k = 0; k < 3; k++) acc[k] += (M[k][0] * uj[0] + M[k][1] * uj[1]) + M[k][2] * uj[2];
+            const double3 u3 = rpy_apply(ri, make_double3(xs[3 * j], xs[3 * j + 1], xs[3 * j + 2]), radi, rad_all[j], a1, a2,
+                                         make_double3(uj[0], uj[1], uj[2]));
+            acc[0] += u3.x;
+            acc[1] += u3.y;
+            acc[2] += u3.z;
         }
     }
 #pragma unroll

@@ -98,37 +98,10 @@ __device__ __forceinline__ void rotate_bead(const Stat &s, const Geo &src, const
     }
 }
 
-// RPY 3x3 block between beads at ri and rj (func.cpp:752-799); rows are
-// the components of bead i.  Identical value for (j, i): only products of
-// pairs of components and squares of r_i - r_j enter.  The far-field
-// quotients by s and s^2 as products with one reciprocal of s.
-__device__ __forceinline__ void rpy_block(double3 ri, double3 rj, double radi, double radj, double a1,
-                                          double a2, double M[3][3]) {
-    double sij[3] = {ri.x - rj.x, ri.y - rj.y, ri.z - rj.z};
-    double ssq = sij[0] * sij[0] + sij[1] * sij[1] + sij[2] * sij[2];
-    double s = sqrt(ssq);
-    if (s >= radi + radj) {
-        const double is = 1.0 / s, iss = is * is;
-        const double f = (radi * radi + radj * radj) * iss;
-        const double f1 = 1.0 + f / 3, f2i = (1.0 - f) * iss;
-        const double pre = a2 * is;
-        for (int k = 0; k < 3; k++)
-            for (int l = 0; l < 3; l++)
-                M[k][l] = (k == l) ? pre * (f1 + f2i * sij[k] * sij[k]) : pre * (f2i * sij[k] * sij[l]);
-    } else {
-        double se = pow((radi * radi * radi + radj * radj * radj) / 2.0, 1.0 / 3);
-        double pre = a1 / se, sq = sqrt(ssq);
-        for (int k = 0; k < 3; k++)
-            for (int l = 0; l < 3; l++)
-                M[k][l] = (k == l) ? pre * (1.0 - 9.0 * sq / (32 * se) + 3.0 * sij[k] * sij[k] / (32.0 * se * sq))
-                                   : pre * (3.0 * sij[k] * sij[l] / (32.0 * se * sq));
-    }
-}
-
 // translation_cal (func_cuda.cu:650-679) without a stored tensor: the drift
 // del * D_blk * F of a bead is summed over the beads of its species block
-// (main / tail / LH) with the RPY blocks recomputed in closed form -- the
-// same entries a row of the stored D holds.  One workgroup per bead of
+// (main / tail / LH) with the RPY blocks applied in closed form -- the
+// blocks a row of the stored D holds.  One workgroup per bead of
 // the hydrodynamic set, threads over partners, fixed-order reduction; the
 // workgroups past n_hi take kTrThreads beads outside the set each
 // (self-mobility a1/rad only).
@@ -180,16 +153,11 @@ __global__ void __launch_bounds__(kTrThreads) k_translate(Stat s, int n_hi, int 
     const double3 ri = ld3(x0 + 3 * i);
     double v[3] = {0.0, 0.0, 0.0};
     for (int j = threadIdx.x; j < cnt; j += blockDim.x) {
-        const double Fj[3] = {fcomp(F, F2, 3 * j), fcomp(F, F2, 3 * j + 1), fcomp(F, F2, 3 * j + 2)};
-        if (j == i) {
-            const double dself = s.a1 / radi;
-            for (int k = 0; k < 3; k++) v[k] += s.del * dself * Fj[k];
-            continue;
-        }
-        double M[3][3];
-        rpy_block(ri, ld3(x0 + 3 * j), radi, rad_all[lo + j], s.a1, s.a2, M);
-        for (int k = 0; k < 3; k++)
-            for (int l = 0; l < 3; l++) v[k] += s.del * M[k][l] * Fj[l];
+        const double3 Fj = make_double3(fcomp(F, F2, 3 * j), fcomp(F, F2, 3 * j + 1), fcomp(F, F2, 3 * j + 2));
+        const double3 u = j == i ? (s.a1 / radi) * Fj : rpy_apply(ri, ld3(x0 + 3 * j), radi, rad_all[lo + j], s.a1, s.a2, Fj);
+        v[0] = __builtin_fma(s.del, u.x, v[0]);
+        v[1] = __builtin_fma(s.del, u.y, v[1]);
+        v[2] = __builtin_fma(s.del, u.z, v[2]);
     }
     block_sum_n<kTrThreads, 3>(v, red);
     if (threadIdx.x == 0)
