@@ -8,27 +8,26 @@
 // Matrix: row-major, lower triangle, padded to a multiple of 64 with an
 // identity block (so the padded factor is [[L,0],[0,I]] and no kernel needs
 // a bounds test).  Right-looking blocked algorithm with 64x64 tiles, one
-// launch per block column kb (k_step): every workgroup forms the two panel
+// launch per block column kb (k_step, k_step2): every workgroup forms the two panel
 // tiles it needs as A_ib,kb inv(L_kb,kb)^T (FP64 matrix cores), updates its
 // trailing tile A_ib,jb -= L_ib,kb L_jb,kb^T (FP64, FP32 or three-slice
 // BF16 matrix-core products), and the workgroup owning tile (kb+1,kb+1)
-// then factors it and inverts the factor (four wavefronts, FP64, the
-// inverse built beside the pivots).  The solved off-diagonal tile L_ib,kb
+// then factors it and inverts the factor (four wavefronts, FP64, one
+// elimination of the tile and the identity).  The solved off-diagonal tile L_ib,kb
 // stays parked in the upper block (kb, ib) of the same storage.
 //
 // Large matrices take super-panels of NB block columns instead: the panel
 // columns are factored as above with their updates restricted to the panel,
-// and the trailing matrix then receives the whole panel in one launch
-// (k_trail: each tile accumulates K = 64 NB in registers before its one
-// read-modify-write), so the trailing matrix streams through HBM once per
+// and the trailing matrix then receives the whole panel at once (each tile
+// accumulates K = 64 NB in registers before its one read-modify-write), so the trailing matrix streams through HBM once per
 // NB block columns rather than once per block column.  The panel tiles lie
 // once more in the operand order of the matrix cores for it (k_trail_pk; in
 // BF16 split into slices, k_trail_bf).  Panels of eight in FP64 and FP32
 // (chol_panels) factor only their diagonal block column by column, beside
 // tiles of the trailing update before it (k_block_step), and solve the rows
 // below in one launch (k_panel_rows).  In the FP32 and BF16 modes only the
-// trailing update takes
-// the reduced precision; the panel's own columns stay FP64.
+// trailing update takes the reduced precision; the panel's own columns stay
+// FP64.
 #include <algorithm>
 #include <type_traits>
 #include <utility>

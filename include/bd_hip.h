@@ -184,8 +184,8 @@ int bd_set_refine(bd_context *ctx, int enable);
 
 /* Schedule of the blocked factor (no counterpart in the reference, which
  * calls cusolverDnDpotrf, func_cuda.cu:3526-3529).  panel_tiles = 0 (the
- * default) chooses: super-panels of 8 block columns of 64 from 84 block
- * columns (D of 5313 rows) up, from 64 (4033 rows) in the FP32 and BF16
+ * default) chooses: super-panels of 8 block columns of 64 from 60 block
+ * columns (D of 3777 rows) up, from 64 (4033 rows) in the FP32 and BF16
  * modes, one block column per launch below; -1 always one block column per
  * launch; k >= 2 super-panels of k block columns
  * whenever the matrix has more than k.  In a super-panel the panel columns
@@ -206,10 +206,10 @@ int bd_get_chol_schedule(bd_context *ctx, int *panel_tiles_used);
  * and L may be the same buffer when ldd == ldl.  mode: BD_CHOL_*.  neg: host
  * int for the count of negative pivots (may be NULL).  stream: a hipStream_t
  * (NULL: the default stream); the call returns once the factor is done.
- * The workspace, (64 ceil(m/64))^2 + 4096 ceil(m/64) doubles and from 60
- * block columns about 1.4 % more, is allocated by the call.  One of at most 256
- * MiB per device is kept for the next call; calls that overlap have one each.
- * bd_cholesky_release frees what is kept. */
+ * The workspace, (64 n)^2 + 4096 n doubles for n = ceil(m/64) block columns and
+ * from 60 (64 in the reduced modes) 32768 n + 262144 more, is allocated by the
+ * call.  One of at most 256 MiB per device is kept for the next call; calls
+ * that overlap have one each.  bd_cholesky_release frees what is kept. */
 int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, int *neg,
                 void *stream);
 int bd_cholesky_release(void);
