@@ -1301,11 +1301,12 @@ constexpr int kCCThreads = 256;   // four wavefronts, a work unit each
 // Bound by the vector instructions of a pair of charges: 38 and a reciprocal
 // root, 44 before k_e q_k left the loop and exp took this form.  With that and
 // the slot's ten sums in 13 exchanges instead of 60 a force pass takes at 250
-// nucleosomes 559 us (633), at 600 1430 (1540).  Eight wavefronts per SIMD,
-// though a few values of the unit's set-up then go through scratch: six left
-// part of the grid for a second round.
+// nucleosomes 559 us (633), at 600 1430 (1540).  Eight wavefronts per SIMD
+// (six left part of the grid for a second round), with energies seven: their
+// sums would put three values of the unit's set-up into scratch, and a launch
+// with scratch cost 25 us more on a stream of single launches.
 template <bool WITH_E>
-__global__ void __launch_bounds__(kCCThreads, 8) k_cc_work(Stat s, Geo g, const double *__restrict__ Qp,
+__global__ void __launch_bounds__(kCCThreads, WITH_E ? 7 : 8) k_cc_work(Stat s, Geo g, const double *__restrict__ Qp,
                                                        const int *__restrict__ list, const int *__restrict__ count,
                                                        int nkb, int nlc, double *__restrict__ slots, ExpCoefF ec,
                                                        Exp2Tab et) {
