@@ -177,7 +177,18 @@ def main():
         mrows = n_hi3 - 64 * (k0 + nb)
         trail_fl.append(64.0 * nb * mrows * (mrows + 1))
         k0 += nb
-    if dominant in ("chol_step", "potrf"):
+    # FP64 and FP32 super-panels of eight run tiles of the trailing update
+    # beside their block columns: the factor is priced as a whole
+    whole = nb == 8 and args.chol != "bf16" and dominant in ("chol_step", "chol_trail")
+    if whole:
+        per_launch = chol_flops(n_hi3)
+        avg_s = (per_step["chol_step"] + per_step["chol_trail"]) / 1e3
+        peak, pipe = {"fp64": (PEAK_FP64, "FP64 MFMA"),
+                      "fp32": (PEAK_FP32_MFMA, "FP32 MFMA, panels FP64")}[args.chol]
+        roof = dict(bound="mfma", achieved=per_launch / avg_s / 1e12, peak=peak / 1e12,
+                    unit="TFLOP/s", kernel="chol_step + chol_trail", pipe=pipe,
+                    flop_per_launch=per_launch, avg_launch_us=avg_s * 1e6, panel_tiles=nb)
+    elif dominant in ("chol_step", "potrf"):
         # the factorisation's algorithmic FLOPs less the trailing updates',
         # spread over the block-column launches (one per 64 columns after
         # the first); with super-panels these are the FP64 panel columns
@@ -210,7 +221,7 @@ def main():
     # takes its traffic only from an explicit --traffic-file
     tfile = args.traffic_file or (os.path.join(ROOT, "profiles", f"hbm_traffic_cfg{cfg}.txt")
                                   if args.chol == "fp64" else None)
-    roof["traffic"] = read_traffic(tfile, dominant) if tfile else None
+    roof["traffic"] = read_traffic(tfile, dominant) if tfile and not whole else None
 
     # end to end: the host draws each batch's noise (MT19937 + polar normals,
     # main.cpp:479-486) on a thread while the GPU runs the previous batch
