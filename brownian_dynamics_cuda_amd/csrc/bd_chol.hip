@@ -972,6 +972,7 @@ __device__ __forceinline__ void step_tile(double *S, double *A, int ld, int kb, 
     trap_index(lb, jcols, ii, jj);
     const int ib = kb + 1 + ii, jb = kb + 1 + jj;
     const bool diag = ib == jb;
+    // ahead of force kernels on its CU (100 nucleosomes 864 us a step, 875 without)
     if (lb == 0) __builtin_amdgcn_s_setprio(3);
     dbl2 vi[PERT], vj[PERT];
     {
