@@ -95,8 +95,8 @@ __device__ __forceinline__ void tri_index(int idx, int &i, int &j) {
     j = idx - r * (r + 1) / 2;
 }
 
-constexpr int kDiagLds = 5376;  // LDS of diag_factor_inv, doubles
-__device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, double *A, int ld, int d0, double *Linv,
+constexpr int kDiagLds = 5408;  // LDS of diag_factor_inv, doubles
+__device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *A, int ld, int d0, double *Linv,
                                                 int *neg);
 
 // FACTOR: workgroup 0 (tile (0,0)) then factors and inverts its tile in
@@ -596,7 +596,10 @@ struct DiagLds {
     __device__ __forceinline__ double *next(int q) const { return base + 4096 + 288 * q; }
     __device__ __forceinline__ double *R() const { return base + 5248; }  // 1/|f|, 64
     __device__ __forceinline__ double *S() const { return base + 5312; }  // 1/sqrt(|f|), 64
+    // exponents the rows are scaled by (rescale_tile), 64; the tile does not reach here
+    __device__ __forceinline__ int *K() const { return reinterpret_cast<int *>(base + 5376); }
 };
+static_assert(TB * LDP <= 5376, "tile and exponents");
 constexpr int kNextPitch = 18;
 
 // the operand register of a panel: lane (k, c) holds row k, column c
@@ -757,21 +760,72 @@ __device__ __forceinline__ void below_row(dbl4 (&Z)[6], const DiagLds &l) {
     if constexpr (B < 2) below_panel<B, U, B + 2, 3>(Z, l, 3);
 }
 
+// The elimination divides by |f| and forms inv(L) from rows over |f|, which
+// overflow where a pivot is below 2^-1024, though its root and 1/sqrt(|f|) do
+// not.  A tile with diagonal entries outside [2^-960, 2^960] is therefore
+// factored as S C S with S = 2^-k, k half the exponent of a row's diagonal
+// entry, and L = inv(S) L', inv(L) = inv(L') S on its way out: the scaling is
+// exact.  Inside the bounds the pivots keep clear of 2^-1022 (cancellation
+// takes 53 bits at most) and nothing is scaled.  The test is one LDS read and
+// one comparison beside the tile's own reads.
+__device__ __forceinline__ bool tile_out_of_range(const double *T) {
+    const double d = fabs(T[(tid() & 63) * (LDP + 1)]);
+    return __builtin_expect(__ballot(!(d >= 0x1p-960 && d <= 0x1p+960)) != 0, false);
+}
+// By all four wavefronts, once they have read T; they read it again after it.
+__device__ __forceinline__ void rescale_tile(const DiagLds &l, double *T) {
+    __syncthreads();
+    if (tid() < TB) {
+        const double d = fabs(T[tid() * (LDP + 1)]);
+        // zero, infinity and NaN have the exponent 0
+        l.K()[tid()] = d >= 0x1p-960 && d <= 0x1p+960 ? 0 : __builtin_amdgcn_frexp_exp(d) / 2;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int e = tid(); e < TB * TB; e += NTHR) {
+        const int r = e / TB, c = e % TB;
+        if (c <= r) T[r * LDP + c] = __builtin_ldexp(T[r * LDP + c], -l.K()[r] - l.K()[c]);
+    }
+    __syncthreads();
+}
+__device__ __forceinline__ void unscale_tile(const DiagLds &l, double *A, int ld, int d0, double *Linv) {
+    __syncthreads();
+#pragma unroll 1
+    for (int e = tid(); e < TB * TB; e += NTHR) {
+        const int r = e / TB, c = e % TB;
+        if (c > r) continue;
+        double *a = A + (size_t)(d0 + r) * ld + d0 + c, *i = Linv + r * TB + c;
+        *a = __builtin_ldexp(*a, l.K()[r]);
+        *i = __builtin_ldexp(*i, -l.K()[c]);
+    }
+}
+
 // Called by all four wavefronts.  lds: kDiagLds doubles; T, LDS that may
-// overlap it, holds the tile (pitch LDP) at (d0, d0), of which the lower
-// triangle is read.  L goes
+// overlap its first 5376 doubles, holds the tile (pitch LDP) at (d0, d0), of
+// which the lower triangle is read.  L goes
 // to A (lower triangle), inv(L), row-major 64x64 with zeros above its
 // diagonal, to Linv.
-__device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, double *A, int ld, int d0, double *Linv,
+__device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *A, int ld, int d0, double *Linv,
                                                 int *neg) {
     const int lane = tid() & 63, wv = __builtin_amdgcn_readfirstlane(tid() >> 6);
     const int g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
     const DiagLds l = {lds};
+    bool scaled;
+    auto read_tile = [&](auto read) {
+        read();
+        scaled = tile_out_of_range(T);
+        if (scaled) {
+            rescale_tile(l, T);
+            read();
+        }
+        __syncthreads();
+    };
     if (wv == 0) {
         double w[16], r[16];
+        read_tile([&]() {
 #pragma unroll
-        for (int k = 0; k < 16; k++) w[k] = T[max(k, ci) * LDP + min(k, ci)];
-        __syncthreads();
+            for (int k = 0; k < 16; k++) w[k] = T[max(k, ci) * LDP + min(k, ci)];
+        });
 #pragma unroll 1
         for (int b = 0; b < 4; b++) {
             if (b) load_rows(w, l.next(3) + kNextPitch * c);
@@ -790,9 +844,10 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, do
         }
     } else if (wv == 1) {
         double x[16];
+        read_tile([&]() {
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = g < 3 ? T[(16 * (g + 1) + ci) * LDP + k] : k == ci ? 1.0 : 0.0;
-        __syncthreads();
+            for (int k = 0; k < 16; k++) x[k] = g < 3 ? T[(16 * (g + 1) + ci) * LDP + k] : k == ci ? 1.0 : 0.0;
+        });
 #pragma unroll 1
         for (int b = 0; b < 4; b++) {
             if (b) {
@@ -818,15 +873,21 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, do
             o[0] = o[1] = dbl2{0.0, 0.0};
         }
         if (wv == 2) {
-            dbl4 Z[6] = {tile_block(T, 1, 1), tile_block(T, 1, 2), tile_block(T, 2, 2), tile_block(T, 2, 3),
-                         tile_block(T, 3, 3), z};
-            __syncthreads();
+            dbl4 Z[6];
+            read_tile([&]() {
+                Z[0] = tile_block(T, 1, 1);
+                Z[1] = tile_block(T, 1, 2);
+                Z[2] = tile_block(T, 2, 2);
+                Z[3] = tile_block(T, 2, 3);
+                Z[4] = tile_block(T, 3, 3);
+                Z[5] = z;
+            });
             below_row<0, 0>(Z, l);
             below_row<1, 0>(Z, l);
             below_row<2, 0>(Z, l);
         } else {
-            dbl4 Z[6] = {tile_block(T, 1, 3), z, z, z, z, z};
-            __syncthreads();
+            dbl4 Z[6] = {z, z, z, z, z, z};
+            read_tile([&]() { Z[0] = tile_block(T, 1, 3); });
             below_row<0, 1>(Z, l);
             below_row<1, 1>(Z, l);
             below_row<2, 1>(Z, l);
@@ -841,6 +902,7 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, const double *T, do
     }
     store_block(l, 3, wv, A, ld, d0, Linv);
     if (wv == 0) store_block(l, 3, 4, A, ld, d0, Linv);
+    if (scaled) unscale_tile(l, A, ld, d0, Linv);
 }
 
 // a tile between global memory, registers and LDS (pitch LDP), 16-byte

@@ -70,6 +70,22 @@ def test_blocks_of_the_diagonal_tile(m):
         assert np.array_equal(Ls, np.ldexp(Lg, k // 2))
 
 
+@pytest.mark.parametrize("m", [3, 17, 64, 130])
+@pytest.mark.parametrize("scale", [(-530,), (505,), (0, -530), (-530, 505, 0)])
+def test_pivots_outside_the_normal_range(m, scale):
+    """Pivots whose reciprocal is no FP64 number (below 2^-1024) or a subnormal
+    one, alone and beside others: D = S T T^T S with T of small whole numbers
+    and S powers of two, exact in FP64, has the factor S T.  T's diagonal of 16
+    outweighs its other entries, so the factor is well conditioned."""
+    g = np.random.default_rng(m)
+    T = np.tril(g.integers(-1, 2, (m, m)) * (g.random((m, m)) < 4.0 / m), -1) + 16.0 * np.eye(m)
+    k = np.resize(scale, m)
+    D = np.ldexp(T @ T.T, k[:, None] + k[None, :])
+    L, neg = E.cholesky_device(D)
+    assert neg == 0
+    assert rel_err(np.ldexp(L, -k[:, None]), T) <= 1e-12
+
+
 @pytest.mark.parametrize("m,mode", [(5312, E.CHOL_FP64), (5313, E.CHOL_FP64), (4033, E.CHOL_FP32), (4033, E.CHOL_BF16)])
 def test_ends_of_the_super_panels(m, mode):
     """The first sizes with super-panels (84 and 64 block columns) and the last
