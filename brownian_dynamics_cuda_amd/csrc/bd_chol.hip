@@ -64,9 +64,9 @@ __device__ __forceinline__ double3 hi_pos(const Stat &s, const Geo &g, int b) {
 __device__ __forceinline__ void rpy_block(double3 ri, double3 rj, double radi, double radj, double a1, double a2,
                                           double (&M)[3][3]) {
     const double sij[3] = {ri.x - rj.x, ri.y - rj.y, ri.z - rj.z};
-    const double ssq = sij[0] * sij[0] + sij[1] * sij[1] + sij[2] * sij[2];
+    const double ssq = rpy_ssq(ri - rj);
     const double s = sqrt(ssq);
-    if (s >= radi + radj) {
+    if (rpy_far(ssq, radi + radj)) {
         const double f = (radi * radi + radj * radj) / ssq;
         const double f1 = 1.0 + f / 3, f2 = 1.0 - f, c = a2 / s;
 #pragma unroll

@@ -427,6 +427,21 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
     return t;  // valid on thread 0
 }
 
+// |z|^2 of the RPY tensor in one fixed order, and its near/far test: the
+// reference's s >= r_i + r_j on s = sqrt(ssq) (func.cpp:754-796).  The assembly
+// of D and the products with it take the same branch by these two, also within
+// rounding of touching beads, where the branches of unequal radii do not meet.
+// Away from the threshold ssq against reach^2 gives what the root gives: below
+// reach^2 (1 - 2^-50) the root is more than half an ulp below reach.
+__host__ __device__ __forceinline__ double rpy_ssq(double3 z) {
+    return __builtin_fma(z.z, z.z, __builtin_fma(z.y, z.y, z.x * z.x));
+}
+__host__ __device__ __forceinline__ bool rpy_far(double ssq, double reach) {
+    const double r2 = reach * reach;
+    if (fabs(ssq - r2) > 0x1p-50 * r2) return ssq > r2;
+    return sqrt(ssq) >= reach;
+}
+
 // M F for the RPY 3x3 block M between beads at ri and rj (func.cpp:752-799)
 // without its entries: both branches are alpha I + beta z z^T, z = ri - rj, so
 // M F = alpha F + beta (z . F) z, with 1/s from a refined reciprocal square
@@ -436,10 +451,10 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
 __device__ __forceinline__ double3 rpy_apply(double3 ri, double3 rj, double radi, double radj, double a1, double a2,
                                              double3 F) {
     const double3 z = ri - rj;
-    const double ssq = dot(z, z), zF = dot(z, F), reach = radi + radj;
+    const double ssq = rpy_ssq(z), zF = dot(z, F);
     const double is = rsqrt_f64(ssq);
     double alpha, beta;
-    if (ssq >= reach * reach) {
+    if (rpy_far(ssq, radi + radj)) {
         const double iss = is * is, f = (radi * radi + radj * radj) * iss, pre = a2 * is;
         alpha = pre * __builtin_fma(f, 1.0 / 3.0, 1.0);
         beta = pre * ((1.0 - f) * iss);

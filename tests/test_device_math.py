@@ -160,3 +160,53 @@ def test_exp_neg_f_accuracy(kappa, tmp_path):
     assert r.returncode == 0, r.stderr[-2000:]
     out = subprocess.run([str(exe), str(kappa)], capture_output=True, text=True, check=True).stdout
     assert float(out) <= 4e-16
+
+
+PROG_R = r"""
+#include "bd_dev.h"
+#include <cstdio>
+#include <random>
+int main() {
+    std::mt19937_64 gen(7);
+    std::uniform_real_distribution<double> ur(0.1, 12.0);
+    const double radii[] = {5.0, 1.5, 1.2, 0.9, 0.6, 0.7};
+    long wrong = 0, near = 0, squares = 0;
+    for (int i = 0; i < 20000; i++) {
+        const double reach = i < 36 ? radii[i / 6] + radii[i % 6] : ur(gen) + ur(gen);
+        // the squared distances within 40 doubles of the threshold, and far ones
+        double x = reach * reach;
+        for (int k = 0; k < 40; k++) x = nextafter(x, 0.0);
+        for (int k = 0; k <= 80; k++, x = nextafter(x, 1e300)) {
+            const bool far = sqrt(x) >= reach;
+            wrong += bd::rpy_far(x, reach) != far;
+            near += !far;
+            squares += (x >= reach * reach) != far;
+        }
+        for (double f : {0.0, 0x1p-1070, 0.3, 1.0 - 0x1p-49, 1.0 + 0x1p-49, 3.0, 1e200, HUGE_VAL})
+            wrong += bd::rpy_far(f * reach * reach, reach) != (sqrt(f * reach * reach) >= reach);
+        wrong += bd::rpy_far(NAN, reach);
+    }
+    printf("%ld %ld %ld\n", wrong, near, squares);
+    return 0;
+}
+"""
+
+
+def test_rpy_branch_of_products_and_assembly(tmp_path):
+    """rpy_far, by which the assembly of the RPY tensor and the products with it
+    choose their branch, is the reference's s >= r_i + r_j (func.cpp:754-796) on
+    every double around the threshold, where a test of squares is not; both
+    form s^2 by the same function."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    src, exe = tmp_path / "far.cpp", tmp_path / "far"
+    src.write_text("#include <cmath>\n" + PROG_R)
+    r = subprocess.run([HIPCC, "-x", "hip", "--cuda-host-only", "-std=c++17", "-O2", "-I" + CSRC, str(src), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    wrong, near, squares = map(int, subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split())
+    assert wrong == 0
+    assert near > 0 and squares > 0  # the sample reaches both branches and doubles where squares differ
+    for f in ("bd_dev.h", "bd_chol.hip"):
+        text = open(os.path.join(CSRC, f)).read()
+        assert "rpy_far(ssq, radi + radj)" in text and "ssq = rpy_ssq(" in text, f
