@@ -207,7 +207,8 @@ __host__ __device__ __forceinline__ double exp_neg_t(double x, const double *tab
     return __builtin_ldexp(tab[im & 31] * p, im >> 5);
 }
 // e^(-kappa d) in the same form from y = k d, k = -kappa 32/ln2: m = rint(y)
-// comes out of the low bits of y + 1.5 2^52, f = y - m is exact, and the series
+// comes out of the low bits of y + 1.5 2^52 (as an int: right for |y| < 2^31,
+// kappa d < 4.6e7), f = y - m is exact, and the series
 // of e^(f ln2/32) takes the powers of ln2/32 into its coefficients: no reduction
 // in two parts and no rounding and converting instructions.  The one rounding
 // of k moves the exponent by at most 2^-53 of itself, as that of the product
@@ -217,7 +218,10 @@ struct ExpCoefF {
     double c[6];  // (ln2/32)^i / i!, i = 6 .. 1
     double k;
 };
+// Above 2^20 kappa counts as 2^20, for which every d up to 44 nm keeps in range
+// (charges of cores within 25 nm); e^(-kappa d) is 0 for both from 0.00072 nm.
 inline ExpCoefF exp_coef_f(double kappa) {
+    if (kappa > 0x1p20) kappa = 0x1p20;
     const long double q = 0.693147180559945309417232121458176568L / 32.0L;
     ExpCoefF e;
     long double p = 1.0L, n = 1.0L;

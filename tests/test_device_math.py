@@ -210,3 +210,46 @@ def test_rpy_branch_of_products_and_assembly(tmp_path):
     for f in ("bd_dev.h", "bd_chol.hip"):
         text = open(os.path.join(CSRC, f)).read()
         assert "rpy_far(ssq, radi + radj)" in text and "ssq = rpy_ssq(" in text, f
+
+
+PROG_X = r"""
+#include "bd_dev.h"
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+int main(int, char **argv) {
+    const double kappa = atof(argv[1]);
+    const bd::ExpCoefF c = bd::exp_coef_f(kappa);
+    long wrong = 0, zero = 0;
+    // distances of charges from 0.001 to 44 nm
+    for (int i = 0; i <= 200000; i++) {
+        const double d = 0.001 * pow(44000.0, i / 200000.0);
+        const long double ref = expl(-(long double)kappa * d);
+        const double e = bd::exp_neg_f(d, c.c[0], bd::kExp2Tab.t, c);
+        // relative while normal, then to the spacing of the subnormals; the
+        // exponent's own rounding is 2^-53 kappa d
+        const long double tol = ref * (4e-16L + ldexpl(kappa * d, -53)) + 0x1p-1074L;
+        wrong += !(fabsl((long double)e - ref) <= tol);
+        zero += e == 0.0;
+    }
+    printf("%ld %ld\n", wrong, zero);
+    return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("kappa", [0.0, 0.7, 30.0, 800.0, 1e5, 1048576.0, 2e6, 1e9, 1e300])
+def test_exp_neg_f_past_underflow(kappa, tmp_path):
+    """exp_neg_f for every screening length and charge distance: through the
+    subnormal results to 0, and 0 where 32/ln2 kappa d leaves the int its low
+    bits are taken as (kappa d > 4.6e7)."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
+    src, exe = tmp_path / "expx.cpp", tmp_path / "expx"
+    src.write_text(PROG_X)
+    r = subprocess.run([HIPCC, "-x", "hip", "--cuda-host-only", "-std=c++17", "-O2", "-I" + CSRC, str(src), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    wrong, zero = map(int, subprocess.run([str(exe), str(kappa)], capture_output=True, text=True, check=True).stdout.split())
+    assert wrong == 0
+    assert (zero > 0) == (kappa * 44.0 > 746.0)
