@@ -115,14 +115,26 @@ constexpr int kMaxDevices = 64;
 // it, so calls that overlap (threads, streams) never share one, and at most one
 // workspace of at most kKeepBytes stays per device.  It is given back by
 // bd_cholesky_release, by a call that needs a larger one and when an allocation
-// of the library fails.
+// of the library fails.  A device reset takes every allocation with it, and the
+// addresses may belong to another one by the next call: a kept workspace is used
+// or freed only if its address still holds the allocation it was kept as (by the
+// number the runtime gives each; 0.3 us).
 constexpr size_t kKeepBytes = (size_t)256 << 20;
 struct Workspace {
     void *ptr;
     size_t bytes;
+    unsigned long long id;
 };
 std::mutex g_kept_mu;
 Workspace g_kept[kMaxDevices] = {};
+
+// the runtime's number of the allocation at p, 0 where there is none
+unsigned long long allocation_id(void *p) {
+    unsigned long long id = 0;
+    if (p && hipPointerGetAttribute(&id, HIP_POINTER_ATTRIBUTE_BUFFER_ID, p) == hipSuccess) return id;
+    if (p) (void)hipGetLastError();
+    return 0;
+}
 
 Workspace exchange_kept(int dev, Workspace w) {
     if (dev < 0 || dev >= kMaxDevices) return w;
@@ -131,19 +143,30 @@ Workspace exchange_kept(int dev, Workspace w) {
     return w;
 }
 
+// the kept workspace out of its place, none if it is gone
+Workspace take_kept(int dev) {
+    const Workspace w = exchange_kept(dev, {});
+    return w.ptr && allocation_id(w.ptr) == w.id ? w : Workspace{};
+}
+
 // at least bytes on the current device dev: the kept workspace if it is large
 // enough, else a new one in its place
 hipError_t take_workspace(int dev, size_t bytes, Workspace *w) {
-    *w = exchange_kept(dev, {});
+    *w = take_kept(dev);
     if (w->bytes >= bytes) return hipSuccess;
     if (w->ptr) (void)hipFree(w->ptr);
-    *w = {nullptr, bytes};
+    *w = {nullptr, bytes, 0};
     const hipError_t e = hipMalloc(&w->ptr, bytes);
     if (e != hipSuccess) *w = {};
+    else w->id = allocation_id(w->ptr);
     return e;
 }
 hipError_t give_workspace(int dev, Workspace w, bool keep) {
-    if (keep && w.bytes <= kKeepBytes) w = exchange_kept(dev, w);
+    if (keep && w.id && w.bytes <= kKeepBytes) {
+        w = exchange_kept(dev, w);
+        // another call's, put back meanwhile
+        if (w.ptr && allocation_id(w.ptr) != w.id) return hipSuccess;
+    }
     return w.ptr ? hipFree(w.ptr) : hipSuccess;
 }
 
@@ -182,7 +205,7 @@ int scratch_of_current_device(double **out) {
 bool bd::release_workspaces() {
     bool any = false;
     for (int dev = 0; dev < kMaxDevices; dev++) {
-        const Workspace w = exchange_kept(dev, {});
+        const Workspace w = take_kept(dev);
         if (!w.ptr) continue;
         any = true;
         (void)hipFree(w.ptr);
