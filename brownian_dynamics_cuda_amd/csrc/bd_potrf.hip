@@ -219,6 +219,11 @@ int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, i
     int r = check_args(m, D, ldd, L, ldl, mode);
     if (r) return r;
     hipStream_t q = static_cast<hipStream_t>(stream);
+    // under capture nothing may be allocated, freed or waited for: refused here,
+    // before launches are on the stream and a workspace is out of its place
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    POTRF_CHK(hipStreamIsCapturing(q, &capture));
+    if (capture != hipStreamCaptureStatusNone) return fail(BD_E_HIP, "bd_cholesky: the stream is being captured");
     int dev = 0;
     POTRF_CHK(hipGetDevice(&dev));
     Workspace ws{};

@@ -209,7 +209,10 @@ int bd_get_chol_schedule(bd_context *ctx, int *panel_tiles_used);
  * The workspace, (64 n)^2 + 4096 n doubles for n = ceil(m/64) block columns and
  * from 60 (64 in the reduced modes) 32768 n + 262144 more, is allocated by the
  * call.  One of at most 256 MiB per device is kept for the next call; calls
- * that overlap have one each.  bd_cholesky_release frees what is kept. */
+ * that overlap have one each.  bd_cholesky_release frees what is kept (this
+ * library's own allocations do so where memory runs out; another library's
+ * cannot); one that a hipDeviceReset took is forgotten.  A stream under capture
+ * is refused (BD_E_HIP) with nothing put on it. */
 int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, int *neg,
                 void *stream);
 int bd_cholesky_release(void);

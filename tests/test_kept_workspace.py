@@ -31,11 +31,13 @@ size_t room = (size_t)1 << 40;  // largest allocation that succeeds
 bool library = true;            // who allocates
 hipError_t last = hipSuccess;
 hipError_t err(hipError_t e) { if (e != hipSuccess) last = e; return e; }
+hipStream_t capturing = nullptr;  // the stream under capture: no allocation, no wait meanwhile
 int launches = 0, dead_used = 0, foreign_used = 0, foreign_freed = 0, dead_freed = 0;
 }  // namespace
 
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) {
+    if (capturing) return err(hipErrorStreamCaptureUnsupported);
     if (n > room) return err(hipErrorOutOfMemory);
     size_t at = 4096;
     for (auto &r : live) {
@@ -47,6 +49,7 @@ hipError_t hipMalloc(void **p, size_t n) {
     return hipSuccess;
 }
 hipError_t hipFree(void *p) {
+    if (capturing) return err(hipErrorStreamCaptureUnsupported);
     auto it = live.find((size_t)p);
     if (it == live.end()) { dead_freed++; return err(hipErrorInvalidValue); }
     if (!it->second.ours) foreign_freed++;
@@ -67,7 +70,11 @@ hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 256; 
 hipError_t hipGetLastError() { hipError_t e = last; last = hipSuccess; return e; }
 const char *hipGetErrorString(hipError_t) { return "error"; }
 hipError_t hipMemcpyAsync(void *d, const void *, size_t n, hipMemcpyKind, hipStream_t) { memset(d, 0, n); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return capturing ? err(hipErrorStreamCaptureUnsupported) : hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t q, hipStreamCaptureStatus *s) {
+    *s = capturing && q == capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 hipError_t hipGetSymbolAddress(void **p, const void *s) { *p = (void *)s; return hipSuccess; }
 void **__hipRegisterFatBinary(const void *) { static void *h; return &h; }
 void __hipUnregisterFatBinary(void **) {}
@@ -132,6 +139,21 @@ SCENES = {
     CHECK(last == hipSuccess || hipGetLastError() == hipErrorOutOfMemory);
     room = (size_t)1 << 40;
     CHECK(factor(3969) == BD_OK);
+    SOUND();
+""",
+    "stream under capture": r"""
+    capturing = (hipStream_t)4096;
+    CHECK(factor(700, capturing) == BD_E_HIP && launches == 0 && live.empty());
+    capturing = nullptr;
+    (void)hipGetLastError();
+    CHECK(factor(700) == BD_OK && live.size() == 1);
+    launches = 0;
+    capturing = (hipStream_t)4096;
+    CHECK(factor(700, capturing) == BD_E_HIP);
+    CHECK(launches == 0);           // refused before anything is on the stream
+    capturing = nullptr;
+    CHECK(live.size() == 1);
+    CHECK(bd_cholesky_release() == BD_OK && live.empty());   // and nothing lost
     SOUND();
 """,
     "device reset": r"""
