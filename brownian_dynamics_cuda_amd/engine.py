@@ -448,6 +448,12 @@ def cholesky_device(D: np.ndarray, mode: int = CHOL_FP64, entry: str = "bd_chole
     return L, neg.value
 
 
+def release_cholesky_workspace():
+    """Free the workspaces bd_cholesky keeps for its next call (at most 256 MiB
+    per device), e.g. ahead of large allocations of another library."""
+    _check(load_library().bd_cholesky_release(), "bd_cholesky_release")
+
+
 class HostRng:
     """Host noise of the step (bd_rng_* in libbdhip.so)."""
 

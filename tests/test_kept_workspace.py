@@ -209,3 +209,10 @@ def test_workspace(scene, potrf):
     assert r.returncode == 0, r.stderr[-3000:]
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.stdout.strip() == "ok", out.stdout + out.stderr
+
+
+def test_release_from_python():
+    """The user's call that gives the kept workspaces back; without a GPU there
+    are none, and it is no error."""
+    from brownian_dynamics_cuda_amd import engine as E
+    assert E.release_cholesky_workspace() is None
