@@ -137,6 +137,86 @@ def test_core_core_blocks(n_c, nq):
     assert rel_err(e.cpu().numpy(), outs["dense"][1]) <= 1e-12
 
 
+@pytest.mark.parametrize("n_c,nq", [(999, 5), (1000, 5), (499, 65), (500, 65), (199, 300), (200, 300)])
+def test_core_core_block_sizes(n_c, nq):
+    """Both sides of the line between blocks of 16 and of 64 charges (1000
+    blocks of 64), forward with a work buffer and adjoint with the gradient of
+    every site's charge; one core with more partner charges than the records
+    held at a time, cores with one partner and cores with none.  Against the
+    dense sums in FP64, and FP32 against FP64 on the same inputs: a pair's
+    terms are off by up to 100 units (18 screening lengths, a 13th power),
+    their sum by one for each of the 100 records a slot adds.  The terms step
+    at 8 nm: sites with a pair within rounding of it have two right answers in
+    FP32 and are left to the FP64 comparison."""
+    import ctypes as C
+    g = torch.Generator().manual_seed(n_c + nq)
+    dev = torch.device("cuda")
+    # cores on a lattice, the nearest to core 0 first
+    k = 6 if n_c > 300 else 4
+    x = torch.cartesian_prod(*[torch.arange(-k, k + 1, dtype=torch.float64)] * 3)
+    r = 8.0 * x[torch.argsort((x * x).sum(1), stable=True)][:n_c]
+    Q = (r[:, None] + 3.0 * torch.rand(n_c, nq, 3, generator=g, dtype=torch.float64)).float()
+    q = (0.2 + 0.8 * torch.rand(nq, generator=g, dtype=torch.float64)).float()
+    gf = torch.randn(Q.shape, generator=g, dtype=torch.float64).float()
+    ge = torch.randn(n_c, generator=g, dtype=torch.float64).float()
+    hub = 1100 // nq + 1
+    pairs = {(0, j) for j in range(1, hub + 1)}
+    for i in range(n_c - 12, n_c):
+        d = (r - r[i]).norm(dim=1)
+        d[i] = np.inf
+        pairs.add(tuple(sorted((i, int(d.argmin())))))
+    nb = [[] for _ in range(n_c)]
+    for i, j in sorted(pairs):
+        nb[i].append(j)
+        nb[j].append(i)
+    assert len(nb[0]) * nq > 1024 and min(map(len, nb)) == 0
+    off = torch.tensor(np.r_[0, np.cumsum([len(v) for v in nb])], dtype=torch.int32, device=dev)
+    nbr = torch.tensor([v for w in nb for v in sorted(w)], dtype=torch.int32, device=dev)
+    consts = (0.7, 1.2, 0.03, 1.8)
+    ke, kap, kex, sig = consts
+    lib = E.load_library()
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def kernels(dt):
+        a = [t.to(dev, dt).contiguous() for t in (Q, q, gf, ge)]
+        f, gQ = torch.empty_like(a[0]), torch.empty_like(a[0])
+        e, gq = torch.empty_like(a[3]), torch.empty(n_c, nq, dtype=dt, device=dev)
+        work = torch.full((n_c, (nq + 15) // 16), float("nan"), dtype=dt, device=dev)
+        geo = [int(dt == torch.float64), n_c, nq, a[0].data_ptr(), a[1].data_ptr(), off.data_ptr(), nbr.data_ptr()]
+        assert lib.bd_cc_forward_work(*geo, *consts, f.data_ptr(), e.data_ptr(), work.data_ptr(), stream) == 0
+        assert lib.bd_cc_backward(*geo, *consts, a[2].data_ptr(), a[3].data_ptr(), gQ.data_ptr(), gq.data_ptr(), stream) == 0
+        torch.cuda.synchronize()
+        return [t.double().cpu().numpy() for t in (f, e, gQ, gq)]
+
+    def dense():
+        P = Q.to(dev, torch.float64).requires_grad_(True)
+        s = q.to(dev, torch.float64).repeat(n_c, 1).requires_grad_(True)
+        f, e = torch.zeros_like(P), torch.zeros(n_c, dtype=torch.float64, device=dev)
+        edge = torch.zeros(n_c, nq, dtype=torch.bool, device=dev)
+        for part in torch.tensor(sorted(pairs), device=dev).split(max(1, 1000000 // nq ** 2)):
+            i, j = part[:, 0], part[:, 1]
+            z = P[i][:, :, None] - P[j][:, None]
+            d = z.norm(dim=-1)
+            p, a, b = (((d * d - 64.0).abs() <= 64.0 * 2.0 ** -20)).nonzero(as_tuple=True)
+            edge[i[p], a] = True
+            edge[j[p], b] = True
+            dh = ke * s[i][:, :, None] * s[j][:, None] * torch.exp(-kap * d)
+            w = (sig / d) ** 6 * (d <= 8.0)
+            fz = ((dh * (kap * d + 1) / d + kex * (12 * w * w - 6 * w)) / (d * d))[..., None] * z
+            en = 0.5 * (dh / d + kex * (w * w - w)).sum((1, 2))
+            f = f.index_add(0, i, fz.sum(2)).index_add(0, j, -fz.sum(1))
+            e = e.index_add(0, i, en).index_add(0, j, en)
+        gQ, gs = torch.autograd.grad((f, e), (P, s), (gf.to(dev, torch.float64), ge.to(dev, torch.float64)))
+        return [t.detach().cpu().numpy() for t in (f, e, gQ, gs)], (~edge).cpu().numpy()
+
+    (ref, inner), k64, k32 = dense(), kernels(torch.float64), kernels(torch.float32)
+    for name, a, b, c in zip("f e gQ gq".split(), ref, k64, k32):
+        assert rel_err(b, a) <= 1e-12, name
+        keep = inner.all(1) if name == "e" else inner
+        assert keep.sum() > 0.9 * keep.size
+        assert np.abs((c - b)[keep]).max() <= 200 * 2.0 ** -24 * np.abs(b).max(), name
+
+
 def thermalized(fib, st, steps, seed=777):
     """positions and frames `steps` oracle steps into a trajectory, and the
     generator to continue it"""
