@@ -86,6 +86,9 @@ def test_pivots_outside_the_normal_range(m, scale):
     assert rel_err(np.ldexp(L, -k[:, None]), T) <= 1e-12
 
 
+# In FP64 super-panels start at 60 block columns: 83 and 84 are panels with a
+# last one of three and of four block columns, and the first sizes with and the
+# last without are those of test_panels_solved_in_one_launch.
 @pytest.mark.parametrize("m,mode", [(5312, E.CHOL_FP64), (5313, E.CHOL_FP64), (4033, E.CHOL_FP32), (4033, E.CHOL_BF16)])
 def test_ends_of_the_super_panels(m, mode):
     """The first sizes with super-panels (84 and 64 block columns) and the last
@@ -122,6 +125,21 @@ def test_panels_solved_in_one_launch(mode, nt):
     assert np.all(np.abs(L @ (L.T @ v) - D @ v) <= bound + (m + 1) * 2.0 ** -53 * (np.abs(D) @ np.abs(v)))
 
 
+@pytest.mark.parametrize("m", [4030, 4032, 4094, 4542])
+def test_super_panels_in_bf16(m):
+    """The last sizes without super-panels in BF16 (63 block columns, with and
+    without padding), the first with (64, a whole last panel) and 71 (a last one
+    of seven).  |L L^T - D| at most (m + 1) u |L| |L^T|, u = 2^-24 for the
+    three-slice products."""
+    D = spd(m, 3)
+    L, neg = E.cholesky_device(D, E.CHOL_BF16)
+    v = np.random.default_rng(1).standard_normal((m, 4))
+    bound = (m + 1) * 2.0 ** -24 * (np.abs(L) @ (np.abs(L.T) @ np.abs(v)))
+    assert neg == 0
+    assert np.all(np.abs(L @ (L.T @ v) - D @ v) <= bound + (m + 1) * 2.0 ** -53 * (np.abs(D) @ np.abs(v)))
+
+
+# In FP64 too: from 60 block columns.
 def test_super_panel_size_and_mixed_modes():
     """4500 rows: 71 block columns, super-panels of 8 in the reduced modes."""
     D = spd(4500, 7)
