@@ -37,8 +37,8 @@
 // ~55 backward.  With one 256-thread workgroup per core (300 charges: three
 // rounds, the last with 44 lanes) 50 cores kept 50 of 256 CUs at 4 wavefronts
 // each, and the IEEE root, quotient and expf of a pair were most of its
-// instructions.  50 cores of 300 charges, forward and backward: 3689 -> 152 us
-// in FP32, 4734 -> 334 us in FP64; 300 cores 3982 -> 741 and 6277 -> 1629 us.
+// instructions.  50 cores of 300 charges, forward and backward: 3692 -> 135 us
+// in FP32, 4734 -> 301 us in FP64; 300 cores 3982 -> 672 and 6277 -> 1581 us.
 // Templated on the arithmetic (float for the FP32 force passes of the
 // differentiable trajectory, double for its FP64 checks).
 #include <hip/hip_runtime.h>
@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(kThreads) k_cc_bwd(int Nq, const T *__restrict
 // charges per block: 16, with fewer idle lanes in the last block (300 charges:
 // 304 lanes against 320) and more workgroups, until the blocks of 64 alone
 // are several rounds of workgroups, which then read half the records from
-// LDS.  Forward and backward with 64 / 16, us: 20 cores FP32 142 / 110, FP64
+// LDS.  Forward and backward with 64 / 16 in turn, us: 20 cores FP32 142 / 110, FP64
 // 270 / 158; 50 cores 158 / 152, 306 / 334; 120 cores 382 / 332, 826 / 731;
 // 300 cores 741 / 760, 1629 / 1726.
 int block_charges(int n_c, int Nq) { return n_c * ((Nq + 63) / 64) >= 1000 ? 64 : 16; }

@@ -1097,7 +1097,8 @@ __global__ void __launch_bounds__(256, 2) k_step(double *A, int ld, int kb, int 
     step_tile<MODE>(S, A, ld, kb, jcols, lb, Linv, neg, nullptr);
 }
 
-// The same with one workgroup of two teams per CU, for 257 to 511 tiles: tile
+// The same with one workgroup of two teams per CU, for 257 to 485 tiles on 256
+// CUs (from 486, split_tiles, k_panel and k_update are the shorter way): tile
 // 0 has workgroup 0, and with it a CU, to itself, so that its factor, a chain
 // of FP64 vector arithmetic, does not stand still beside another workgroup's
 // matrix products; the others go in contiguous runs to the XCDs (workgroups go
@@ -1407,8 +1408,9 @@ __device__ __forceinline__ void bf_body(const __bf16 *sp, int ra, int rbw, int n
         }
     }
 }
-// The blocks of an XCD follow each other in 8x8 groups (group_index), so a
-// group's 16 row and 16 column panel tiles are read into one L2.
+// The blocks of an XCD follow each other in 4x4 groups (group_index), so a
+// group's 8 row and 8 column panel tiles are read into one L2 (8x8 groups, 16
+// and 16 tiles: 17.6 ms of trailing updates at 1000 nucleosomes against 16.8).
 constexpr int kBfLds = 48 * 512;  // of BF16
 __device__ __forceinline__ void trail_bf_block(__bf16 *S, double *A, int ld, const __bf16 *sp, int nb, int j0, int nt, int IB,
                                                int JB, double *Linv, int *neg) {
@@ -1505,15 +1507,16 @@ __global__ void __launch_bounds__(256) k_pack64(const double *A, int ld, int k0,
 // from global memory straight into registers, the next step's while the
 // matrix cores work on the current one's.  No LDS, no barrier, and a
 // quarter that lies above the diagonal costs nothing.  What bounds it is the
-// matrix cores: 67 TF in FP64, of 78 that a loop of nothing but products
-// reaches, and 112 of 157 in FP32, where reading and writing the tile takes
-// its share.  A CU reads 32 bytes of operands a cycle, half of what its L1
-// gives.  The form before (128x128 blocks staged through LDS by direct copies,
-// two barriers per 16 of K) reached in FP64 60.0 / 54.0 / 48.2 TF at 320 / 156
-// / 80 trailing block rows, this one 64 / 66.9 / 67.5; 64x64 per wavefront in
-// this form reached 64.4 / 62.0 / 52.8 (as few as 3 such blocks per CU) and in
-// FP32 66 against 97 TF.  With the operand addresses in vector registers it
-// was 65 and 100 TF.  Three workgroups share a CU (the LDS of the first tile's
+// matrix cores, 85% busy in FP64 and 71% in FP32, where reading and writing the
+// tile takes its share: over the launches of a factor 63 TF at 1000 nucleosomes
+// (61 to 67 a launch) and 61 at 500, in FP32 110 at 1000, of 78 and 157 that a
+// loop of nothing but products reaches.  A CU reads 32 bytes of operands a
+// cycle, half of what its L1 gives.  A launch alone, repeated: the form before
+// (128x128 blocks staged through LDS by direct copies, two barriers per 16 of K)
+// in FP64 60.0 / 54.0 / 48.2 TF at 320 / 156 / 80 trailing block rows, this one
+// 64 / 66.9 / 67.5; 64x64 per wavefront in this form 64.4 / 62.0 / 52.8 (as few
+// as 3 such blocks per CU) and in FP32 66 against 97 TF.  With the operand
+// addresses in vector registers 65 and 100 TF where now 67 and 112.  Three workgroups share a CU (the LDS of the first tile's
 // factor); a fourth changed nothing, nor did the tile's own loads before the
 // loop (FP32 slower by a fifth: the registers).
 //
@@ -1676,7 +1679,8 @@ __global__ void __launch_bounds__(256, 1) k_block_step(double *A, int ld, int kb
 // workgroups (64 block rows; 16 of them the products at the matrix cores'
 // rate), 50 up to 512, where column by column beside the block's own steps the
 // rows took 3 to 11 us per column, with the trailing update's tiles left
-// outside.  Operands in other layouts, with a transposition through LDS on
+// outside; 80 up to 768, 105 up to 1024, 135 at 1280 (matrix cores 47% busy over
+// a factor at 1000 nucleosomes).  Operands in other layouts, with a transposition through LDS on
 // either side of each column: 31 and 56 us.
 constexpr int kPanelTiles = kPanel * (kPanel + 1) / 2;
 // Order of the products of k_panel_rows: the solve of column 0, then for each
@@ -2003,9 +2007,12 @@ void launch_rpy(const Stat &s, int n_hi, const Geo &g, const double *rad_all, co
     // the positions D is built from, kept only where a refinement can read them
     if (refine_active(c)) k_hi_snapshot<<<nblk(c.m / 3, 256), 256, 0, q>>>(s, g, c.m / 3, c.xs);
     // the first tile's factor inside the assembly launch saves a launch on
-    // the factor's chain, but gives every workgroup the factor's LDS (one
-    // per CU): from 64 block columns the assembly takes its own launch
-    // (four workgroups per CU) and k_diag the first tile
+    // the factor's chain, but gives every workgroup the factor's LDS (43 KB,
+    // three per CU): for many tiles the assembly takes its own launch (33 KB,
+    // four per CU) and k_diag the first tile.  One launch / two, us: 17 block
+    // columns 21 / 26, 33 21 / 29, 52 25 / 39, 66 30 / 42, 99 64 / 70, 164 160
+    // / 127, 328 515 / 445; the factor as a whole differs by more than its
+    // runs up to 66 only (33: 504 / 515 us, 66: 1357 / 1366)
     if (factor_first && nt < 64) {
         k_rpy<true><<<nt * (nt + 1) / 2, 256, 0, q>>>(s, g, rad_all, c.A, c.m, c.ld, s.a1, s.a2, c.neg, c.Linv);
     } else {

@@ -192,7 +192,9 @@ constexpr ExpCoef6 kExpCoef6 = {{1.0 / 720.0, 1.0 / 120.0, 1.0 / 24.0, 1.0 / 6.0
 // ln2/32 + r with m = 32n + j = rint(32x/ln2) and |r| <= ln2/64, the two-part
 // ln2 above scaled by 1/32 (so m ln2_hi/32 is exact); e^r by its Taylor
 // series to r^6 (truncation below 4e-18), times tab[j] = 2^(j/32) and 2^n.
-// Seven FMAs instead of the twelve of exp_neg_c, for one table read.
+// Seven FMAs instead of the twelve of exp_neg_c, for one table read.  No kernel
+// takes it: it is the plain form of exp_neg_f, held beside it by the host's
+// checks of the table and the series.
 template <typename C>
 __host__ __device__ __forceinline__ double exp_neg_t(double x, const double *tab, const C &k) {
     const double m = rint(x * 46.166241308446828);
@@ -206,7 +208,7 @@ __host__ __device__ __forceinline__ double exp_neg_t(double x, const double *tab
     p = __builtin_fma(p, r, 1.0);
     return __builtin_ldexp(tab[im & 31] * p, im >> 5);
 }
-// e^(-kappa d) in the same form from y = k d, k = -kappa 32/ln2: m = rint(y)
+// The core-core kernel's e^(-kappa d), the same from y = k d, k = -kappa 32/ln2: m = rint(y)
 // comes out of the low bits of y + 1.5 2^52 (as an int: right for |y| < 2^31,
 // kappa d < 4.6e7), f = y - m is exact, and the series
 // of e^(f ln2/32) takes the powers of ln2/32 into its coefficients: no reduction

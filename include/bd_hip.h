@@ -218,8 +218,9 @@ int bd_cholesky(int m, const double *D, int ldd, double *L, int ldl, int mode, i
 int bd_cholesky_release(void);
 
 /* bd_cholesky without any allocation: no counterpart in the reference; for
- * callers that cannot allocate device memory (code under HIP graph capture,
- * tight serving loops, harnesses that forbid hipMalloc).  The workspace is a
+ * callers that cannot allocate device memory (beside another thread's HIP graph
+ * capture, in tight serving loops, in harnesses that forbid hipMalloc; the call
+ * waits for its stream, which must not be under capture itself).  The workspace is a
  * static device array of the library, BD_CHOLESKY_NOALLOC_MAX_M rows at
  * most (36.8 MB, held by every GPU the library runs on until the process
  * ends); larger m returns BD_E_CAPACITY.  All calls on one GPU share that
@@ -268,7 +269,11 @@ int bd_cc_backward(int fp64, int n_c, int Nq, const void *Q, const void *q, cons
  * (it uses the self-mobilities). */
 int bd_set_frequency_rp(bd_context *ctx, int frequency_rp);
 
-/* Per-kernel timing with HIP events on the context's stream (0 = off). */
+/* Per-kernel timing with HIP events on the context's stream (0 = off).
+ * bd_get_timing lists the launches that ran, by what they belong to.  The
+ * factor's are chol_step and chol_trail: a diagonal tile is factored inside
+ * one of them (the first inside rpy) and has no entry of its own (chol_diag
+ * once). */
 int bd_set_timing(bd_context *ctx, int enable);
 typedef struct bd_kernel_time {
     char name[48];

@@ -85,6 +85,7 @@ def test_exp_table_correctly_rounded(measured):
         assert measured["tab"][j] == float(exact), j
 
 
+# The core-core kernel takes exp_neg_f (below), exp_neg_t is its plain form.
 def test_exp_neg_t_accuracy(measured):
     # table entry (half an ulp), series and product roundings: a few ulps at most
     assert measured["exp"] <= 4e-16

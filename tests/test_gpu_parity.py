@@ -406,6 +406,8 @@ def test_super_panel_schedule_factor(panel):
         assert e <= 1e-6 and rel_err(Ls[mode], L0) <= 1e-5
 
 
+# The packed form is the default at every size now; the variable set below keeps
+# it so.
 @pytest.mark.parametrize("mode", [E.CHOL_FP64, E.CHOL_FP32, E.CHOL_BF16])
 @pytest.mark.parametrize("panel", [2, 3, 8])
 def test_packed_panels_equal_direct(mode, panel, monkeypatch):
