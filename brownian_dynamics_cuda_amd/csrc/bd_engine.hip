@@ -207,6 +207,17 @@ void enqueue_forces(bd_context *c, const Geo &g, const Frc &f, double *Epart, in
 // columns, 356 / 368; 16 block columns, all beads, 380 / 411).
 constexpr int kBranchTiles = 9;
 
+// bd_forces, with no factor beside it: branches cost the streams' events and
+// hand-overs, about 30 us, and hide the core-core kernels behind the others
+// (us on one stream / branched, without linker histones: all terms 12
+// nucleosomes 169 / 176, 50 232 / 233, 80 267 / 260, 300 575 / 540; the
+// electrostatic term alone 12 151 / 166, 100 243 / 253, 300 477 / 469); without
+// it they hide nothing (134 / 171 at 12, 272 / 296 at 300).
+bool forces_branch(const bd_context *c, int terms) {
+    if (!(terms & BD_TERM_ELEC)) return false;
+    return c->n_c >= ((terms & BD_TERM_TAIL) && c->n_tail ? 75 : 250);
+}
+
 void enqueue_factor(bd_context *c, const Geo &g, hipStream_t q, hipEvent_t gate = nullptr, int gate_kb = -1) {
     Marker M{c};
     M(K_RPY, 0);
@@ -897,7 +908,7 @@ int bd_forces(bd_context *c, int terms, double *F, double *T, double *tF, double
     if (check(c)) return BD_E_ARG;
     if (!c->state_set) return fail(BD_E_STATE, "bd_set_state must be called first");
     HIPCHK(hipSetDevice(c->device));
-    enqueue_forces(c, c->cur, c->f0, c->Epart, terms, 0, true);
+    enqueue_forces(c, c->cur, c->f0, c->Epart, terms, 0, forces_branch(c, terms));
     launch_energy_reduce(c->Epart, c->ne, c->energy, c->stream);
     HIPCHK(hipGetLastError());
     if (c->timing) collect_timing(c);

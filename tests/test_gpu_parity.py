@@ -218,6 +218,23 @@ def test_fused_launches_equal_timed_separate_launches(kind):
         assert np.array_equal(v, outs[1][2][k]), k
 
 
+@pytest.mark.parametrize("n_c, lh", [(74, True), (75, True), (249, False), (250, False)])
+def test_force_branches_equal_one_stream(n_c, lh):
+    """bd_forces on the sizes around its lines between one stream and branches,
+    term by term: the timing mode's launches, on one stream always, give the
+    same forces, torques and energies bit for bit."""
+    fib, st = Fb.make_fiber(n_c, seed=n_c, with_lh=lh)
+    with E.BDEngine(fib) as eng:
+        eng.set_state(st, rebuild=True)
+        for terms in (E.TERM_ALL, E.TERM_ELEC, E.TERM_ELEC | E.TERM_TAIL, E.TERM_MECH, E.TERM_TAIL | E.TERM_LH):
+            got = []
+            for timed in (False, True):
+                eng.set_timing(timed)
+                got.append(eng.forces(terms))
+            for k, v in got[0].items():
+                assert np.array_equal(v, got[1][k]), (terms, k)
+
+
 def test_device_noise_path_equals_host_noise_path():
     fib, st = deck("tiny")
     rr, p = noise(fib)
