@@ -22,15 +22,15 @@
 // and dphi/dq_k = q_l (uz gh + eps eh) with gh = g_DH / (q_k q_l),
 // eh = E_DH / (q_k q_l) (the excluded volume does not depend on charge).
 //
-// Layout: a workgroup owns a block of KB charges of a core i (blockIdx.y),
-// one per lane; the partner charges of the core (CSR list, both directions)
-// pass through LDS as one stream of records, dealt over the workgroup's
+// Layout: a workgroup of NT threads owns a block of KB charges of a core i
+// (blockIdx.y), one per lane; the partner charges of the core (CSR list, both directions)
+// pass through LDS as one stream of records, NT at a time, dealt over the workgroup's
 // wavefronts (and, for KB < 64, over the lanes' groups of KB), and their
 // partial sums are added in a fixed order at the end.  Every pair is
 // evaluated from both sides, so each site's output has one owner and there
 // are no atomics: the results are deterministic.  A core's energy needs its
-// blocks' parts: with a work buffer each block leaves its part there and
-// k_cc_esum adds them, without one a single workgroup takes all the core's
+// blocks' parts: with a work buffer each of several blocks leaves its part there
+// and k_cc_esum adds them, without one a single workgroup takes all the core's
 // blocks in turn (bd_cc_forward).
 //
 // What bounds it: FP32 (FP64) VALU issue, ~40 instructions a pair forward and
@@ -52,9 +52,7 @@
 namespace bd {
 namespace {
 
-constexpr int kThreads = 1024;
 constexpr int kMaxSites = 640;  // charges per core
-constexpr int kTile = 1024;     // partner records in LDS at a time
 
 struct CCParams {
     double ke, kappa, kex, sigma;
@@ -117,9 +115,9 @@ template <typename T> struct alignas(4 * sizeof(T)) Rec4 {
 // The sums v of the workgroup's slots (SL slots of KB lanes), added in slot
 // order by the first KB NV threads: result of value u of lane k on thread
 // u KB + k.
-template <typename T, int KB, int NV>
+template <typename T, int KB, int NT, int NV>
 __device__ __forceinline__ T slot_sum(const T (&v)[NV], T *buf) {
-    constexpr int SL = kThreads / KB;
+    constexpr int SL = NT / KB;
     const int k = threadIdx.x % KB, s = threadIdx.x / KB;
     __syncthreads();
 #pragma unroll
@@ -134,24 +132,24 @@ __device__ __forceinline__ T slot_sum(const T (&v)[NV], T *buf) {
 // f[i][k][3] of the block's charges, and half the energy of its pairs into
 // eo: e[i] where the workgroup takes every block (gridDim.y = 1), else the
 // block's part work[i gridDim.y + block]
-template <typename T, int KB>
-__global__ void __launch_bounds__(kThreads) k_cc_fwd(int Nq, const T *__restrict__ Q, const T *__restrict__ q,
+template <typename T, int KB, int NT>
+__global__ void __launch_bounds__(NT) k_cc_fwd(int Nq, const T *__restrict__ Q, const T *__restrict__ q,
                                                      const int *__restrict__ off, const int *__restrict__ nbr,
                                                      CCParams p, T *__restrict__ f, T *__restrict__ eo) {
-    constexpr int SL = kThreads / KB;
-    __shared__ Rec4<T> S[kTile];
+    constexpr int SL = NT / KB;
+    __shared__ Rec4<T> S[NT];
     const int i = blockIdx.x, slot = threadIdx.x / KB, s0 = off[i], M = (off[i + 1] - s0) * Nq;
-    static_assert(sizeof(S) >= kThreads * 4 * sizeof(T), "the slots' sums take the records' place");
+    static_assert(sizeof(S) >= NT * 4 * sizeof(T), "the slots' sums take the records' place");
     T en = T(0);
     for (int k0 = blockIdx.y * KB; k0 < Nq; k0 += gridDim.y * KB) {
         const int k = min(k0 + (int)threadIdx.x % KB, Nq - 1);
         const T *src = Q + ((size_t)i * Nq + k) * 3;
         const T px = src[0], py = src[1], pz = src[2], qk = q[k];
         T v[4] = {T(0), T(0), T(0), T(0)};
-        for (int t0 = 0; t0 < M; t0 += kTile) {
-            const int R = min(M - t0, kTile);
+        for (int t0 = 0; t0 < M; t0 += NT) {
+            const int R = min(M - t0, NT);
             __syncthreads();
-            for (int r = threadIdx.x; r < R; r += kThreads) {
+            for (int r = threadIdx.x; r < R; r += NT) {
                 const int m = t0 + r, l = m % Nq;
                 const T *o = Q + ((size_t)nbr[s0 + m / Nq] * Nq + l) * 3;
                 S[r] = Rec4<T>{o[0], o[1], o[2], q[l]};
@@ -169,7 +167,7 @@ __global__ void __launch_bounds__(kThreads) k_cc_fwd(int Nq, const T *__restrict
                 v[3] += t.e;
             }
         }
-        const T sum = slot_sum<T, KB, 4>(v, reinterpret_cast<T *>(S));
+        const T sum = slot_sum<T, KB, NT, 4>(v, reinterpret_cast<T *>(S));
         const int u = threadIdx.x / KB, kk = k0 + threadIdx.x % KB;
         if (threadIdx.x < 3 * KB && kk < Nq) f[((size_t)i * Nq + kk) * 3 + u] = sum;
         if (u == 3 && kk < Nq) en += T(0.5) * sum;
@@ -193,23 +191,23 @@ __global__ void k_cc_esum(int n_c, int parts, const T *__restrict__ work, T *__r
 
 // gQ[i][k][3] and gq[i][k] (per-site charge gradient; the template
 // gradient is its sum over cores), both written
-template <typename T, int KB>
-__global__ void __launch_bounds__(kThreads) k_cc_bwd(int Nq, const T *__restrict__ Q, const T *__restrict__ q,
+template <typename T, int KB, int NT>
+__global__ void __launch_bounds__(NT) k_cc_bwd(int Nq, const T *__restrict__ Q, const T *__restrict__ q,
                                                      const int *__restrict__ off, const int *__restrict__ nbr,
                                                      CCParams p, const T *__restrict__ gf, const T *__restrict__ ge,
                                                      T *__restrict__ gQ, T *__restrict__ gqs) {
-    constexpr int SL = kThreads / KB;
-    __shared__ Rec4<T> S[2 * kTile];
+    constexpr int SL = NT / KB;
+    __shared__ Rec4<T> S[2 * NT];
     const int i = blockIdx.x, slot = threadIdx.x / KB, s0 = off[i], M = (off[i + 1] - s0) * Nq;
     const int k0 = blockIdx.y * KB, k = min(k0 + (int)threadIdx.x % KB, Nq - 1);
     const size_t ok = ((size_t)i * Nq + k) * 3;
     const T px = Q[ok], py = Q[ok + 1], pz = Q[ok + 2], lx = gf[ok], ly = gf[ok + 1], lz = gf[ok + 2], qk = q[k];
     const T ei = ge[i];
     T v[4] = {T(0), T(0), T(0), T(0)};
-    for (int t0 = 0; t0 < M; t0 += kTile) {
-        const int R = min(M - t0, kTile);
+    for (int t0 = 0; t0 < M; t0 += NT) {
+        const int R = min(M - t0, NT);
         __syncthreads();
-        for (int r = threadIdx.x; r < R; r += kThreads) {
+        for (int r = threadIdx.x; r < R; r += NT) {
             const int m = t0 + r, l = m % Nq, j = nbr[s0 + m / Nq];
             const size_t o = ((size_t)j * Nq + l) * 3;
             S[2 * r] = Rec4<T>{Q[o], Q[o + 1], Q[o + 2], q[l]};
@@ -230,7 +228,7 @@ __global__ void __launch_bounds__(kThreads) k_cc_bwd(int Nq, const T *__restrict
             v[3] += o.w * (uz * t.gh + w.w * t.eh);
         }
     }
-    const T sum = slot_sum<T, KB, 4>(v, reinterpret_cast<T *>(S));
+    const T sum = slot_sum<T, KB, NT, 4>(v, reinterpret_cast<T *>(S));
     const int u = threadIdx.x / KB, kk = k0 + threadIdx.x % KB;
     if (kk < Nq) {
         if (u < 3) gQ[((size_t)i * Nq + kk) * 3 + u] = sum;
@@ -238,36 +236,55 @@ __global__ void __launch_bounds__(kThreads) k_cc_bwd(int Nq, const T *__restrict
     }
 }
 
-// charges per block: 16, with fewer idle lanes in the last block (300 charges:
-// 304 lanes against 320) and more workgroups, until the blocks of 64 alone
-// are several rounds of workgroups, which then read half the records from
-// LDS.  Forward and backward with 64 / 16 in turn, us: 20 cores FP32 142 / 110, FP64
-// 270 / 158; 50 cores 158 / 152, 306 / 334; 120 cores 382 / 332, 826 / 731;
-// 300 cores 741 / 760, 1629 / 1726.
-int block_charges(int n_c, int Nq) { return n_c * ((Nq + 63) / 64) >= 1000 ? 64 : 16; }
+// Charges and threads of a block.  16 charges, with fewer idle lanes in the last
+// block (300 charges: 304 lanes against 320) and more workgroups, until the
+// blocks of 64 alone are several rounds of workgroups, which then read half the
+// records from LDS; 64 only if their lanes are hardly more (5 charges: 64 lanes
+// against 16).  Forward and backward with 64 / 16 in turn, us: 20 cores of 300
+// FP32 142 / 110, FP64 270 / 158; 50 cores 158 / 152, 306 / 334; 120 cores 382 /
+// 332, 826 / 731; 300 cores 741 / 760, 1629 / 1726.  1024 threads share a core's
+// records, but for cores of one block and many of them, where the launch of the
+// wavefronts counts: forward with 1024 / 256 threads, 16 charges, us: 1000 cores
+// with 2 partners FP32 6.4 / 5.2, FP64 9.5 / 5.5, with 80 partners 21.0 / 22.8 and
+// 46.1 / 40.7; 2048 cores 10.4 / 5.0, 16.4 / 7.1, 37.4 / 37.1, 92.1 / 74.5.
+struct Shape {
+    int KB, NT;
+};
+template <typename T>
+Shape block_shape(int n_c, int Nq) {
+    const int b64 = (Nq + 63) / 64, b16 = (Nq + 15) / 16;
+    if (b16 == 1 && n_c >= (sizeof(T) == 8 ? 1000 : 2048)) return {16, 256};
+    if ((long long)n_c * b64 >= 1000 && 10 * 64 * b64 <= 11 * 16 * b16) return {64, 1024};
+    return {16, 1024};
+}
 
 template <typename T>
 void cc_fwd(int n_c, int Nq, const void *Q, const void *q, const int *off, const int *nbr, const CCParams &p, void *f,
             void *e, void *work, hipStream_t s) {
-    const int KB = work ? block_charges(n_c, Nq) : 64, nb = work ? (Nq + KB - 1) / KB : 1;
-    auto *eo = static_cast<T *>(work ? work : e);
-    if (KB == 64)
-        k_cc_fwd<T, 64><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (T *)f, eo);
-    else
-        k_cc_fwd<T, 16><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (T *)f, eo);
-    if (work) k_cc_esum<T><<<(n_c + 255) / 256, 256, 0, s>>>(n_c, nb, eo, (T *)e);
+    const Shape b = work || Nq <= 16 ? block_shape<T>(n_c, Nq) : Shape{64, 1024};
+    const int nb = work ? (Nq + b.KB - 1) / b.KB : 1;
+    // a core of one block has its energy from that
+    auto *eo = static_cast<T *>(nb > 1 ? work : e);
+    auto launch = [&](auto kernel) {
+        kernel<<<dim3(n_c, nb), b.NT, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (T *)f, eo);
+    };
+    if (b.KB == 64) launch(k_cc_fwd<T, 64, 1024>);
+    else if (b.NT == 1024) launch(k_cc_fwd<T, 16, 1024>);
+    else launch(k_cc_fwd<T, 16, 256>);
+    if (nb > 1) k_cc_esum<T><<<(n_c + 255) / 256, 256, 0, s>>>(n_c, nb, eo, (T *)e);
 }
 
 template <typename T>
 void cc_bwd(int n_c, int Nq, const void *Q, const void *q, const int *off, const int *nbr, const CCParams &p,
             const void *gf, const void *ge, void *gQ, void *gqs, hipStream_t s) {
-    const int KB = block_charges(n_c, Nq), nb = (Nq + KB - 1) / KB;
-    if (KB == 64)
-        k_cc_bwd<T, 64><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (const T *)gf,
-                                                           (const T *)ge, (T *)gQ, (T *)gqs);
-    else
-        k_cc_bwd<T, 16><<<dim3(n_c, nb), kThreads, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (const T *)gf,
-                                                           (const T *)ge, (T *)gQ, (T *)gqs);
+    const Shape b = block_shape<T>(n_c, Nq);
+    auto launch = [&](auto kernel) {
+        kernel<<<dim3(n_c, (Nq + b.KB - 1) / b.KB), b.NT, 0, s>>>(Nq, (const T *)Q, (const T *)q, off, nbr, p, (const T *)gf,
+                                                                  (const T *)ge, (T *)gQ, (T *)gqs);
+    };
+    if (b.KB == 64) launch(k_cc_bwd<T, 64, 1024>);
+    else if (b.NT == 1024) launch(k_cc_bwd<T, 16, 1024>);
+    else launch(k_cc_bwd<T, 16, 256>);
 }
 
 int cc_fail(int code, const char *fmt, ...) {

@@ -137,10 +137,12 @@ def test_core_core_blocks(n_c, nq):
     assert rel_err(e.cpu().numpy(), outs["dense"][1]) <= 1e-12
 
 
-@pytest.mark.parametrize("n_c,nq", [(999, 5), (1000, 5), (499, 65), (500, 65), (199, 300), (200, 300)])
+@pytest.mark.parametrize("n_c,nq", [(999, 5), (1000, 5), (499, 65), (500, 65), (199, 300), (200, 300),
+                                    (2047, 5), (2048, 5), (2048, 16), (2048, 17)])
 def test_core_core_block_sizes(n_c, nq):
-    """Both sides of the line between blocks of 16 and of 64 charges (1000
-    blocks of 64), forward with a work buffer and adjoint with the gradient of
+    """Both sides of the lines between blocks of 16 and of 64 charges (1000
+    blocks of 64) and between 1024 and 256 threads (1000 cores of one block
+    in FP64, 2048 in FP32), forward with a work buffer and adjoint with the gradient of
     every site's charge; one core with more partner charges than the records
     held at a time, cores with one partner and cores with none.  Against the
     dense sums in FP64, and FP32 against FP64 on the same inputs: a pair's
