@@ -218,6 +218,16 @@ bool forces_branch(const bd_context *c, int terms) {
     return c->n_c >= ((terms & BD_TERM_TAIL) && c->n_tail ? 75 : 250);
 }
 
+// Launched one by one and not replayed from a graph, the branches' events are
+// host time too, which a fiber of a few nucleosomes does not win back, nor one
+// without linker histones before bd_forces does (us a step on one stream / branched: 2 nucleosomes 212 / 263, 4
+// 298 / 323, 12 322 / 331, 25 364 / 378; with linker histones 4 346 / 347, 12 380
+// / 370, 25 444 / 429).
+bool pass1_branch(const bd_context *c, bool refactor, int nt) {
+    if (refactor && nt > kBranchTiles) return false;
+    return c->use_graph || (c->n_LH && c->n_c >= 6) || forces_branch(c, BD_TERM_ALL);
+}
+
 void enqueue_factor(bd_context *c, const Geo &g, hipStream_t q, hipEvent_t gate = nullptr, int gate_kb = -1) {
     Marker M{c};
     M(K_RPY, 0);
@@ -274,7 +284,7 @@ void enqueue_step(bd_context *c, bool refactor) {
     // LH bending angles at the current state (3497)
     M(K_BETAS, 0); launch_betas(s, c->cur, 0, 1, q); M(K_BETAS, 1);
     // force pass 1 at x0 and its energy (3556-3615)
-    enqueue_forces(c, c->cur, c->f0, c->Epart, BD_TERM_ALL, 0, !refactor || nt <= kBranchTiles);
+    enqueue_forces(c, c->cur, c->f0, c->Epart, BD_TERM_ALL, 0, pass1_branch(c, refactor, nt));
     M(K_EREDUCE, 0); launch_energy_reduce(c->Epart, c->ne, c->energy, q); M(K_EREDUCE, 1);
     if (qf != q) {
         (void)hipEventRecord(c->ev_join, qf);
