@@ -767,12 +767,14 @@ __device__ __forceinline__ void below_row(dbl4 (&Z)[6], const DiagLds &l) {
 // entry, and L = inv(S) L', inv(L) = inv(L') S on its way out: the scaling is
 // exact.  Inside the bounds the pivots keep clear of 2^-1022 (cancellation
 // takes 53 bits at most) and nothing is scaled.  The test is one LDS read and
-// one comparison beside the tile's own reads.
+// one comparison ahead of the tile's own reads (33 block columns 500.2 -> 501.3
+// us a factor, 49 847.0 -> 848.8); beside them, a copy of the
+// scaling to each wavefront's role, it cost three times that.
 __device__ __forceinline__ bool tile_out_of_range(const double *T) {
     const double d = fabs(T[(tid() & 63) * (LDP + 1)]);
-    return __builtin_expect(__ballot(!(d >= 0x1p-960 && d <= 0x1p+960)) != 0, false);
+    return __ballot(!(d >= 0x1p-960 && d <= 0x1p+960)) != 0;
 }
-// By all four wavefronts, once they have read T; they read it again after it.
+// By all four wavefronts, before they read T.
 __device__ __forceinline__ void rescale_tile(const DiagLds &l, double *T) {
     __syncthreads();
     if (tid() < TB) {
@@ -810,22 +812,13 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
     const int lane = tid() & 63, wv = __builtin_amdgcn_readfirstlane(tid() >> 6);
     const int g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
     const DiagLds l = {lds};
-    bool scaled;
-    auto read_tile = [&](auto read) {
-        read();
-        scaled = tile_out_of_range(T);
-        if (scaled) {
-            rescale_tile(l, T);
-            read();
-        }
-        __syncthreads();
-    };
+    const bool scaled = tile_out_of_range(T);
+    if (__builtin_expect(scaled, false)) rescale_tile(l, T);
     if (wv == 0) {
         double w[16], r[16];
-        read_tile([&]() {
 #pragma unroll
-            for (int k = 0; k < 16; k++) w[k] = T[max(k, ci) * LDP + min(k, ci)];
-        });
+        for (int k = 0; k < 16; k++) w[k] = T[max(k, ci) * LDP + min(k, ci)];
+        __syncthreads();
 #pragma unroll 1
         for (int b = 0; b < 4; b++) {
             if (b) load_rows(w, l.next(3) + kNextPitch * c);
@@ -844,10 +837,9 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
         }
     } else if (wv == 1) {
         double x[16];
-        read_tile([&]() {
 #pragma unroll
-            for (int k = 0; k < 16; k++) x[k] = g < 3 ? T[(16 * (g + 1) + ci) * LDP + k] : k == ci ? 1.0 : 0.0;
-        });
+        for (int k = 0; k < 16; k++) x[k] = g < 3 ? T[(16 * (g + 1) + ci) * LDP + k] : k == ci ? 1.0 : 0.0;
+        __syncthreads();
 #pragma unroll 1
         for (int b = 0; b < 4; b++) {
             if (b) {
@@ -873,21 +865,15 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
             o[0] = o[1] = dbl2{0.0, 0.0};
         }
         if (wv == 2) {
-            dbl4 Z[6];
-            read_tile([&]() {
-                Z[0] = tile_block(T, 1, 1);
-                Z[1] = tile_block(T, 1, 2);
-                Z[2] = tile_block(T, 2, 2);
-                Z[3] = tile_block(T, 2, 3);
-                Z[4] = tile_block(T, 3, 3);
-                Z[5] = z;
-            });
+            dbl4 Z[6] = {tile_block(T, 1, 1), tile_block(T, 1, 2), tile_block(T, 2, 2), tile_block(T, 2, 3),
+                         tile_block(T, 3, 3), z};
+            __syncthreads();
             below_row<0, 0>(Z, l);
             below_row<1, 0>(Z, l);
             below_row<2, 0>(Z, l);
         } else {
-            dbl4 Z[6] = {z, z, z, z, z, z};
-            read_tile([&]() { Z[0] = tile_block(T, 1, 3); });
+            dbl4 Z[6] = {tile_block(T, 1, 3), z, z, z, z, z};
+            __syncthreads();
             below_row<0, 1>(Z, l);
             below_row<1, 1>(Z, l);
             below_row<2, 1>(Z, l);
@@ -902,7 +888,7 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
     }
     store_block(l, 3, wv, A, ld, d0, Linv);
     if (wv == 0) store_block(l, 3, 4, A, ld, d0, Linv);
-    if (scaled) unscale_tile(l, A, ld, d0, Linv);
+    if (__builtin_expect(scaled, false)) unscale_tile(l, A, ld, d0, Linv);
 }
 
 // a tile between global memory, registers and LDS (pitch LDP), 16-byte
