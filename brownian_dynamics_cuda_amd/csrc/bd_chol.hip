@@ -802,11 +802,74 @@ __device__ __forceinline__ void unscale_tile(const DiagLds &l, double *A, int ld
     }
 }
 
+// A pivot of exactly 0, which rows that depend on each other leave where the
+// column-wise form had a rounding error (a reciprocal times its pivot is mostly
+// exactly 1, a root squared is not), makes all that follows NaN.  The
+// elimination therefore keeps a copy of its tile (save, row-major, the lower
+// triangle), and a tile with a pivot that has no reciprocal root is factored
+// again from it column by column: L's column and inv(L)'s row of a zero pivot
+// are 0, so that L L^T is D for dependent rows.
+__device__ __forceinline__ void save_block(double *save, int i, int j, dbl4 x) {
+    const int lane = tid() & 63, g = lane >> 4, c = lane & 15, ci = 4 * (c & 3) + (c >> 2);
+    dbl2 *d = reinterpret_cast<dbl2 *>(save + (16 * j + ci) * TB + 16 * i + 4 * g);
+    d[0] = dbl2{x[0], x[1]};
+    d[1] = dbl2{x[2], x[3]};
+}
+__device__ __forceinline__ bool pivot_without_root(const DiagLds &l) {
+    return __ballot(!(l.S()[tid() & 63] < HUGE_VAL)) != 0;
+}
+__device__ __forceinline__ void refactor_tile(const DiagLds &l, const double *save, double *A, int ld, int d0, double *Linv,
+                                              int *neg) {
+    double *T = l.base, *I = l.base + TB * LDP;  // inv(L) above T's diagonal, transposed, and its diagonal in I
+    static_assert(TB * LDP + TB <= 5376, "below the exponents");
+    __syncthreads();
+#pragma unroll 1
+    for (int e = tid(); e < TB * TB; e += NTHR)
+        if (e % TB <= e / TB) T[(e / TB) * LDP + e % TB] = save[e];
+    __syncthreads();
+    int n = 0;
+#pragma unroll 1
+    for (int j = 0; j < TB; j++) {
+        const double f = T[j * (LDP + 1)], a = fabs(f), inv = a == 0.0 ? 0.0 : rsqrt_f64(a);
+        n += f < 0;
+        __syncthreads();
+        if (tid() < TB && tid() >= j) T[tid() * LDP + j] = tid() == j ? a * inv : T[tid() * LDP + j] * inv;
+        if (tid() == j) I[j] = inv;
+        __syncthreads();
+#pragma unroll 1
+        for (int e = tid(); e < TB * TB; e += NTHR) {
+            const int r = e / TB, c = e % TB;
+            if (c > j && c <= r) T[r * LDP + c] -= T[r * LDP + j] * T[c * LDP + j];
+        }
+        __syncthreads();
+    }
+    if (tid() == 0 && n) atomicAdd(neg, n);
+#pragma unroll 1
+    for (int e = tid(); e < TB * TB; e += NTHR) {
+        const int r = e / TB, c = e % TB;
+        if (c <= r) A[(size_t)(d0 + r) * ld + d0 + c] = T[r * LDP + c];
+    }
+    if (tid() < TB) {
+        const int c = tid();
+#pragma unroll 1
+        for (int i = 0; i < TB; i++) {
+            double x = i == c ? I[c] : 0.0;
+            if (i > c) {
+                x = -T[i * LDP + c] * I[c];
+                for (int k = c + 1; k < i; k++) x -= T[i * LDP + k] * T[c * LDP + k];
+                x *= I[i];
+                T[c * LDP + i] = x;
+            }
+            Linv[i * TB + c] = x;
+        }
+    }
+}
+
 // Called by all four wavefronts.  lds: kDiagLds doubles; T, LDS that may
 // overlap its first 5376 doubles, holds the tile (pitch LDP) at (d0, d0), of
 // which the lower triangle is read.  L goes
 // to A (lower triangle), inv(L), row-major 64x64 with zeros above its
-// diagonal, to Linv.
+// diagonal, to Linv; the tile behind it there, the next column's, is scratch.
 __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *A, int ld, int d0, double *Linv,
                                                 int *neg) {
     const int lane = tid() & 63, wv = __builtin_amdgcn_readfirstlane(tid() >> 6);
@@ -814,6 +877,8 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
     const DiagLds l = {lds};
     const bool scaled = tile_out_of_range(T);
     if (__builtin_expect(scaled, false)) rescale_tile(l, T);
+    double *save = Linv + TB * TB;
+    int nneg = 0;  // of wavefront 0
     if (wv == 0) {
         double w[16], r[16];
 #pragma unroll
@@ -830,8 +895,7 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
             // the scale factors of the block row and its negative pivots
             const double fd = l.W(b, b)[64 * (c >> 2) + 4 * pos16(c) + (c & 3)];
             if (lane < 16) l.S()[16 * b + c] = rsqrt_f64(fabs(fd));
-            const unsigned long long nm = __ballot(lane < 16 && fd < 0);
-            if (nm && lane == 0) atomicAdd(neg, __popcll(nm));
+            nneg += __popcll(__ballot(lane < 16 && fd < 0));
             __syncthreads();
             if (b < 3) __syncthreads();
         }
@@ -840,6 +904,10 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
 #pragma unroll
         for (int k = 0; k < 16; k++) x[k] = g < 3 ? T[(16 * (g + 1) + ci) * LDP + k] : k == ci ? 1.0 : 0.0;
         __syncthreads();
+        if (g < 3)
+#pragma unroll
+            for (int k = 0; k < 16; k += 2)
+                *reinterpret_cast<dbl2 *>(save + (16 * (g + 1) + ci) * TB + k) = dbl2{x[k], x[k + 1]};
 #pragma unroll 1
         for (int b = 0; b < 4; b++) {
             if (b) {
@@ -868,12 +936,20 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
             dbl4 Z[6] = {tile_block(T, 1, 1), tile_block(T, 1, 2), tile_block(T, 2, 2), tile_block(T, 2, 3),
                          tile_block(T, 3, 3), z};
             __syncthreads();
+            save_block(save, 1, 1, Z[0]);
+            save_block(save, 1, 2, Z[1]);
+            save_block(save, 2, 2, Z[2]);
+            save_block(save, 2, 3, Z[3]);
+            save_block(save, 3, 3, Z[4]);
             below_row<0, 0>(Z, l);
             below_row<1, 0>(Z, l);
             below_row<2, 0>(Z, l);
         } else {
             dbl4 Z[6] = {tile_block(T, 1, 3), z, z, z, z, z};
+            const dbl4 first = tile_block(T, 0, 0);
             __syncthreads();
+            save_block(save, 0, 0, first);
+            save_block(save, 1, 3, Z[0]);
             below_row<0, 1>(Z, l);
             below_row<1, 1>(Z, l);
             below_row<2, 1>(Z, l);
@@ -886,8 +962,11 @@ __device__ __forceinline__ void diag_factor_inv(double *lds, double *T, double *
                 for (int t = 4 * p + wv - 2; t < min(4 * p + 4, 15); t += 2) store_block(l, t / 5, t % 5, A, ld, d0, Linv);
         }
     }
+    const bool broken = pivot_without_root(l);
     store_block(l, 3, wv, A, ld, d0, Linv);
     if (wv == 0) store_block(l, 3, 4, A, ld, d0, Linv);
+    if (__builtin_expect(broken, false)) refactor_tile(l, save, A, ld, d0, Linv, neg);
+    else if (wv == 0 && lane == 0 && nneg) atomicAdd(neg, nneg);
     if (__builtin_expect(scaled, false)) unscale_tile(l, A, ld, d0, Linv);
 }
 

@@ -626,6 +626,7 @@ int bd_create(const bd_system *sys, const bd_options *opt, bd_context **out) {
     }
     r |= c->alloc(&c->chol.A, (size_t)c->chol.ld * c->chol.ld);
     r |= c->alloc(&c->chol.Linv, (size_t)(c->chol.ld / 64) * 64 * 64 + kPanelDoubles);
+    // the last diagonal tile's scratch is Lp's first tile, read by then
     c->chol.Lp = c->chol.Linv + (size_t)(c->chol.ld / 64) * 64 * 64;
     r |= c->alloc(&c->chol.neg, 1);
     c->chol.refine = 1;

@@ -71,7 +71,7 @@ void launch_commit(const Stat &s, const Geo &from, const Geo &to, hipStream_t q)
 struct CholWork {
     double *A;       // mpad x ld, row-major; lower triangle holds D then L
     int m, mpad, ld;
-    double *Linv;    // (ld/64) tiles of 64x64: inverses of the diagonal factors, row-major
+    double *Linv;    // (ld/64) tiles of 64x64: inverses of the diagonal factors, row-major; one tile of scratch behind
     int *neg;        // negative-pivot counter
     int mode;        // BD_CHOL_*
     // block columns with at least this many trailing tiles take the

@@ -68,12 +68,12 @@ CholWork work_of(int m, int mode) {
 
 // Work of one factor in the workspace at ws (doubles): the padded matrix
 // (mpad x mpad), the inverses of the diagonal factors (one 64x64 tile per
-// block column) and the negative-pivot counter; behind these, where packed,
+// block column and one of scratch) and the negative-pivot counter; behind these, where packed,
 // the packed panel tiles of the super-panels (pack_bytes, 0 for a matrix that
 // has none).
 size_t workspace_doubles(int m) {
     const size_t mpad = ((size_t)m + 63) / 64 * 64;
-    return mpad * mpad + (mpad / 64) * 64 * 64 + 32;
+    return mpad * mpad + (mpad / 64 + 1) * 64 * 64 + 32;
 }
 
 size_t pack_bytes(int m, int mode) {
@@ -87,7 +87,7 @@ int run_factor(int m, const double *D, int ldd, double *L, int ldl, int mode, in
     CholWork c = work_of(m, mode);
     c.A = ws;
     c.Linv = ws + (size_t)c.mpad * c.mpad;
-    c.neg = reinterpret_cast<int *>(c.Linv + (size_t)(c.mpad / 64) * 64 * 64);
+    c.neg = reinterpret_cast<int *>(c.Linv + (size_t)(c.mpad / 64 + 1) * 64 * 64);
     c.Lp = ws + workspace_doubles(m);
     if (packed) {
         c.sp = c.Lp + kPanelDoubles;
@@ -178,7 +178,7 @@ hipError_t give_workspace(int dev, Workspace w, bool keep) {
 // hipGetSymbolAddress, once per device, and is kept in g_scratch.
 constexpr int kNoallocMaxM = BD_CHOLESKY_NOALLOC_MAX_M;
 constexpr size_t kNoallocDoubles =
-    (size_t)kNoallocMaxM * kNoallocMaxM + (size_t)(kNoallocMaxM / 64) * 64 * 64 + 32;
+    (size_t)kNoallocMaxM * kNoallocMaxM + (size_t)(kNoallocMaxM / 64 + 1) * 64 * 64 + 32;
 static __device__ __align__(256) double scratch[kNoallocDoubles];
 
 std::mutex g_scratch_mu;

@@ -200,13 +200,14 @@ int bd_get_chol_schedule(bd_context *ctx, int *panel_tiles_used);
  * library's blocked factor: replaces cusolverDnDpotrf +
  * Cholesky_Decomposition_mod (func_cuda.cu:3513-3534, 614-630), with the CPU
  * rule of func.cpp:806-836 on a negative pivot (|f| taken and counted;
- * cuSOLVER instead stops and the reference maps the NaNs to 0).
+ * cuSOLVER instead stops and the reference maps the NaNs to 0).  A pivot of
+ * exactly 0 (dependent rows, a row of zeros) has a column of zeros in L.
  * D: m x m row-major, only its lower triangle read (ldd >= m); L: m x m
  * row-major (ldl >= m), the lower factor with zeros above the diagonal; D
  * and L may be the same buffer when ldd == ldl.  mode: BD_CHOL_*.  neg: host
  * int for the count of negative pivots (may be NULL).  stream: a hipStream_t
  * (NULL: the default stream); the call returns once the factor is done.
- * The workspace, (64 n)^2 + 4096 n doubles for n = ceil(m/64) block columns and
+ * The workspace, (64 n)^2 + 4096 (n + 1) doubles for n = ceil(m/64) block columns and
  * from 60 (64 in the reduced modes) 32768 n + 262144 more, is allocated by the
  * call.  One of at most 256 MiB per device is kept for the next call; calls
  * that overlap have one each.  bd_cholesky_release frees what is kept (this

@@ -86,6 +86,27 @@ def test_pivots_outside_the_normal_range(m, scale):
     assert rel_err(np.ldexp(L, -k[:, None]), T) <= 1e-12
 
 
+@pytest.mark.parametrize("m", [2, 17, 64, 130, 200])
+@pytest.mark.parametrize("mode", [E.CHOL_FP64, E.CHOL_FP32, E.CHOL_BF16])
+def test_dependent_rows(m, mode):
+    """Matrices with rows that are the same, a multiple of another or 0: the
+    pivot is a rounding error or exactly 0, and the factor is finite with
+    |L L^T - D| at most (m + 1) u |L| |L^T|, twice for the |f| of a pivot below
+    0, u = 2^-53, and 2^-24 for the products of the reduced modes."""
+    for j in [k for k in (0, 3, 15, 16, 40, 62, 63, 64, 100, 128) if k < m - 1]:
+        for scale in (1.0, -1.0, 0.0):
+            D = spd(m, m)
+            D[j + 1, :] = scale * D[j, :]
+            D[:, j + 1] = scale * D[:, j]
+            D[j + 1, j + 1] = scale * scale * D[j, j]
+            L, neg = E.cholesky_device(D, mode)
+            assert np.all(np.isfinite(L)), (j, scale)
+            assert neg <= 1
+            A = np.abs(L) @ np.abs(L.T)
+            u = 2.0 ** (-53 if mode == E.CHOL_FP64 else -24)
+            assert np.all(np.abs(L @ L.T - D) <= (2 * m + 2) * u * A + (m + 1) * 2.0 ** -53 * np.abs(D)), (j, scale)
+
+
 # In FP64 super-panels start at 60 block columns: 83 and 84 are panels with a
 # last one of three and of four block columns, and the first sizes with and the
 # last without are those of test_panels_solved_in_one_launch.

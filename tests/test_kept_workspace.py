@@ -132,7 +132,7 @@ SCENES = {
     SOUND();
 """,
     "memory runs out": r"""
-    room = (size_t)3968 * 3968 * 8 + ((size_t)62 * 4096 + 32 + 64 * 64 * 64) * 8;
+    room = (size_t)3968 * 3968 * 8 + ((size_t)63 * 4096 + 32 + 64 * 64 * 64) * 8;
     CHECK(factor(3968) == BD_OK);      // without room for the packed tiles
     room = 1 << 20;
     CHECK(factor(3969) == BD_E_HIP);
